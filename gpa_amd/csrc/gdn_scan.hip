@@ -9,7 +9,7 @@
 //   S_{n+1} = e^{G_C} S_n + (diag(e^{G_C-G}) K)^T D.
 // Kernels:
 //   gdn_prep_mfma  chunk-parallel: normalise, G, T, W, U (gdn_prep_mfma.hip)
-//   gdn_state_fwd  sequential over chunks, parallel over (stream, 32-column tile):
+//   gdn_state_fwd  sequential over chunks, parallel over (stream, 16-column tile):
 //                  S_n (saved), D
 //   gdn_out_fwd    chunk-parallel: O
 //   gdn_dd0        chunk-parallel: P^T dO (the in-chunk part of dD)
@@ -28,84 +28,185 @@
 #include "gpa_common.h"
 #include "gdn_common.h"
 #include "gdn_strip.h"
+#include "mfma_tiles.h"
 
 namespace gpa {
 
 // ---------------------------------------------------------------------------
-// gdn_state_fwd: block (column tile blockIdx.x, stream blockIdx.y), loops chunks.
-template <int KM>
-__global__ __launch_bounds__(NT) void gdn_state_fwd(gpa_gdn_problem p, gpa_gdn_saved sv, int nch) {
-  extern __shared__ float smem[];
-  float* st_s = smem;                   // [KM][VT+1]
-  float* w_s = st_s + KM * (VT + 1);    // [R][LDS_]
-  float* d_s = w_s + R * LDS_;          // [R][VT+1]
-  float* gam_s = d_s + R * (VT + 1);    // [R]
-  float* rs_s = gam_s + R;              // [R] row scales
-  const int s = blockIdx.y, b = s / p.heads, h = s % p.heads;
-  const int K = p.kdim, V = p.vdim, tid = threadIdx.x;
-  const int r = tid / VT, c = tid % VT;  // r in 0..7
-  const int v = blockIdx.x * VT + c;
-  const bool vok = v < V;
+// The float32 state recurrences on v_mfma_f32_16x16x4f32 (float32 products and
+// sums): gdn_state_fwd, gdn_state_bwd.  One workgroup carries 16 columns of a
+// stream's state (blockIdx.x, stream blockIdx.y) through every chunk, held in
+// its four waves' accumulators: wave w has the key rows KM/4 w .. +KM/4-1.
+// Per chunk the state goes once through LDS (value-major) as the B operand of
+// the product over the keys, of which a wave forms 16 chunk positions, and the
+// result once as the B operand of the product over the positions: two
+// barriers.  The A operands come straight from the saved rows (16-byte reads
+// along the keys; KM/64 adjacent keys per lane and position the other way, so
+// tile i of a wave holds every KM/64-th of its keys), a chunk ahead of their
+// use where the registers allow (PF).  Bound: the chain of chunks, its MFMAs
+// (16 KM/64 for each of the two or three products of a wave, 32 cycles each) and the
+// two exchanges.  16 columns rather than 32 double the workgroups: a scan of
+// 32 streams by 64 columns is 128 of them.  FULL: K is a multiple of 16.
+// Measured at 32 streams x 16 chunks against scalar FMA products over operands
+// staged through LDS: K = 64, V = 64: 349 -> 28 us forward, 509 -> 38 us
+// backward; K = 128, V = 64: 681 -> 54 us and 1021 -> 64 us.
+constexpr int SC = 16;  // state columns per workgroup
 
-  for (int i = 0; i < KM / 8; ++i) {
-    const int k = r + 8 * i;
-    st_s[k * (VT + 1) + c] = (p.s0 && k < K && vok)
-        ? p.s0[(int64_t)b * p.s0_sb + (int64_t)h * p.s0_sh + (int64_t)k * V + v] : 0.f;
+// Element 4 j + e (e < 4) of a lane's KM/16 keys, as the accumulators hold them.
+template <int VEC>
+__device__ __forceinline__ f32x4 state_keys(const f32x4 (&s)[VEC], int j) {
+  f32x4 x;
+#pragma unroll
+  for (int e = 0; e < 4; ++e) x[e] = s[(4 * j + e) % VEC][(4 * j + e) / VEC];
+  return x;
+}
+// Four consecutive elements of a row of `width` floats from c; zeros past it.
+template <bool FULL>
+__device__ __forceinline__ f32x4 row4(const float* row, int c, int width) {
+  if (FULL) return *reinterpret_cast<const f32x4*>(row + (c < width ? c : 0));  // groups past the width are not used
+  f32x4 x;
+#pragma unroll
+  for (int e = 0; e < 4; ++e) x[e] = row[c + e < width ? c + e : 0];
+#pragma unroll
+  for (int e = 0; e < 4; ++e) x[e] = c + e < width ? x[e] : 0.f;
+  return x;
+}
+// The rows of a chunk as the A operand of a product over the keys: position
+// 16 w + l%16, keys 16 g + 4 (l/16) + 0..3.
+template <int KM, bool FULL>
+__device__ __forceinline__ void load_rows(f32x4 (&a)[KM / 16], const float* rows, int pos, int q, int K) {
+#pragma unroll
+  for (int g = 0; g < KM / 16; ++g)
+    a[g] = row4<FULL>(rows + (int64_t)pos * K, 16 * g + 4 * q, K);
+}
+// The rows of a chunk as the A operand of a product over the positions:
+// positions 16 g + 4 (l/16) + e, keys k0 .. k0 + VEC-1 (tile i holds key k0 + i).
+template <int VEC, bool FULL>
+__device__ __forceinline__ void load_cols(f32x4 (&a)[4 * VEC], const float* rows, int k0, int q, int K) {
+#pragma unroll
+  for (int g = 0; g < 4; ++g)
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      const float* row = rows + (int64_t)(16 * g + 4 * q + e) * K;
+      float x[VEC];
+      if (FULL) {
+        __builtin_memcpy(x, __builtin_assume_aligned(row + (k0 < K ? k0 : 0), 4 * VEC), sizeof x);
+      } else {
+#pragma unroll
+        for (int i = 0; i < VEC; ++i) x[i] = row[k0 + i < K ? k0 + i : 0];
+      }
+#pragma unroll
+      for (int i = 0; i < VEC; ++i) a[4 * i + g][e] = x[i];
+    }
+}
+// rows A (load_rows) times the 16 state columns in LDS.
+template <int KM>
+__device__ __forceinline__ f32x4 keys_product(const f32x4 (&a)[KM / 16], const float* st, int q, int K) {
+  f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+  for (int g = 0; g < KM / 16; ++g)
+    if (16 * g < K) mma16(acc, a[g], *reinterpret_cast<const f32x4*>(st + 16 * g + 4 * q));
+  return acc;
+}
+// A lane's state column to global memory, value-major (and to LDS as the next
+// product's B operand, keys past K zero).
+template <int VEC, bool FULL>
+__device__ __forceinline__ void put_state(const f32x4 (&s)[VEC], float* global, float* lds, int kb, int K, bool store) {
+#pragma unroll
+  for (int j = 0; j < VEC; ++j) {
+    f32x4 x = state_keys(s, j);
+    const int k = kb + 4 * j;
+    if (FULL) {
+      if (store && k < K) *reinterpret_cast<f32x4*>(global + k) = x;
+    } else {
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        if (store && k + e < K) global[k + e] = x[e];
+        x[e] = k + e < K ? x[e] : 0.f;
+      }
+    }
+    *reinterpret_cast<f32x4*>(lds + k) = x;
   }
-  __syncthreads();
+}
+
+template <int KM, bool FULL>
+__global__ __launch_bounds__(NT) void gdn_state_fwd(gpa_gdn_problem p, gpa_gdn_saved sv, int nch) {
+  constexpr int VEC = KM / 64;
+  constexpr bool PF = KM <= 128;  // operands of the next chunk in registers of their own
+  __shared__ __align__(16) float st_s[SC * (KM + 4)];
+  __shared__ __align__(16) float d_s[SC * (R + 4)];
+  const int s = blockIdx.y, b = s / p.heads, h = s % p.heads;
+  const int K = p.kdim, V = p.vdim, tid = threadIdx.x, w = tid / 64, col = tid % 16, q = tid % 64 / 16;
+  const int v = blockIdx.x * SC + col, vc = v < V ? v : V - 1;
+  const bool vok = v < V;
+  const int k0 = KM / 4 * w + VEC * col, kb = KM / 4 * w + 4 * VEC * q, t0 = 16 * w + 4 * q;
+  float* st = st_s + col * (KM + 4);
+  float* ds = d_s + col * (R + 4);
+
+  f32x4 S[VEC], wr[KM / 16], kc[4 * VEC], u, gm;
+  float gc;
+#pragma unroll
+  for (int j = 0; j < 4 * VEC; ++j) {
+    const int k = kb + j;
+    const float x = p.s0 ? p.s0[(int64_t)b * p.s0_sb + (int64_t)h * p.s0_sh + (int64_t)(k < K ? k : 0) * V + vc] : 0.f;
+    S[j % VEC][j / VEC] = k < K ? x : 0.f;
+  }
+  auto load_first = [&](int n, f32x4 (&wr)[KM / 16], f32x4& u, f32x4& gm, float& gc) {
+    const float* gam = sv.gam + rows_off(s, n, nch, 0, 1);
+    load_rows<KM, FULL>(wr, sv.w + rows_off(s, n, nch, 0, K), 16 * w + col, q, K);
+    u = *reinterpret_cast<const f32x4*>(sv.u + vc_off(s, n, nch, V) + (int64_t)vc * R + t0);
+    gm = *reinterpret_cast<const f32x4*>(gam + t0);
+    gc = gam[R - 1];
+  };
+  auto load_second = [&](int n, f32x4 (&kc)[4 * VEC]) {
+    load_cols<VEC, FULL>(kc, sv.kn + rows_off(s, n, nch, 0, K), k0, q, K);
+  };
+  load_first(0, wr, u, gm, gc);
+  load_second(0, kc);
   for (int n = 0; n < nch; ++n) {
-    const int64_t so = state_off(s, n, nch, K, V);
-    if (vok)
-      for (int i = 0; i < KM / 8; ++i) {
-        const int k = r + 8 * i;
-        if (k < K) sv.states[so + (int64_t)v * K + k] = st_s[k * (VT + 1) + c];
-      }
+    const int nn = n + 1 < nch ? n + 1 : n;
+    f32x4 wr2[KM / 16], kc2[4 * VEC], u2, gm2;
+    float gc2;
+    if (PF) {
+      load_first(nn, wr2, u2, gm2, gc2);
+      load_second(nn, kc2);
+    }
+    put_state<VEC, FULL>(S, sv.states + state_off(s, n, nch, K, V) + (int64_t)vc * K, st, kb, K, vok);
+    lds_barrier();
     // D = U - W S
-    const float* um = sv.u + vc_off(s, n, nch, V);
-    float acc[R / 8];
+    const f32x4 d = u - keys_product<KM>(wr, st, q, K);
+    if (vok) *reinterpret_cast<f32x4*>(sv.delta + vc_off(s, n, nch, V) + (int64_t)v * R + t0) = d;
+    f32x4 ds4;
 #pragma unroll
-    for (int j = 0; j < R / 8; ++j) acc[j] = vok ? um[(int64_t)v * R + r + 8 * j] : 0.f;
-    for (int k0 = 0; k0 < KM; k0 += KS) {
-      __syncthreads();
-      stage_rows(w_s, sv.w + rows_off(s, n, nch, 0, K), K, k0, nullptr);
-      __syncthreads();
-      for (int kk = 0; kk < KS; ++kk) {
-        const float sk = st_s[(k0 + kk) * (VT + 1) + c];
-#pragma unroll
-        for (int j = 0; j < R / 8; ++j) acc[j] -= w_s[(r + 8 * j) * LDS_ + kk] * sk;
-      }
-    }
-    float* dm = sv.delta + vc_off(s, n, nch, V);
-#pragma unroll
-    for (int j = 0; j < R / 8; ++j) {
-      d_s[(r + 8 * j) * (VT + 1) + c] = acc[j];
-      if (vok) dm[(int64_t)v * R + r + 8 * j] = acc[j];
-    }
-    if (tid < R) gam_s[tid] = sv.gam[rows_off(s, n, nch, 0, 1) + tid];
-    __syncthreads();
-    const float gc = gam_s[R - 1];
+    for (int e = 0; e < 4; ++e) ds4[e] = __expf(gc - gm[e]) * d[e];
+    *reinterpret_cast<f32x4*>(ds + t0) = ds4;
     const float decay = __expf(gc);
-    if (tid < R) rs_s[tid] = __expf(gc - gam_s[tid]);
-    // S = e^{G_C} S + (diag(e^{G_C-G}) Kn)^T D
-    for (int k0 = 0; k0 < KM; k0 += KS) {
-      __syncthreads();
-      stage_rows(w_s, sv.kn + rows_off(s, n, nch, 0, K), K, k0, rs_s);
-      __syncthreads();
+    if (!PF) load_first(nn, wr, u, gm, gc);
+    lds_barrier();
+    // S = e^{G_C} S + Kn^T diag(e^{G_C-G}) D
 #pragma unroll
-      for (int i = 0; i < KS / 8; ++i) {
-        const int kk = r + 8 * i;
-        float x = decay * st_s[(k0 + kk) * (VT + 1) + c];
-        for (int t = 0; t < R; ++t) x += w_s[t * LDS_ + kk] * d_s[t * (VT + 1) + c];
-        st_s[(k0 + kk) * (VT + 1) + c] = x;
+    for (int i = 0; i < VEC; ++i) S[i] *= decay;
+    if (KM / 4 * w < K)
+#pragma unroll
+      for (int g = 0; g < 4; ++g) {
+        const f32x4 x = *reinterpret_cast<const f32x4*>(ds + 16 * g + 4 * q);
+#pragma unroll
+        for (int i = 0; i < VEC; ++i) mma16(S[i], kc[4 * i + g], x);
       }
+    if (PF) {
+#pragma unroll
+      for (int g = 0; g < KM / 16; ++g) wr[g] = wr2[g];
+#pragma unroll
+      for (int j = 0; j < 4 * VEC; ++j) kc[j] = kc2[j];
+      u = u2; gm = gm2; gc = gc2;
+    } else {
+      load_second(nn, kc);
     }
-    __syncthreads();
   }
   if (vok)
-    for (int i = 0; i < KM / 8; ++i) {
-      const int k = r + 8 * i;
-      if (k < K) sv.final[(int64_t)s * K * V + (int64_t)k * V + v] = st_s[k * (VT + 1) + c];
-    }
+#pragma unroll
+    for (int j = 0; j < 4 * VEC; ++j)
+      if (kb + j < K) sv.final[(int64_t)s * K * V + (int64_t)(kb + j) * V + v] = S[j % VEC][j / VEC];
 }
 
 // P = causal e^{G_t-G_s} Qn Kn^T into p_s ([R][LDR]); uses two R x KS slices.
@@ -278,89 +379,109 @@ __global__ __launch_bounds__(NT) void gdn_dd0(gpa_gdn_problem p, gpa_gdn_saved s
 
 // ---------------------------------------------------------------------------
 // gdn_state_bwd: reverse sequential dS; writes dS at every chunk end and dD.
-template <typename E, int KM>
+// (The layout of gdn_state_fwd; has_q and has_inj are uniform.)
+template <int KM, bool FULL>
 __global__ __launch_bounds__(NT) void gdn_state_bwd(gpa_gdn_problem p, gpa_gdn_saved sv, gpa_gdn_grads gr,
                                                      int nch) {
-  extern __shared__ float smem[];
-  float* ds_s = smem;                   // [KM][VT+1]
-  float* x_s = ds_s + KM * (VT + 1);    // [R][LDS_]
-  float* y_s = x_s + R * LDS_;          // [R][LDS_]
-  float* dd_s = y_s + R * LDS_;         // [R][VT+1]
-  float* o_s = dd_s + R * (VT + 1);     // [R][VT+1]
-  float* gam_s = o_s + R * (VT + 1);    // [R]
-  float* rs_s = gam_s + R;              // [R]
-  const int s = blockIdx.y, b = s / p.heads, h = s % p.heads;
-  const int K = p.kdim, V = p.vdim, tid = threadIdx.x;
-  const int r = tid / VT, c = tid % VT;
-  const int v = blockIdx.x * VT + c;
+  constexpr int VEC = KM / 64;
+  constexpr bool PF = KM <= 64;
+  __shared__ __align__(16) float st_s[SC * (KM + 4)];
+  __shared__ __align__(16) float d_s[SC * (R + 4)];
+  const int s = blockIdx.y;
+  const int K = p.kdim, V = p.vdim, tid = threadIdx.x, w = tid / 64, col = tid % 16, q = tid % 64 / 16;
+  const int v = blockIdx.x * SC + col, vc = v < V ? v : V - 1;
   const bool vok = v < V;
   const bool has_q = p.q.ptr != nullptr && gr.dout.ptr != nullptr;
+  const int k0 = KM / 4 * w + VEC * col, kb = KM / 4 * w + 4 * VEC * q, t0 = 16 * w + 4 * q;
+  float* st = st_s + col * (KM + 4);
+  float* ds = d_s + col * (R + 4);
+  const f32x4 zero = {0.f, 0.f, 0.f, 0.f};
 
-  for (int i = 0; i < KM / 8; ++i) {
-    const int k = r + 8 * i;
-    ds_s[k * (VT + 1) + c] = (gr.dfinal && k < K && vok) ? gr.dfinal[(int64_t)s * K * V + (int64_t)k * V + v] : 0.f;
+  f32x4 S[VEC], kr[KM / 16], qc[4 * VEC], wc[4 * VEC], o[4], d0, gm;
+  float gc;
+#pragma unroll
+  for (int j = 0; j < 4 * VEC; ++j) {
+    const int k = kb + j;
+    const float x = gr.dfinal ? gr.dfinal[(int64_t)s * K * V + (int64_t)(k < K ? k : 0) * V + vc] : 0.f;
+    S[j % VEC][j / VEC] = k < K ? x : 0.f;
   }
+  auto load_first = [&](int n, f32x4 (&kr)[KM / 16], f32x4& d0, f32x4& gm, float& gc) {
+    const float* gam = sv.gam + rows_off(s, n, nch, 0, 1);
+    load_rows<KM, FULL>(kr, sv.kn + rows_off(s, n, nch, 0, K), 16 * w + col, q, K);
+    d0 = gr.dd0 ? *reinterpret_cast<const f32x4*>(gr.dd0 + vc_off(s, n, nch, V) + (int64_t)vc * R + t0) : zero;
+    gm = *reinterpret_cast<const f32x4*>(gam + t0);
+    gc = gam[R - 1];
+  };
+  auto load_second = [&](int n, f32x4 (&qc)[4 * VEC], f32x4 (&wc)[4 * VEC], f32x4 (&o)[4]) {
+    if (has_q) {
+      load_cols<VEC, FULL>(qc, sv.qn + rows_off(s, n, nch, 0, K), k0, q, K);
+#pragma unroll
+      for (int g = 0; g < 4; ++g)
+        o[g] = *reinterpret_cast<const f32x4*>(gr.o + vc_off(s, n, nch, V) + (int64_t)vc * R + 16 * g + 4 * q);
+    }
+    load_cols<VEC, FULL>(wc, sv.w + rows_off(s, n, nch, 0, K), k0, q, K);
+  };
+  load_first(nch - 1, kr, d0, gm, gc);
+  load_second(nch - 1, qc, wc, o);
   for (int n = nch - 1; n >= 0; --n) {
-    __syncthreads();
-    const int64_t so = state_off(s, n, nch, K, V);
-    if (vok)
-      for (int i = 0; i < KM / 8; ++i) {
-        const int k = r + 8 * i;
-        if (k < K) gr.dhend[so + (int64_t)v * K + k] = ds_s[k * (VT + 1) + c];
-      }
-    if (tid < R) gam_s[tid] = sv.gam[rows_off(s, n, nch, 0, 1) + tid];
-    __syncthreads();
-    const float gc = gam_s[R - 1];
-    if (tid < R) rs_s[tid] = __expf(gc - gam_s[tid]);
+    const int nn = n > 0 ? n - 1 : 0;
+    f32x4 kr2[KM / 16], qc2[4 * VEC], wc2[4 * VEC], o2[4], d02, gm2;
+    float gc2;
+    if (PF) {
+      load_first(nn, kr2, d02, gm2, gc2);
+      load_second(nn, qc2, wc2, o2);
+    }
+    const int64_t so = state_off(s, n, nch, K, V) + (int64_t)vc * K;
+    f32x4 inj[VEC];
+    if (gr.dstates)
+#pragma unroll
+      for (int j = 0; j < VEC; ++j) inj[j] = row4<FULL>(gr.dstates + so, kb + 4 * j, K);
+    put_state<VEC, FULL>(S, gr.dhend + so, st, kb, K, vok);
+    lds_barrier();
     // dD = dd0 + diag(e^{G_C-G}) Kn dS
-    const float* d0 = gr.dd0 ? gr.dd0 + vc_off(s, n, nch, V) : nullptr;
-    const float* om = has_q ? gr.o + vc_off(s, n, nch, V) : nullptr;
-    float* ddm = gr.ddelta + vc_off(s, n, nch, V);
-    float acc[R / 8];
+    f32x4 dd = keys_product<KM>(kr, st, q, K);
 #pragma unroll
-    for (int j = 0; j < R / 8; ++j) acc[j] = (d0 && vok) ? d0[(int64_t)v * R + r + 8 * j] : 0.f;
-    for (int k0 = 0; k0 < KM; k0 += KS) {
-      __syncthreads();
-      stage_rows(x_s, sv.kn + rows_off(s, n, nch, 0, K), K, k0, rs_s);
-      __syncthreads();
-      for (int kk = 0; kk < KS; ++kk) {
-        const float d = ds_s[(k0 + kk) * (VT + 1) + c];
-#pragma unroll
-        for (int j = 0; j < R / 8; ++j) acc[j] += x_s[(r + 8 * j) * LDS_ + kk] * d;
-      }
-    }
-#pragma unroll
-    for (int j = 0; j < R / 8; ++j) {
-      const int t = r + 8 * j;
-      dd_s[t * (VT + 1) + c] = acc[j];
-      if (vok) ddm[(int64_t)v * R + t] = acc[j];
-      o_s[t * (VT + 1) + c] = (om && vok) ? om[(int64_t)v * R + t] : 0.f;
-    }
-    // dS_prev = e^{G_C} dS + Qn^T diag(e^G) dO - W^T dD + dstates[n]
+    for (int e = 0; e < 4; ++e) dd[e] = d0[e] + __expf(gc - gm[e]) * dd[e];
+    if (vok) *reinterpret_cast<f32x4*>(gr.ddelta + vc_off(s, n, nch, V) + (int64_t)v * R + t0) = dd;
+    *reinterpret_cast<f32x4*>(ds + t0) = -dd;
     const float decay = __expf(gc);
-    for (int k0 = 0; k0 < KM; k0 += KS) {
-      __syncthreads();
-      if (has_q) stage_rows(x_s, sv.qn + rows_off(s, n, nch, 0, K), K, k0, nullptr);
-      stage_rows(y_s, sv.w + rows_off(s, n, nch, 0, K), K, k0, nullptr);
-      __syncthreads();
+    if (!PF) load_first(nn, kr, d0, gm, gc);
+    lds_barrier();
+    // dS_prev = e^{G_C} dS + Qn^T diag(e^G) dO - W^T dD + dstates[n]
 #pragma unroll
-      for (int i = 0; i < KS / 8; ++i) {
-        const int kk = r + 8 * i, k = k0 + kk;
-        float x = decay * ds_s[k * (VT + 1) + c];
-        if (has_q)
-          for (int t = 0; t < R; ++t) x += x_s[t * LDS_ + kk] * o_s[t * (VT + 1) + c];
-        for (int t = 0; t < R; ++t) x -= y_s[t * LDS_ + kk] * dd_s[t * (VT + 1) + c];
-        if (gr.dstates && vok && k < K) x += gr.dstates[so + (int64_t)v * K + k];
-        ds_s[k * (VT + 1) + c] = x;
+    for (int i = 0; i < VEC; ++i) S[i] *= decay;
+    if (KM / 4 * w < K) {
+      if (has_q)
+#pragma unroll
+        for (int g = 0; g < 4; ++g)
+#pragma unroll
+          for (int i = 0; i < VEC; ++i) mma16(S[i], qc[4 * i + g], o[g]);
+#pragma unroll
+      for (int g = 0; g < 4; ++g) {
+        const f32x4 x = *reinterpret_cast<const f32x4*>(ds + 16 * g + 4 * q);
+#pragma unroll
+        for (int i = 0; i < VEC; ++i) mma16(S[i], wc[4 * i + g], x);
       }
+    }
+    if (gr.dstates)
+#pragma unroll
+      for (int j = 0; j < 4 * VEC; ++j) S[j % VEC][j / VEC] += inj[j / 4][j % 4];
+    if (PF) {
+#pragma unroll
+      for (int g = 0; g < KM / 16; ++g) kr[g] = kr2[g];
+#pragma unroll
+      for (int j = 0; j < 4 * VEC; ++j) { qc[j] = qc2[j]; wc[j] = wc2[j]; }
+#pragma unroll
+      for (int g = 0; g < 4; ++g) o[g] = o2[g];
+      d0 = d02; gm = gm2; gc = gc2;
+    } else {
+      load_second(nn, qc, wc, o);
     }
   }
-  __syncthreads();
   if (vok)
-    for (int i = 0; i < KM / 8; ++i) {
-      const int k = r + 8 * i;
-      if (k < K) gr.ds0[(int64_t)s * K * V + (int64_t)k * V + v] = ds_s[k * (VT + 1) + c];
-    }
+#pragma unroll
+    for (int j = 0; j < 4 * VEC; ++j)
+      if (kb + j < K) gr.ds0[(int64_t)s * K * V + (int64_t)(kb + j) * V + v] = S[j % VEC][j / VEC];
 }
 
 // ---------------------------------------------------------------------------
@@ -924,7 +1045,6 @@ int strip_form(int km, bool fast, bool wide_ok, bool quarter_ok, int quarter_wor
 // The state recurrence of one problem outside a pack.
 template <typename E, int KM>
 int fwd_state(const gpa_gdn_problem& p, const gpa_gdn_saved& sv, int nch, hipStream_t st) {
-  const dim3 block(NT);
   if (strip_path<E>(p)) {
     StripFwdPack pk{};
     pk.n = 1;
@@ -935,10 +1055,9 @@ int fwd_state(const gpa_gdn_problem& p, const gpa_gdn_saved& sv, int nch, hipStr
     return launch_state_fwd_strip<KM <= 64 ? 64 : 128>(pk, strip_workgroups(p, nq), fast, nq, st);
   }
   if (use_mfma<E>(p)) return launch_state_fwd_mfma<KM>(p, sv, nch, st);
-  const dim3 grid_s((p.vdim + VT - 1) / VT, p.batch * p.heads);
-  const size_t lds_state = sizeof(float) * (KM * (VT + 1) + R * LDS_ + R * (VT + 1) + 2 * R);
-  if (int rc = allow_lds(gdn_state_fwd<KM>, lds_state)) return rc;
-  hipLaunchKernelGGL((gdn_state_fwd<KM>), grid_s, block, lds_state, st, p, sv, nch);
+  const dim3 grid((p.vdim + SC - 1) / SC, p.batch * p.heads);
+  if (p.kdim % 16 == 0) hipLaunchKernelGGL((gdn_state_fwd<KM, true>), grid, dim3(NT), 0, st, p, sv, nch);
+  else hipLaunchKernelGGL((gdn_state_fwd<KM, false>), grid, dim3(NT), 0, st, p, sv, nch);
   return GPA_HIP_OK;
 }
 
@@ -973,7 +1092,6 @@ int bwd_dd0(const gpa_gdn_problem& p, const gpa_gdn_saved& sv, const gpa_gdn_gra
 
 template <typename E, int KM>
 int bwd_state(const gpa_gdn_problem& p, const gpa_gdn_saved& sv, const gpa_gdn_grads& gr, int nch, hipStream_t st) {
-  const dim3 block(NT);
   if (strip_path<E>(p)) {
     const bool has_q = has_read(p, gr);
     StripBwdPack pk{};
@@ -985,10 +1103,11 @@ int bwd_state(const gpa_gdn_problem& p, const gpa_gdn_saved& sv, const gpa_gdn_g
     return launch_state_bwd_strip<KM <= 64 ? 64 : 128>(pk, strip_workgroups(p, nq), fast, has_q, has_inj, nq, st);
   }
   if (use_mfma<E>(p)) return launch_state_bwd_mfma<KM>(p, sv, gr, nch, st);
-  const dim3 grid_s((p.vdim + VT - 1) / VT, p.batch * p.heads);
-  const size_t lds_state = sizeof(float) * (KM * (VT + 1) + 2 * R * LDS_ + 2 * R * (VT + 1) + 2 * R);
-  if (int rc = allow_lds(gdn_state_bwd<E, KM>, lds_state)) return rc;
-  hipLaunchKernelGGL((gdn_state_bwd<E, KM>), grid_s, block, lds_state, st, p, sv, gr, nch);
+  const dim3 grid((p.vdim + SC - 1) / SC, p.batch * p.heads);
+  // the injections are the caller's tensor: 16-byte reads only where its rows allow them
+  const bool full = p.kdim % 16 == 0 && reinterpret_cast<uintptr_t>(gr.dstates) % 16 == 0;
+  if (full) hipLaunchKernelGGL((gdn_state_bwd<KM, true>), grid, dim3(NT), 0, st, p, sv, gr, nch);
+  else hipLaunchKernelGGL((gdn_state_bwd<KM, false>), grid, dim3(NT), 0, st, p, sv, gr, nch);
   return GPA_HIP_OK;
 }
 

@@ -79,8 +79,8 @@ typedef struct gpa_gdn_problem {
     int64_t s0_sb, s0_sh;
 } gpa_gdn_problem;
 
-/* Caller-owned intermediates, stream-major and contiguous (S = streams,
- * N = nchunks, per chunk):
+/* Caller-owned intermediates, stream-major and contiguous, each starting on a
+ * 16-byte boundary (S = streams, N = nchunks, per chunk):
  *   kn, qn         f32 [S,N,64,K]   normalised keys / queries (rows = positions); for bf16
  *                                   problems with K % 16 == 0 and V <= 256, qn holds its
  *                                   exact bf16 values instead (bf16 [S,N,64,K] in the first

@@ -1,0 +1,34 @@
+"""The float32 state recurrences (gdn_state_fwd / gdn_state_bwd, 16 state
+columns per workgroup, key rows split over four waves) at the edges of their
+tiles: key widths at and around the 64/128/256 classes, whole and partial
+16-wide key groups, one and partial 16-column tiles, chunks of few rows.
+Compared with the oracle's recurrence in float64 at 1e-5: sums of at most 256
+float32 products, each scaled by e^g <= 1, over a chain of at most 4 chunks."""
+import pytest
+import torch
+
+from tests.test_gpu_gdn_scan import DEV, _inputs, _oracle_segments_autograd, _rel
+
+pytestmark = pytest.mark.gpu
+
+# (T, K, V, chunk, offset)
+CASES = [(1, 16, 16, 64, 0), (70, 80, 17, 64, 5), (9, 64, 1, 3, 1), (130, 144, 33, 64, 63), (20, 256, 15, 8, 3),
+         (67, 18, 16, 32, 0), (40, 130, 5, 16, 2), (33, 68, 48, 64, 0)]
+
+
+@pytest.mark.parametrize("case", CASES, ids=lambda c: "T{}K{}V{}C{}o{}".format(*c))
+def test_float32_state_matches_recurrence(case):
+    from gpa_amd.ops import gdn_scan_hip
+    t, kd, vd, chunk, offset = case
+    inputs = _inputs(2, t, 2, kd, vd, torch.float32, seed=21)
+    leaves = [x.to(DEV).requires_grad_() for x in inputs]
+    refs = [x.double().requires_grad_() for x in inputs]
+    got = gdn_scan_hip(*leaves, chunk=chunk, offset=offset)
+    want = _oracle_segments_autograd(refs[:3], *refs[3:], chunk, offset)
+    gen = torch.Generator().manual_seed(3)
+    grads = [torch.randn(x.shape, generator=gen, dtype=torch.float64) for x in want]
+    dg = torch.autograd.grad(got, leaves, [x.to(DEV, torch.float32) for x in grads])
+    dr = torch.autograd.grad(want, refs, [x.float().double() for x in grads])
+    errs = [_rel(a, b) for a, b in zip((*got, *dg), (*want, *dr))]
+    print(case, errs)
+    assert max(errs) < 1e-5, errs
