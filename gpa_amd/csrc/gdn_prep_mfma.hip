@@ -3,8 +3,7 @@
 //   G     in-chunk cumulative log decay (a wave scan of g)
 //   Kn,Qn x/|x| rounded to the activation type, and their bf16 fragments
 //   A     strictly lower b_t e^{G_t-G_u} Kn_t . Kn_u          (K Kn^T on MFMA)
-//   T     (I + A)^-1: 16 x 16 diagonal blocks by forward substitution, then
-//         block rows i = 1..3: T_ij = -T_ii sum_{j<=m<i} A_im T_mj
+//   T     (I + A)^-1 (unit_lower_inverse)
 //   W     T diag(b e^G) Kn   (bf16 hi/lo fragments, or fp32 rows)
 //   U     T diag(b) V        (value-major fp32)
 // with the layouts of include/gpa_hip.h.  Reference: the WY form of the
@@ -19,17 +18,82 @@ namespace gpa {
 
 constexpr int PREP_WAVES = 8, PREP_NT = 64 * PREP_WAVES;
 
+constexpr int PREP_LT = R + 4;  // row pitch of A and T in LDS
+
+// T = (I + A)^-1 of a strictly lower 64 x 64 A (zeros on and above the diagonal
+// of its 16 x 16 diagonal blocks; the blocks above them are not read), by every
+// thread of the workgroup: t_s starts as zeros, A and T rows PREP_LT apart.
+// Wave 0 inverts the four diagonal blocks by forward substitution, a column
+// per lane, in registers; then the inverses of neighbouring diagonal blocks
+// T11, T22 give that of twice their size, T21 = -T22 (A21 T11), for 32 and for
+// 64 rows on 16 x 16 tiles of the fp32 MFMA.  An accumulator tile is the B
+// operand of the next product as it stands (mma16 takes contraction index
+// 4 (l/16) + s, the accumulator's row), so A21 T11 stays in registers.
+// Bound: the latency of its three short phases.  Against forward substitution
+// through LDS with run-time trip counts and scalar block products, the prep of
+// 32 streams x 64 chunks of 128 keys takes 27 us less (of 170).
+__device__ __forceinline__ void unit_lower_inverse(const float* a_s, float* t_s, int wave, int lane) {
+  constexpr int LT = PREP_LT;
+  const int c = lane & 15, q = lane >> 4;
+  if (wave == 0) {
+    const float* ab = a_s + 16 * q * (LT + 1);
+    float x[16];
+#pragma unroll
+    for (int t = 0; t < 16; ++t) {
+      float acc = t == c ? 1.f : 0.f;
+#pragma unroll
+      for (int g = 0; 4 * g < t; ++g) {
+        const f32x4 a = *reinterpret_cast<const f32x4*>(ab + t * LT + 4 * g);
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+          if (4 * g + e < t) acc -= a[e] * x[4 * g + e];
+      }
+      x[t] = acc;
+    }
+#pragma unroll
+    for (int t = 0; t < 16; ++t) t_s[(16 * q + t) * LT + 16 * q + c] = x[t];
+  }
+  lds_barrier();
+  const f32x4 zero = {0.f, 0.f, 0.f, 0.f};
+  if (wave < 2) {  // 16 -> 32 rows: pair `wave`
+    const int lo = 32 * wave, hi = lo + 16;
+    f32x4 x = zero, y = zero;
+    mma16(x, ld_c(a_s, LT, hi + c, lo + 4 * q), ld_x(t_s, LT, lo + c, lo + 4 * q));
+    mma16(y, ld_c(t_s, LT, hi + c, hi + 4 * q), x);
+#pragma unroll
+    for (int e = 0; e < 4; ++e) t_s[(hi + 4 * q + e) * LT + lo + c] = -y[e];
+  }
+  lds_barrier();
+  if (wave < 4) {  // 32 -> 64 rows: tile (i, j) of the corner
+    const int i = wave >> 1, j = wave & 1;
+    f32x4 x[2] = {zero, zero}, y = zero;
+#pragma unroll
+    for (int m = 0; m < 2; ++m) {
+      if (m > i) continue;
+#pragma unroll
+      for (int k = 0; k < 2; ++k)
+        if (k >= j)
+          mma16(x[m], ld_c(a_s, LT, 32 + 16 * m + c, 16 * k + 4 * q), ld_x(t_s, LT, 16 * j + c, 16 * k + 4 * q));
+    }
+#pragma unroll
+    for (int m = 0; m < 2; ++m)
+      if (m <= i) mma16(y, ld_c(t_s, LT, 32 + 16 * i + c, 32 + 16 * m + 4 * q), x[m]);
+#pragma unroll
+    for (int e = 0; e < 4; ++e) t_s[(32 + 16 * i + 4 * q + e) * LT + 16 * j + c] = -y[e];
+  }
+  lds_barrier();
+}
+
 // LDS plan (floats): one region holds Kn rows, then W (the fragment source,
 // once the W product has read Kn), then the b-scaled V slices; T; A (until T
 // is done); per-row scalars.  Up to 128 keys this is under 80 KB, so two
 // workgroups share a compute unit.
 template <int KM>
 struct PrepLayout {
-  static constexpr int LK = KM + 4, LT = R + 4, VC = 128, LV = VC + 4;
+  static constexpr int LK = KM + 4, LT = PREP_LT, VC = 128, LV = VC + 4;
   static constexpr int BIG = R * LK > R * LV ? R * LK : R * LV;
   static constexpr int KN_OFF = 0, T_OFF = BIG, A_OFF = T_OFF + R * LT;
-  static constexpr int BLK_OFF = A_OFF + R * LT;  // 3 x 16 x 16 block products
-  static constexpr int SC_OFF = BLK_OFF + 3 * 256;
+  static constexpr int SC_OFF = A_OFF + R * LT;
   static constexpr int TOTAL = SC_OFF + 4 * R;
   static constexpr size_t BYTES = sizeof(float) * TOTAL;
 };
@@ -45,7 +109,6 @@ __global__ __launch_bounds__(PREP_NT, 1) void gdn_prep_mfma(gpa_gdn_problem p, g
   float* v_s = kn_s;
   float* t_s = smem + L::T_OFF;    // [R][LT] T
   float* a_s = smem + L::A_OFF;    // [R][LT] A
-  float* blk = smem + L::BLK_OFF;  // [3][16][16]
   float* gam_s = smem + L::SC_OFF;
   float* bet_s = gam_s + R;
   float* sc_s = bet_s + R;  // b e^G
@@ -182,35 +245,7 @@ __global__ __launch_bounds__(PREP_NT, 1) void gdn_prep_mfma(gpa_gdn_problem p, g
   }
   __syncthreads();
 
-  // ---- T = (I + A)^-1.  Diagonal 16x16 blocks: thread c of wave 0 owns column c.
-  if (tid < R) {
-    const int base = 16 * (tid >> 4), c = tid & 15;
-    t_s[(base + c) * LT + base + c] = 1.f;
-    for (int t = c + 1; t < 16; ++t) {
-      float acc = 0.f;
-      for (int u = c; u < t; ++u) acc += a_s[(base + t) * LT + base + u] * t_s[(base + u) * LT + base + c];
-      t_s[(base + t) * LT + base + c] = -acc;
-    }
-  }
-  __syncthreads();
-  // Block rows: X_j = sum_{j<=m<i} A_im T_mj, then T_ij = -T_ii X_j.
-  for (int i = 1; i < 4; ++i) {
-    for (int idx = tid; idx < i * 256; idx += NTH) {
-      const int j = idx >> 8, r = (idx >> 4) & 15, c = idx & 15;
-      float acc = 0.f;
-      for (int m = 16 * j; m < 16 * i; ++m) acc += a_s[(16 * i + r) * LT + m] * t_s[m * LT + 16 * j + c];
-      blk[idx] = acc;
-    }
-    __syncthreads();
-    for (int idx = tid; idx < i * 256; idx += NTH) {
-      const int j = idx >> 8, r = (idx >> 4) & 15, c = idx & 15;
-      float acc = 0.f;
-#pragma unroll
-      for (int m = 0; m < 16; ++m) acc += t_s[(16 * i + r) * LT + 16 * i + m] * blk[(j << 8) + m * 16 + c];
-      t_s[(16 * i + r) * LT + 16 * j + c] = -acc;
-    }
-    __syncthreads();
-  }
+  unit_lower_inverse(a_s, t_s, wave, lane);
   {
     float* tri = sv.tri + rows_off(s, n, nch, 0, R);
     for (int i = tid; i < R * R / 4; i += NTH) {
