@@ -167,9 +167,10 @@ template <int KM>
 int launch_state_fwd_mfma_pack(const MfmaPack& pk, int total, bool fast, hipStream_t st);
 template <int KM>
 int launch_state_bwd_mfma_pack(const MfmaPack& pk, int total, bool fast, bool has_q, bool has_inj, hipStream_t st);
-// MFMA chunk preparation (gdn_prep_mfma.hip); mf: write the bf16 fragments.
+// Chunk preparation (gdn_prep_mfma.hip); bf16 with K % 16 == 0 writes the bf16
+// fragments, the rest the float32 W rows.
 template <typename E, int KM>
-int launch_prep_mfma(const gpa_gdn_problem& p, const gpa_gdn_saved& sv, bool mf, int nch, hipStream_t st);
+int launch_prep(const gpa_gdn_problem& p, const gpa_gdn_saved& sv, int nch, hipStream_t st);
 // bf16-MFMA output read and its chunk-local gradient (gdn_out_mfma.hip); bf16,
 // kdim % 16 == 0 and vdim <= GPA_OUT_MFMA_MAX_V.
 constexpr int GPA_OUT_MFMA_MAX_V = 256;

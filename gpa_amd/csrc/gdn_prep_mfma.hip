@@ -1,11 +1,12 @@
-// Chunk preparation of the GDN scan on fp32 MFMA: one block per (chunk,
-// stream), 8 waves.  Per chunk of positions t, u < 64:
+// Chunk preparation of the GDN scan on MFMA: one block per (chunk, stream), 8
+// waves (gdn_prep_mfma, gdn_prep_frag).  Per chunk of positions t, u < 64:
 //   G     in-chunk cumulative log decay (a wave scan of g)
-//   Kn,Qn x/|x| rounded to the activation type, and their bf16 fragments
+//   Kn,Qn x/|x| rounded to the activation type, on the bf16 MFMA path also as
+//         fragments
 //   A     strictly lower b_t e^{G_t-G_u} Kn_t . Kn_u          (K Kn^T on MFMA)
 //   T     (I + A)^-1 (unit_lower_inverse)
 //   W     T diag(b e^G) Kn   (bf16 hi/lo fragments, or fp32 rows)
-//   U     T diag(b) V        (value-major fp32)
+//   U     T diag(b) V        (fp32, value-major or in fragment order)
 // with the layouts of include/gpa_hip.h.  Reference: the WY form of the
 // chunked gated delta rule that src/gpa/ops.py:49-85 runs per token.
 #include <hip/hip_runtime.h>
@@ -84,9 +85,9 @@ __device__ __forceinline__ void unit_lower_inverse(const float* a_s, float* t_s,
   lds_barrier();
 }
 
-// LDS plan (floats): one region holds Kn rows, then W (the fragment source,
-// once the W product has read Kn), then the b-scaled V slices; T; A (until T
-// is done); per-row scalars.  Up to 128 keys this is under 80 KB, so two
+// gdn_prep_mfma: float32, and bf16 with K not a multiple of 16.  LDS plan
+// (floats): one region holds Kn rows, then the b-scaled V slices; T; A (until
+// T is done); per-row scalars.  Up to 128 keys this is under 80 KB, so two
 // workgroups share a compute unit.
 template <int KM>
 struct PrepLayout {
@@ -98,14 +99,13 @@ struct PrepLayout {
   static constexpr size_t BYTES = sizeof(float) * TOTAL;
 };
 
-template <typename E, int KM, bool MF>
+template <typename E, int KM>
 __global__ __launch_bounds__(PREP_NT, 1) void gdn_prep_mfma(gpa_gdn_problem p, gpa_gdn_saved sv, int nch) {
   using L = PrepLayout<KM>;
   constexpr int LK = L::LK, LT = L::LT, VC = L::VC, LV = L::LV, NW = PREP_WAVES, NTH = PREP_NT;
   constexpr int KT = KM / 32, NTW = KT >= 4 ? KT / 4 : 1;
   extern __shared__ __align__(16) float smem[];
-  float* kn_s = smem + L::KN_OFF;  // [R][LK] Kn (rounded), then W [R][LK], then b V slices [R][LV]
-  float* w_s = kn_s;
+  float* kn_s = smem + L::KN_OFF;  // [R][LK] Kn (rounded), then b V slices [R][LV]
   float* v_s = kn_s;
   float* t_s = smem + L::T_OFF;    // [R][LT] T
   float* a_s = smem + L::A_OFF;    // [R][LT] A
@@ -117,9 +117,7 @@ __global__ __launch_bounds__(PREP_NT, 1) void gdn_prep_mfma(gpa_gdn_problem p, g
   const int n = blockIdx.x, s = blockIdx.y, b = s / p.heads, h = s % p.heads;
   const int K = p.kdim, V = p.vdim, tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int li = lane & 31, hh = lane >> 5;
-  const int K16 = K / 16;
-  const int64_t chunk_id = (int64_t)s * nch + n;
-  const bool has_q = p.q.ptr != nullptr, rows16 = MF && qk_rows_bf16(p);
+  const bool has_q = p.q.ptr != nullptr;
 
   // ---- gates: G by a wave-wide inclusive scan (wave 0).
   if (wave == 0) {
@@ -144,7 +142,6 @@ __global__ __launch_bounds__(PREP_NT, 1) void gdn_prep_mfma(gpa_gdn_problem p, g
 
   // ---- normalise keys and queries: wave w owns rows w, w + 8, ...; every
   // load is issued (at a clamped address) before the first use.
-  __bf16* qcol = MF && has_q ? reinterpret_cast<__bf16*>(sv.qcol) + chunk_id * frag_col_elems(K, 8) : nullptr;
   {
     constexpr int NI = KM / 64, NR = R / NW;
     const gpa_operand& qsrc = has_q ? p.q : p.k;
@@ -177,46 +174,12 @@ __global__ __launch_bounds__(PREP_NT, 1) void gdn_prep_mfma(gpa_gdn_problem p, g
         const int d = lane + 64 * i;
         const float yk = round_as<E>(xk[j][i] / dk);
         kn_s[r * LK + d] = yk;
-        // (where the bf16 out and dd0 kernels read them, the Kn rows are the
-        // krow fragments written below)
-        if (d < K && !rows16) sv.kn[rows_off(s, n, nch, r, K) + d] = yk;
-        if (has_q && d < K) {
-          const float yq = round_as<E>(xq[j][i] / dq);
-          if (rows16) reinterpret_cast<bf16_t*>(sv.qn)[rows_off(s, n, nch, r, K) + d] = from_f32<bf16_t>(yq);
-          else sv.qn[rows_off(s, n, nch, r, K) + d] = yq;
-          if (MF) {  // Qn^T fragment (d/32, r/16), lane d%32 + 32 ((r/8) % 2), element r % 8
-            const int rb = d >> 5, cs = r >> 4, ln = (d & 31) + 32 * ((r >> 3) & 1);
-            qcol[((rb * 4 + cs) * 64 + ln) * 8 + (r & 7)] = (__bf16)yq;
-          }
-        }
+        if (d < K) sv.kn[rows_off(s, n, nch, r, K) + d] = yk;
+        if (has_q && d < K) sv.qn[rows_off(s, n, nch, r, K) + d] = round_as<E>(xq[j][i] / dq);
       }
     }
   }
   __syncthreads();
-
-  typedef __bf16 bf16x8v __attribute__((ext_vector_type(8)));
-  if (MF) {
-    // Kn row and column fragments (exact in bf16), one 16-byte piece per step.
-    __bf16* krow = reinterpret_cast<__bf16*>(sv.krow) + chunk_id * frag_row_elems(K, 8);
-    __bf16* kcol = reinterpret_cast<__bf16*>(sv.kcol) + chunk_id * frag_col_elems(K, 8);
-    for (int piece = tid; piece < 2 * K16 * 64; piece += NTH) {
-      const int ln = piece & 63, ks = (piece >> 6) % K16, rt = (piece >> 6) / K16;
-      const float* src = kn_s + (32 * rt + (ln & 31)) * LK + 16 * ks + 8 * (ln >> 5);
-      bf16x8v f;
-#pragma unroll
-      for (int e = 0; e < 8; ++e) f[e] = (__bf16)src[e];
-      *reinterpret_cast<bf16x8v*>(krow + (int64_t)piece * 8) = f;
-    }
-    const int RB = (K + 31) / 32;
-    for (int piece = tid; piece < RB * 4 * 64; piece += NTH) {
-      const int ln = piece & 63, cs = (piece >> 6) & 3, rb = piece >> 8;
-      const int k = 32 * rb + (ln & 31), c0 = 16 * cs + 8 * (ln >> 5);
-      bf16x8v f;
-#pragma unroll
-      for (int e = 0; e < 8; ++e) f[e] = (__bf16)(k < K ? kn_s[(c0 + e) * LK + k] : 0.f);
-      *reinterpret_cast<bf16x8v*>(kcol + (int64_t)piece * 8) = f;
-    }
-  }
 
   // ---- A = strictly lower b_t e^{G_t-G_u} Kn Kn^T: waves 0-3, one 32x32 tile each.
   if (wave < 4) {
@@ -271,65 +234,21 @@ __global__ __launch_bounds__(PREP_NT, 1) void gdn_prep_mfma(gpa_gdn_problem p, g
       for (int m = 0; m < NTW; ++m) mma8(acc[m], ld_c(t_s, LT, 32 * tile_rt(m) + li, c0) * sc, bk);
     }
   }
-  if (MF) __syncthreads();  // every wave has read Kn before W takes its place
   if (own) {
     const int k = 32 * kt + li;
-    if (MF) {
-      // W rows to LDS for the fragment writers.
-#pragma unroll
-      for (int m = 0; m < NTW; ++m)
-#pragma unroll
-        for (int r = 0; r < 16; ++r) w_s[(32 * tile_rt(m) + acc_row(r, hh)) * LK + k] = acc[m][r];
-    } else if (k < K) {
+    if (k < K) {
 #pragma unroll
       for (int m = 0; m < NTW; ++m)
 #pragma unroll
         for (int r = 0; r < 16; ++r) sv.w[rows_off(s, n, nch, 32 * tile_rt(m) + acc_row(r, hh), K) + k] = acc[m][r];
     }
   }
-  __syncthreads();
-  if (MF) {
-    // Row fragments: piece (t/32, k/16, lane t%32 + 32 ((k/8) % 2)); fragment f
-    // = piece / 64 holds the 64 lanes' hi parts, then their lo parts.
-    __bf16* wrow = reinterpret_cast<__bf16*>(sv.wrow) + chunk_id * frag_row_elems(K, 16);
-    __bf16* wcol = reinterpret_cast<__bf16*>(sv.wcol) + chunk_id * frag_col_elems(K, 16);
-    for (int piece = tid; piece < 2 * K16 * 64; piece += NTH) {
-      const int ln = piece & 63, ks = (piece >> 6) % K16, rt = (piece >> 6) / K16;
-      const float* src = w_s + (32 * rt + (ln & 31)) * LK + 16 * ks + 8 * (ln >> 5);
-      bf16x8v hi, lo;
-      {
-        const float v[8] = {src[0], src[1], src[2], src[3], src[4], src[5], src[6], src[7]};
-        split8(v, hi, lo);
-      }
-      __bf16* dst = wrow + (int64_t)(piece >> 6) * 1024 + ln * 8;
-      *reinterpret_cast<bf16x8v*>(dst) = hi;
-      *reinterpret_cast<bf16x8v*>(dst + 512) = lo;
-    }
-    // Column fragments: piece (k/32, t/16, lane k%32 + 32 ((t/8) % 2)), rows t..t+7,
-    // planar like the row fragments.
-    const int RB = (K + 31) / 32;
-    for (int piece = tid; piece < RB * 4 * 64; piece += NTH) {
-      const int ln = piece & 63, cs = (piece >> 6) & 3, rb = piece >> 8;
-      const int k = 32 * rb + (ln & 31), c0 = 16 * cs + 8 * (ln >> 5);
-      bf16x8v hi, lo;
-      {
-        float v[8];
-#pragma unroll
-        for (int e = 0; e < 8; ++e) v[e] = k < K ? w_s[(c0 + e) * LK + k] : 0.f;
-        split8(v, hi, lo);
-      }
-      __bf16* dst = wcol + (int64_t)(piece >> 6) * 1024 + ln * 8;
-      *reinterpret_cast<bf16x8v*>(dst) = hi;
-      *reinterpret_cast<bf16x8v*>(dst + 512) = lo;
-    }
-  }
 
   // ---- U = T diag(b) V in slices of 128 values; every wave owns one 32x32 tile.
-  // Value-major on the FMA path, fragment order (ufrag_idx) on the MFMA path.
-  float* um = sv.u + (MF ? ufrag_off(s, n, nch, V) : vc_off(s, n, nch, V));
+  float* um = sv.u + vc_off(s, n, nch, V);
   const int urt = wave >> 2, uvt = wave & 3;
   for (int v0 = 0; v0 < V; v0 += VC) {
-    __syncthreads();  // W fragments (or the previous slice) are done with the region
+    __syncthreads();  // Kn (or the previous slice) is done with
     {
       constexpr int PER = R * VC / PREP_NT;
       float x[PER];
@@ -355,16 +274,7 @@ __global__ __launch_bounds__(PREP_NT, 1) void gdn_prep_mfma(gpa_gdn_problem p, g
       mma8(acc, ld_c(t_s, LT, 32 * urt + li, c0), ld_x(v_s, LV, 32 * uvt + li, c0));
     }
     const int v = v0 + 32 * uvt + li;
-    if (MF) {
-      // Whole 32-column strips, zero past V (the padded strip is read too).
-      const int c = (v0 + 32 * uvt) >> 5;
-      if (v0 + 32 * uvt < V) {
-#pragma unroll
-        for (int q = 0; q < 4; ++q)
-          *reinterpret_cast<f32x4*>(um + ufrag_idx(c, urt, q, lane)) =
-              v < V ? f32x4{acc[4 * q], acc[4 * q + 1], acc[4 * q + 2], acc[4 * q + 3]} : f32x4{0.f, 0.f, 0.f, 0.f};
-      }
-    } else if (v < V) {
+    if (v < V) {
 #pragma unroll
       for (int q = 0; q < 4; ++q)
         *reinterpret_cast<f32x4*>(um + (int64_t)v * R + 32 * urt + 8 * q + 4 * hh) =
@@ -373,24 +283,396 @@ __global__ __launch_bounds__(PREP_NT, 1) void gdn_prep_mfma(gpa_gdn_problem p, g
   }
 }
 
-template <typename E, int KM>
-int launch_prep_mfma(const gpa_gdn_problem& p, const gpa_gdn_saved& sv, bool mf, int nch, hipStream_t st) {
-  const size_t lds = PrepLayout<KM>::BYTES;
-  const void* fn = mf ? reinterpret_cast<const void*>(gdn_prep_mfma<E, KM, true>)
-                      : reinterpret_cast<const void*>(gdn_prep_mfma<E, KM, false>);
+// ---------------------------------------------------------------------------
+// gdn_prep_frag: the same chunk preparation for the bf16 MFMA path (bf16
+// activations, K a multiple of 16), built around the fragments it writes.  Wave w
+// holds rows 8 w .. 8 w + 7; lane (r = l/8, l%8) holds 8-key pieces (or 8-value
+// ones) of row 8 w + r, read in 16-byte loads that are all issued first.  A
+// normalised key piece is a krow piece as it stands; the 8 x 8 in-wave
+// transpose (transpose8) of a piece is a kcol / qcol piece, and of a value
+// piece the B operand of U.  krow, then kcol pass through LDS (same place) as
+// the operands of A and W.  The fp32 T enters the products as three bf16 parts
+// (all of its 24 bits; keys and values are exact), and W is formed twice, as T Kn
+// and as Kn^T T^T, so that both orders of its fragments leave the
+// accumulators after one half-wave exchange.  The barriers order LDS alone,
+// so stores drain behind the later phases.  52 KB of LDS and 80 registers at
+// 128 keys (three workgroups per compute unit), 68 KB at 256 (two).
+// Bound: HBM.  At 128 x 128 a chunk reads 48 KB and writes 176 KB: 32 streams x
+// 64 chunks take 87 us, 5.3 TB/s; the rows and fragments through float32 LDS
+// rows, with fp32 MFMA and element-wise loads and transposed stores, took 170 us.
+// K = 256, 16 streams x 32 chunks: 92 -> 40 us; one workgroup alone: 34 -> 18 us.
+__device__ __forceinline__ void swap_halves(uint32_t& x, uint32_t& y) {  // x of lanes 32..63 with y of lanes 0..31
+  const auto r = __builtin_amdgcn_permlane32_swap(x, y, false, false);
+  x = r[0];
+  y = r[1];
+}
+__device__ __forceinline__ void swap_quarters(uint32_t& x, uint32_t& y) {  // lanes 16..31 / 48..63 of x with 0..15 / 32..47 of y
+  const auto r = __builtin_amdgcn_permlane16_swap(x, y, false, false);
+  x = r[0];
+  y = r[1];
+}
+// Lanes l/8 = 0..7 of one l%8 hold the rows of an 8 x 8 bf16 matrix; returns
+// its columns the same way.  Bits 2 and 1 of the row trade places with the
+// dword index, bit 0 with the half of a dword.
+__device__ __forceinline__ uint4 transpose8(uint4 v, int lane) {
+  swap_halves(v.x, v.z);
+  swap_halves(v.y, v.w);
+  swap_quarters(v.x, v.y);
+  swap_quarters(v.z, v.w);
+  const uint32_t sel = lane & 8 ? 0x07060302u : 0x01000504u;
+  uint32_t d[4] = {v.x, v.y, v.z, v.w};
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const uint32_t other = __builtin_amdgcn_mov_dpp(d[i], 0x128, 0xf, 0xf, false);  // row_ror:8, lane ^ 8
+    d[i] = __builtin_amdgcn_perm(d[i], other, sel);
+  }
+  return make_uint4(d[0], d[1], d[2], d[3]);
+}
+
+__device__ __forceinline__ bf16x8 as_bf16x8(uint4 v) {
+  bf16x8 r;
+  __builtin_memcpy(&r, &v, 16);
+  return r;
+}
+
+// Eight floats as three bf16 parts whose sum is the float (24 bits).
+struct Split3 {
+  bf16x8 part[3];
+};
+__device__ __forceinline__ Split3 split3(const float (&x)[8]) {
+  Split3 s;
+  float y[8];
+#pragma unroll
+  for (int e = 0; e < 8; ++e) y[e] = x[e];
+#pragma unroll
+  for (int i = 0; i < 3; ++i) {
+    uint32_t w[4];
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      w[j] = bf2_pack(y[2 * j], y[2 * j + 1]);
+      y[2 * j] -= bf2_low(w[j]);
+      y[2 * j + 1] -= bf2_high(w[j]);
+    }
+    __builtin_memcpy(&s.part[i], w, 16);
+  }
+  return s;
+}
+
+// The accumulator tile's rows 16 gp .. 16 gp + 15, eight consecutive rows per lane
+// (rows + 8 in the upper lanes), as bf16 hi and lo fragment pieces.
+__device__ __forceinline__ void put_split_rows(const f32x16& acc, int gp, __bf16* frag, int lane) {
+  float v[8];
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    uint32_t x = __float_as_uint(acc[8 * gp + i]), y = __float_as_uint(acc[8 * gp + 4 + i]);
+    swap_halves(x, y);
+    v[i] = __uint_as_float(x);
+    v[4 + i] = __uint_as_float(y);
+  }
+  bf16x8 hi, lo;
+  split8(v, hi, lo);
+  *reinterpret_cast<bf16x8*>(frag + lane * 8) = hi;
+  *reinterpret_cast<bf16x8*>(frag + 512 + lane * 8) = lo;
+}
+
+template <int KM>
+struct PrepFragLayout {
+  static constexpr int FRAG = (KM < 128 ? 128 : KM) * R * 2;  // bytes of the krow / kcol fragments
+  static constexpr int T_OFF = FRAG, A_OFF = T_OFF + 4 * R * PREP_LT, SC_OFF = A_OFF + 4 * R * PREP_LT;
+  static constexpr size_t BYTES = SC_OFF + 4 * 3 * R;
+};
+
+// VEC: every row of q, k and v starts on a 16-byte boundary and V % 8 == 0.
+template <int KM, bool VEC>
+__global__ __launch_bounds__(PREP_NT, KM <= 128 ? 6 : 4) void gdn_prep_frag(gpa_gdn_problem p, gpa_gdn_saved sv, int nch) {
+  using L = PrepFragLayout<KM>;
+  constexpr int LT = PREP_LT, NP = KM / 64, VC = 128, NM = KM >= 256 ? KM / 128 : 1;
+  extern __shared__ __align__(16) unsigned char smem_b[];
+  uint4* frag_s = reinterpret_cast<uint4*>(smem_b);           // krow pieces, then kcol pieces
+  float* t_s = reinterpret_cast<float*>(smem_b + L::T_OFF);   // [R][LT] T
+  float* a_s = reinterpret_cast<float*>(smem_b + L::A_OFF);   // [R][LT] A, then the value pieces of a slice
+  uint4* vf_s = reinterpret_cast<uint4*>(smem_b + L::A_OFF);
+  float* gam_s = reinterpret_cast<float*>(smem_b + L::SC_OFF);
+  float* bet_s = gam_s + R;
+  float* sc_s = bet_s + R;  // b e^G
+
+  const int n = blockIdx.x, s = blockIdx.y, b = s / p.heads, h = s % p.heads;
+  const int K = p.kdim, V = p.vdim, tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int li = lane & 31, hh = lane >> 5, r8 = lane >> 3, pc = lane & 7;
+  const int K16 = K / 16, RB = (K + 31) / 32;
+  const int64_t chunk_id = (int64_t)s * nch + n;
+  const bool has_q = p.q.ptr != nullptr, rows16 = qk_rows_bf16(p);
+  const int row = 8 * wave + r8, tok = token_at(p, n, row);
+
+  // Eight elements of this lane's row from column d (clamped), zeros outside.
+  auto load8 = [&](const gpa_operand& o, int d, int width) {
+    const uint16_t* src = reinterpret_cast<const uint16_t*>(o.ptr) + op_base(o, b, h) + (int64_t)(tok >= 0 ? tok : 0) * o.st;
+    if (VEC) return *reinterpret_cast<const uint4*>(src + (d < width ? d : 0));
+    uint32_t w[4];
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      const int d0 = d + 2 * e, d1 = d0 + 1;
+      const uint32_t x = src[d0 < width ? d0 : 0], y = src[d1 < width ? d1 : 0];
+      w[e] = (d0 < width ? x : 0u) | (d1 < width ? y << 16 : 0u);
+    }
+    return make_uint4(w[0], w[1], w[2], w[3]);
+  };
+  const uint4 zero4 = make_uint4(0u, 0u, 0u, 0u);
+  auto keep = [&](uint4 x, int d, int width) { return tok >= 0 && d < width ? x : zero4; };
+
+  uint4 xk[NP], xq[NP], xv[2];
+#pragma unroll
+  for (int j = 0; j < NP; ++j) xk[j] = load8(p.k, 64 * j + 8 * pc, K);
+  if (has_q)
+#pragma unroll
+    for (int j = 0; j < NP; ++j) xq[j] = load8(p.q, 64 * j + 8 * pc, K);
+#pragma unroll
+  for (int j = 0; j < 2; ++j) xv[j] = load8(p.v, 64 * j + 8 * pc, V);
+
+  // ---- gates: G by a wave-wide inclusive scan (wave 0).
+  if (wave == 0) {
+    const int tg = token_at(p, n, lane), tt = tg >= 0 ? tg : 0;
+    float g = scalar_load(p.g, b, h, tt), be = scalar_load(p.beta, b, h, tt);
+    g = tg >= 0 ? g : 0.f;
+    be = tg >= 0 ? be : 0.f;
+#pragma unroll
+    for (int off = 1; off < 64; off <<= 1) {
+      const float y = __shfl_up(g, off);
+      if (lane >= off) g += y;
+    }
+    gam_s[lane] = g;
+    bet_s[lane] = be;
+    sc_s[lane] = be * __expf(g);
+    sv.gam[rows_off(s, n, nch, 0, 1) + lane] = g;
+    sv.beta[rows_off(s, n, nch, 0, 1) + lane] = be;
+  }
+  for (int i = tid; i < R * LT / 4; i += PREP_NT)  // T starts as zeros (its upper blocks stay so)
+    *reinterpret_cast<f32x4*>(t_s + 4 * i) = f32x4{0.f, 0.f, 0.f, 0.f};
+
+  // ---- normalise: x / |x| in float32, rounded to bf16.
+  auto normalise = [&](uint4 (&x)[NP]) {
+    float ss = 0.f;
+#pragma unroll
+    for (int j = 0; j < NP; ++j) {
+      x[j] = keep(x[j], 64 * j + 8 * pc, K);
+      const uint32_t w[4] = {x[j].x, x[j].y, x[j].z, x[j].w};
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const float lo = bf2_low(w[e]), hi = bf2_high(w[e]);
+        ss += lo * lo;
+        ss += hi * hi;
+      }
+    }
+    ss += __shfl_xor(ss, 1);
+    ss += __shfl_xor(ss, 2);
+    ss += __shfl_xor(ss, 4);
+    const float den = fmaxf(sqrtf(ss), 1e-6f);
+#pragma unroll
+    for (int j = 0; j < NP; ++j) {
+      uint32_t w[4] = {x[j].x, x[j].y, x[j].z, x[j].w};
+#pragma unroll
+      for (int e = 0; e < 4; ++e) w[e] = bf2_pack(bf2_low(w[e]) / den, bf2_high(w[e]) / den);
+      x[j] = make_uint4(w[0], w[1], w[2], w[3]);
+    }
+  };
+  // A normalised piece as saved rows: bf16 where the MFMA read kernels take
+  // them, else float32.
+  auto put_rows = [&](float* rows, uint4 x, int d) {
+    const int64_t at = rows_off(s, n, nch, row, K) + d;
+    if (rows16) {
+      *reinterpret_cast<uint4*>(reinterpret_cast<bf16_t*>(rows) + at) = x;
+    } else {
+      const uint32_t w[4] = {x.x, x.y, x.z, x.w};
+#pragma unroll
+      for (int e = 0; e < 2; ++e)
+        *reinterpret_cast<f32x4*>(rows + at + 4 * e) = f32x4{bf2_low(w[2 * e]), bf2_high(w[2 * e]),
+                                                             bf2_low(w[2 * e + 1]), bf2_high(w[2 * e + 1])};
+    }
+  };
+  // Place of this lane's transposed piece j in a column-fragment buffer.
+  auto col_piece = [&](int k) { return ((k >> 5) * 4 + (wave >> 1)) * 64 + (k & 31) + 32 * (wave & 1); };
+  normalise(xk);
+  {
+    uint4* krow = reinterpret_cast<uint4*>(reinterpret_cast<__bf16*>(sv.krow) + chunk_id * frag_row_elems(K, 8));
+    uint4* kcol = reinterpret_cast<uint4*>(reinterpret_cast<__bf16*>(sv.kcol) + chunk_id * frag_col_elems(K, 8));
+#pragma unroll
+    for (int j = 0; j < NP; ++j) {
+      const int d = 64 * j + 8 * pc, k = d + r8;
+      if (d < K) {
+        const int piece = ((row >> 5) * K16 + (d >> 4)) * 64 + (row & 31) + 32 * ((d >> 3) & 1);
+        frag_s[piece] = xk[j];
+        krow[piece] = xk[j];
+        if (!rows16) put_rows(sv.kn, xk[j], d);
+      }
+      xk[j] = transpose8(xk[j], lane);
+      if (k < 32 * RB) kcol[col_piece(k)] = xk[j];
+    }
+  }
+  lds_barrier();
+  // ---- A = strictly lower b_t e^{G_t-G_u} Kn Kn^T: waves 0-2, one 32x32 tile each.
+  if (wave < 3) {
+    const int rr = (wave + 1) >> 1, ru = wave >> 1;  // (0, 0), (1, 0), (1, 1)
+    f32x16 acc = {};
+#pragma unroll 4
+    for (int g = 0; g < K16; ++g)
+      mma_bf16(acc, as_bf16x8(frag_s[(rr * K16 + g) * 64 + lane]), as_bf16x8(frag_s[(ru * K16 + g) * 64 + lane]));
+    const int u = 32 * ru + li;
+#pragma unroll
+    for (int r = 0; r < 16; ++r) {
+      const int t = 32 * rr + acc_row(r, hh);
+      a_s[t * LT + u] = (u < t) ? bet_s[t] * __expf(gam_s[t] - gam_s[u]) * acc[r] : 0.f;
+    }
+  }
+  if (has_q) {
+    normalise(xq);
+    uint4* qcol = reinterpret_cast<uint4*>(reinterpret_cast<__bf16*>(sv.qcol) + chunk_id * frag_col_elems(K, 8));
+#pragma unroll
+    for (int j = 0; j < NP; ++j) {
+      const int d = 64 * j + 8 * pc, k = d + r8;
+      if (d < K) put_rows(sv.qn, xq[j], d);
+      xq[j] = transpose8(xq[j], lane);
+      if (k < 32 * RB) qcol[col_piece(k)] = xq[j];
+    }
+  }
+  lds_barrier();
+#pragma unroll
+  for (int j = 0; j < NP; ++j) {
+    const int k = 64 * j + 8 * pc + r8;
+    if (k < 32 * RB) frag_s[col_piece(k)] = xk[j];
+  }
+  unit_lower_inverse(a_s, t_s, wave, lane);
+
+  // ---- V pieces of a slice (in A's place), T out, W = T diag(b e^G) Kn.
+  auto put_values = [&](int v0) {
+#pragma unroll
+    for (int j = 0; j < 2; ++j) {
+      const int d = 64 * j + 8 * pc;
+      vf_s[col_piece(d + r8)] = transpose8(keep(xv[j], v0 + d, V), lane);
+    }
+  };
+  put_values(0);
+  if (VC < V)
+#pragma unroll
+    for (int j = 0; j < 2; ++j) xv[j] = load8(p.v, VC + 64 * j + 8 * pc, V);
+  {
+    float* tri = sv.tri + rows_off(s, n, nch, 0, R);
+    for (int i = tid; i < R * R / 4; i += PREP_NT) {
+      const int t = i / (R / 4), c = 4 * (i % (R / 4));
+      *reinterpret_cast<f32x4*>(tri + t * R + c) = *reinterpret_cast<const f32x4*>(t_s + t * LT + c);
+    }
+  }
+  // T rows 32 rt + l%32, columns 16 ks + 8 (l/32) .. +7, scaled per column.
+  const int rt = wave & 1, w4 = wave >> 1;
+  auto t_parts = [&](const float* scale, int ks) {
+    const int c0 = 16 * ks + 8 * hh;
+    const float* t = t_s + (32 * rt + li) * LT + c0;
+    float x[8];
+#pragma unroll
+    for (int e = 0; e < 2; ++e) {
+      const f32x4 y = *reinterpret_cast<const f32x4*>(t + 4 * e) * *reinterpret_cast<const f32x4*>(scale + c0 + 4 * e);
+#pragma unroll
+      for (int i = 0; i < 4; ++i) x[4 * e + i] = y[i];
+    }
+    return split3(x);
+  };
+  if (w4 < RB) {
+    f32x16 w[NM], wt[NM];
+#pragma unroll
+    for (int m = 0; m < NM; ++m) w[m] = wt[m] = f32x16{};
+#pragma unroll
+    for (int ks = 0; ks < 4; ++ks) {
+      if (ks >= 2 + 2 * rt) continue;  // T is lower triangular
+      const Split3 t = t_parts(sc_s, ks);
+#pragma unroll
+      for (int m = 0; m < NM; ++m) {
+        if (w4 + 4 * m >= RB) continue;
+        const bf16x8 k = as_bf16x8(frag_s[((w4 + 4 * m) * 4 + ks) * 64 + lane]);
+#pragma unroll
+        for (int i = 0; i < 3; ++i) {
+          mma_bf16(w[m], t.part[i], k);
+          mma_bf16(wt[m], k, t.part[i]);
+        }
+      }
+    }
+    __bf16* wrow = reinterpret_cast<__bf16*>(sv.wrow) + chunk_id * frag_row_elems(K, 16);
+    __bf16* wcol = reinterpret_cast<__bf16*>(sv.wcol) + chunk_id * frag_col_elems(K, 16);
+#pragma unroll
+    for (int m = 0; m < NM; ++m) {
+      const int kt = w4 + 4 * m;
+      if (kt >= RB) continue;
+#pragma unroll
+      for (int gp = 0; gp < 2; ++gp) {
+        put_split_rows(w[m], gp, wcol + (int64_t)(kt * 4 + 2 * rt + gp) * 1024, lane);
+        if (2 * kt + gp < K16) put_split_rows(wt[m], gp, wrow + (int64_t)(rt * K16 + 2 * kt + gp) * 1024, lane);
+      }
+    }
+  }
+
+  // ---- U = T diag(b) V in slices of 128 values; every wave owns one 32x32 tile.
+  float* um = sv.u + ufrag_off(s, n, nch, V);
+  for (int v0 = 0; v0 < V; v0 += VC) {
+    if (v0) {
+      lds_barrier();  // every wave is done with the previous slice
+      put_values(v0);
+      if (v0 + VC < V)
+#pragma unroll
+        for (int j = 0; j < 2; ++j) xv[j] = load8(p.v, v0 + VC + 64 * j + 8 * pc, V);
+    }
+    lds_barrier();
+    if (v0 + 32 * w4 < V) {
+      f32x16 acc = {};
+#pragma unroll
+      for (int ks = 0; ks < 4; ++ks) {
+        if (ks >= 2 + 2 * rt) continue;
+        const Split3 t = t_parts(bet_s, ks);
+        const bf16x8 x = as_bf16x8(vf_s[(w4 * 4 + ks) * 64 + lane]);
+#pragma unroll
+        for (int i = 0; i < 3; ++i) mma_bf16(acc, t.part[i], x);
+      }
+      // Whole 32-column strips, zero past V (the padded strip is read too).
+      const bool ok = v0 + 32 * w4 + li < V;
+#pragma unroll
+      for (int q = 0; q < 4; ++q)
+        *reinterpret_cast<f32x4*>(um + ufrag_idx((v0 >> 5) + w4, rt, q, lane)) =
+            ok ? f32x4{acc[4 * q], acc[4 * q + 1], acc[4 * q + 2], acc[4 * q + 3]} : f32x4{0.f, 0.f, 0.f, 0.f};
+    }
+  }
+}
+
+// Rows of a bf16 operand all start on 16-byte boundaries.
+bool rows_aligned(const gpa_operand& o) {
+  return reinterpret_cast<uintptr_t>(o.ptr) % 16 == 0 && o.sb % 8 == 0 && o.st % 8 == 0 && o.sh % 8 == 0;
+}
+
+template <int KM>
+int launch_prep_frag(const gpa_gdn_problem& p, const gpa_gdn_saved& sv, int nch, hipStream_t st) {
+  const bool vec = rows_aligned(p.k) && rows_aligned(p.v) && p.vdim % 8 == 0 && (!p.q.ptr || rows_aligned(p.q));
+  const size_t lds = PrepFragLayout<KM>::BYTES;
+  const void* fn = vec ? reinterpret_cast<const void*>(gdn_prep_frag<KM, true>)
+                       : reinterpret_cast<const void*>(gdn_prep_frag<KM, false>);
   if (lds > 65536 &&
       hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds) != hipSuccess)
     return fail(GPA_HIP_EHIP, "hipFuncSetAttribute(max dynamic LDS) failed");
   const dim3 grid(nch, p.batch * p.heads), block(PREP_NT);
-  if (mf)
-    hipLaunchKernelGGL((gdn_prep_mfma<E, KM, true>), grid, block, lds, st, p, sv, nch);
-  else
-    hipLaunchKernelGGL((gdn_prep_mfma<E, KM, false>), grid, block, lds, st, p, sv, nch);
+  if (vec) hipLaunchKernelGGL((gdn_prep_frag<KM, true>), grid, block, lds, st, p, sv, nch);
+  else hipLaunchKernelGGL((gdn_prep_frag<KM, false>), grid, block, lds, st, p, sv, nch);
+  return GPA_HIP_OK;
+}
+
+template <typename E, int KM>
+int launch_prep(const gpa_gdn_problem& p, const gpa_gdn_saved& sv, int nch, hipStream_t st) {
+  if constexpr (std::is_same<E, bf16_t>::value)
+    if (p.kdim % 16 == 0) return launch_prep_frag<KM>(p, sv, nch, st);
+  const size_t lds = PrepLayout<KM>::BYTES;
+  if (lds > 65536 && hipFuncSetAttribute(reinterpret_cast<const void*>(gdn_prep_mfma<E, KM>),
+                                         hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds) != hipSuccess)
+    return fail(GPA_HIP_EHIP, "hipFuncSetAttribute(max dynamic LDS) failed");
+  hipLaunchKernelGGL((gdn_prep_mfma<E, KM>), dim3(nch, p.batch * p.heads), dim3(PREP_NT), lds, st, p, sv, nch);
   return GPA_HIP_OK;
 }
 
 #define GPA_PREP_MFMA(E, KM) \
-  template int launch_prep_mfma<E, KM>(const gpa_gdn_problem&, const gpa_gdn_saved&, bool, int, hipStream_t);
+  template int launch_prep<E, KM>(const gpa_gdn_problem&, const gpa_gdn_saved&, int, hipStream_t);
 GPA_PREP_MFMA(float, 64)
 GPA_PREP_MFMA(float, 128)
 GPA_PREP_MFMA(float, 256)

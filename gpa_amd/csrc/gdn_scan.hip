@@ -8,7 +8,7 @@
 //   O = diag(e^G) Q S_n + (causal e^{G_t-G_s} Q K^T) D,
 //   S_{n+1} = e^{G_C} S_n + (diag(e^{G_C-G}) K)^T D.
 // Kernels:
-//   gdn_prep_mfma  chunk-parallel: normalise, G, T, W, U (gdn_prep_mfma.hip)
+//   gdn_prep_*     chunk-parallel: normalise, G, T, W, U (gdn_prep_mfma.hip)
 //   gdn_state_fwd  sequential over chunks, parallel over (stream, 16-column tile):
 //                  S_n (saved), D
 //   gdn_out_fwd    chunk-parallel: O
@@ -1009,7 +1009,7 @@ int allow_lds(F kernel, size_t bytes) {
 
 template <typename E, int KM>
 int fwd_prep(const gpa_gdn_problem& p, const gpa_gdn_saved& sv, int nch, hipStream_t st) {
-  return launch_prep_mfma<E, KM>(p, sv, use_mfma<E>(p), nch, st);
+  return launch_prep<E, KM>(p, sv, nch, st);
 }
 
 // A problem whose state recurrence runs on the strip kernels (bf16 MFMA, K <= 128).

@@ -112,7 +112,7 @@ def kernel_timer():
 
 def _prep(k, v, c, tokens, dtype):
     e, km = _tag(dtype), _kmax(k)
-    return (f"gdn_prep_mfma<{e},{km},{'true' if _mfma(k, dtype) else 'false'}>",
+    return (f"gdn_prep_frag<{km}>" if _mfma(k, dtype) else f"gdn_prep_mfma<{e},{km}>",
             (4 * c * k + 2 * c * v + c * c / 3) * tokens)
 
 

@@ -161,6 +161,37 @@ inline uint32_t emu_perm(uint32_t a, uint32_t b, uint32_t sel) {
 #define __builtin_amdgcn_mfma_f32_32x32x2f32(a, b, c, x, y, z) emu_mfma_32x32x2_f32(a, b, c)
 #define __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, x, y, z) emu_mfma_16x16x4_f32(a, b, c)
 
+// v_permlane32_swap / v_permlane16_swap: the upper half (odd 16-lane rows) of
+// the first operand trades places with the lower half (even rows) of the second.
+struct emu_pair {
+  uint32_t v[2];
+  uint32_t operator[](int i) const { return v[i]; }
+};
+inline emu_pair emu_permlane_swap(uint32_t x, uint32_t y, int n) {
+  float fx, fy;
+  memcpy(&fx, &x, 4);
+  memcpy(&fy, &y, 4);
+  const float px = __shfl_xor(fx, n), py = __shfl_xor(fy, n);
+  emu_pair r{{x, y}};
+  memcpy(threadIdx.x & n ? &r.v[0] : &r.v[1], threadIdx.x & n ? &py : &px, 4);
+  return r;
+}
+#define __builtin_amdgcn_permlane32_swap(x, y, a, b) emu_permlane_swap(x, y, 32)
+#define __builtin_amdgcn_permlane16_swap(x, y, a, b) emu_permlane_swap(x, y, 16)
+// The DPP control in use: row_ror:8, the value of lane l ^ 8.
+inline uint32_t emu_row_ror8(uint32_t x) {
+  float f;
+  memcpy(&f, &x, 4);
+  f = __shfl_xor(f, 8);
+  memcpy(&x, &f, 4);
+  return x;
+}
+#define __builtin_amdgcn_mov_dpp(x, ctrl, rm, bm, bc) (static_assert_dpp<ctrl>(), emu_row_ror8(x))
+template <int C>
+inline void static_assert_dpp() {
+  static_assert(C == 0x128, "row_ror:8 only");
+}
+
 // Dynamic LDS: an allocation of exactly the launch's size per workgroup.
 extern char* emu_dynamic_lds;
 #define HIP_DYNAMIC_SHARED(type, var) type* var = reinterpret_cast<type*>(emu_dynamic_lds);
