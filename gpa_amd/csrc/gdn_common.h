@@ -186,6 +186,15 @@ int launch_out_mfma(const gpa_gdn_problem& p, const gpa_gdn_saved& sv, gpa_opera
 template <int KM>
 int launch_dd0_mfma(const gpa_gdn_problem& p, const gpa_gdn_saved& sv, const gpa_gdn_grads& gr, int nch,
                     hipStream_t st);
+// Rows of a bf16 operand all start on 16-byte boundaries.
+inline bool rows_aligned(const gpa_operand& o) {
+  return reinterpret_cast<uintptr_t>(o.ptr) % 16 == 0 && o.sb % 8 == 0 && o.st % 8 == 0 && o.sh % 8 == 0;
+}
+// Chunk backward of the bf16 MFMA path (gdn_chunk_bwd_frag.hip); needs kdim % 16
+// == 0, vdim % 8 == 0 and aligned rows of k, dk, dq and, with a read, q and dout.
+template <int KM>
+int launch_chunk_bwd_frag(const gpa_gdn_problem& p, const gpa_gdn_saved& sv, const gpa_gdn_grads& gr, int nch,
+                          hipStream_t st);
 // fp32-MFMA chunk backward (gdn_chunk_bwd_mfma.hip); needs kdim % 4 == 0.
 template <typename E, int KM>
 int launch_chunk_bwd_mfma(const gpa_gdn_problem& p, const gpa_gdn_saved& sv, const gpa_gdn_grads& gr, int nch,

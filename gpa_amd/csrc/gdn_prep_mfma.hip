@@ -301,16 +301,6 @@ __global__ __launch_bounds__(PREP_NT, 1) void gdn_prep_mfma(gpa_gdn_problem p, g
 // 64 chunks take 87 us, 5.3 TB/s; the rows and fragments through float32 LDS
 // rows, with fp32 MFMA and element-wise loads and transposed stores, took 170 us.
 // K = 256, 16 streams x 32 chunks: 92 -> 40 us; one workgroup alone: 34 -> 18 us.
-__device__ __forceinline__ void swap_halves(uint32_t& x, uint32_t& y) {  // x of lanes 32..63 with y of lanes 0..31
-  const auto r = __builtin_amdgcn_permlane32_swap(x, y, false, false);
-  x = r[0];
-  y = r[1];
-}
-__device__ __forceinline__ void swap_quarters(uint32_t& x, uint32_t& y) {  // lanes 16..31 / 48..63 of x with 0..15 / 32..47 of y
-  const auto r = __builtin_amdgcn_permlane16_swap(x, y, false, false);
-  x = r[0];
-  y = r[1];
-}
 // Lanes l/8 = 0..7 of one l%8 hold the rows of an 8 x 8 bf16 matrix; returns
 // its columns the same way.  Bits 2 and 1 of the row trade places with the
 // dword index, bit 0 with the half of a dword.
@@ -323,7 +313,7 @@ __device__ __forceinline__ uint4 transpose8(uint4 v, int lane) {
   uint32_t d[4] = {v.x, v.y, v.z, v.w};
 #pragma unroll
   for (int i = 0; i < 4; ++i) {
-    const uint32_t other = __builtin_amdgcn_mov_dpp(d[i], 0x128, 0xf, 0xf, false);  // row_ror:8, lane ^ 8
+    const uint32_t other = __builtin_amdgcn_mov_dpp(d[i], DPP_XOR8, 0xf, 0xf, false);
     d[i] = __builtin_amdgcn_perm(d[i], other, sel);
   }
   return make_uint4(d[0], d[1], d[2], d[3]);
@@ -361,18 +351,9 @@ __device__ __forceinline__ Split3 split3(const float (&x)[8]) {
 // The accumulator tile's rows 16 gp .. 16 gp + 15, eight consecutive rows per lane
 // (rows + 8 in the upper lanes), as bf16 hi and lo fragment pieces.
 __device__ __forceinline__ void put_split_rows(const f32x16& acc, int gp, __bf16* frag, int lane) {
-  float v[8];
-#pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    uint32_t x = __float_as_uint(acc[8 * gp + i]), y = __float_as_uint(acc[8 * gp + 4 + i]);
-    swap_halves(x, y);
-    v[i] = __uint_as_float(x);
-    v[4 + i] = __uint_as_float(y);
-  }
-  bf16x8 hi, lo;
-  split8(v, hi, lo);
-  *reinterpret_cast<bf16x8*>(frag + lane * 8) = hi;
-  *reinterpret_cast<bf16x8*>(frag + 512 + lane * 8) = lo;
+  const SplitBf8 x = split_rows(acc, gp);
+  *reinterpret_cast<bf16x8*>(frag + lane * 8) = x.hi;
+  *reinterpret_cast<bf16x8*>(frag + 512 + lane * 8) = x.lo;
 }
 
 template <int KM>
@@ -637,11 +618,6 @@ __global__ __launch_bounds__(PREP_NT, KM <= 128 ? 6 : 4) void gdn_prep_frag(gpa_
             ok ? f32x4{acc[4 * q], acc[4 * q + 1], acc[4 * q + 2], acc[4 * q + 3]} : f32x4{0.f, 0.f, 0.f, 0.f};
     }
   }
-}
-
-// Rows of a bf16 operand all start on 16-byte boundaries.
-bool rows_aligned(const gpa_operand& o) {
-  return reinterpret_cast<uintptr_t>(o.ptr) % 16 == 0 && o.sb % 8 == 0 && o.st % 8 == 0 && o.sh % 8 == 0;
 }
 
 template <int KM>

@@ -1113,6 +1113,11 @@ int bwd_state(const gpa_gdn_problem& p, const gpa_gdn_saved& sv, const gpa_gdn_g
 
 template <typename E, int KM>
 int bwd_chunk(const gpa_gdn_problem& p, const gpa_gdn_saved& sv, const gpa_gdn_grads& gr, int nch, hipStream_t st) {
+  if constexpr (std::is_same<E, bf16_t>::value) {
+    const bool rows = rows_aligned(p.k) && rows_aligned(gr.dk) && (!p.q.ptr || !gr.dq.ptr || rows_aligned(gr.dq)) &&
+                      (!has_read(p, gr) || (rows_aligned(p.q) && rows_aligned(gr.dout)));
+    if (use_mfma<E>(p) && p.vdim % 8 == 0 && rows) return launch_chunk_bwd_frag<KM>(p, sv, gr, nch, st);
+  }
   // The MFMA chunk kernel keeps 64 x 256 fp32 rows in LDS only for bf16.
   constexpr bool mfma_chunk = !(std::is_same<E, float>::value && KM == 256);
   if (mfma_chunk && p.kdim % 4 == 0) {

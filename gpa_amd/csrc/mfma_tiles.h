@@ -48,34 +48,80 @@ __device__ __forceinline__ f32x4 ld_x(const float* m, int ld, int x, int c0) {
 
 __device__ __forceinline__ int acc_row(int r, int half) { return 8 * (r >> 2) + 4 * half + (r & 3); }
 
+// x of lanes 32..63 trades places with y of lanes 0..31 ...
+__device__ __forceinline__ void swap_halves(uint32_t& x, uint32_t& y) {
+  const auto r = __builtin_amdgcn_permlane32_swap(x, y, false, false);
+  x = r[0];
+  y = r[1];
+}
+// ... and x of lanes 16..31, 48..63 with y of lanes 0..15, 32..47.
+__device__ __forceinline__ void swap_quarters(uint32_t& x, uint32_t& y) {
+  const auto r = __builtin_amdgcn_permlane16_swap(x, y, false, false);
+  x = r[0];
+  y = r[1];
+}
+// The value of another lane of the row of 16: l ^ 8, l ^ 7, l ^ 3, l ^ 2, l ^ 1.
+constexpr int DPP_XOR8 = 0x128, DPP_XOR7 = 0x141, DPP_XOR3 = 0x1b, DPP_XOR2 = 0x4e, DPP_XOR1 = 0xb1;
+template <int CTRL>
+__device__ __forceinline__ float dpp(float x) {
+  return __uint_as_float(__builtin_amdgcn_mov_dpp(__float_as_uint(x), CTRL, 0xf, 0xf, false));
+}
+
+__device__ __forceinline__ uint32_t dpp_xor4(uint32_t x) {
+  return __builtin_amdgcn_mov_dpp(__builtin_amdgcn_mov_dpp(x, DPP_XOR7, 0xf, 0xf, false), DPP_XOR3, 0xf, 0xf, false);
+}
+// Eight consecutive lanes hold the rows of an 8 x 8 bf16 matrix; returns its
+// columns the same way.  Bits 2 and 1 of the row trade places with the dword
+// index, bit 0 with the half of a dword.
+__device__ __forceinline__ uint4 transpose8_lanes(uint4 v, int lane) {
+  uint32_t d[4] = {v.x, v.y, v.z, v.w};
+#pragma unroll
+  for (int i = 0; i < 2; ++i) {
+    const bool up = lane & 4;
+    const uint32_t got = dpp_xor4(up ? d[i] : d[i + 2]);
+    d[i] = up ? got : d[i];
+    d[i + 2] = up ? d[i + 2] : got;
+  }
+#pragma unroll
+  for (int i = 0; i < 4; i += 2) {
+    const bool up = lane & 2;
+    const uint32_t got = __builtin_amdgcn_mov_dpp(up ? d[i] : d[i + 1], DPP_XOR2, 0xf, 0xf, false);
+    d[i] = up ? got : d[i];
+    d[i + 1] = up ? d[i + 1] : got;
+  }
+  const uint32_t sel = lane & 1 ? 0x07060302u : 0x01000504u;
+#pragma unroll
+  for (int i = 0; i < 4; ++i)
+    d[i] = __builtin_amdgcn_perm(d[i], __builtin_amdgcn_mov_dpp(d[i], DPP_XOR1, 0xf, 0xf, false), sel);
+  return make_uint4(d[0], d[1], d[2], d[3]);
+}
+
 // Sums of each of a lane's 16 accumulator-row values over the 32 lanes of its
-// half-wave, by recursive halving (16 exchanges instead of 16 x 5).  Every
-// lane returns the sum for register index sum_index(lane).
+// half-wave, by recursive halving (lanes l ^ 16, 8, 7, 2, 1) without LDS.
+// Every lane returns the sum for register index sum_index(lane).
 __device__ __forceinline__ float tile_row_sum(float (&v)[16], int lane) {
 #pragma unroll
   for (int j = 0; j < 8; ++j) {
-    const bool up = lane & 16;
-    const float send = up ? v[j] : v[j + 8], keep = up ? v[j + 8] : v[j];
-    v[j] = keep + __shfl_xor(send, 16);
+    uint32_t x = __float_as_uint(v[j]), y = __float_as_uint(v[j + 8]);
+    swap_quarters(x, y);
+    v[j] = __uint_as_float(x) + __uint_as_float(y);
   }
 #pragma unroll
   for (int j = 0; j < 4; ++j) {
     const bool up = lane & 8;
     const float send = up ? v[j] : v[j + 4], keep = up ? v[j + 4] : v[j];
-    v[j] = keep + __shfl_xor(send, 8);
+    v[j] = keep + dpp<DPP_XOR8>(send);
   }
 #pragma unroll
   for (int j = 0; j < 2; ++j) {
     const bool up = lane & 4;
     const float send = up ? v[j] : v[j + 2], keep = up ? v[j + 2] : v[j];
-    v[j] = keep + __shfl_xor(send, 4);
+    v[j] = keep + dpp<DPP_XOR7>(send);
   }
-  {
-    const bool up = lane & 2;
-    const float send = up ? v[0] : v[1], keep = up ? v[1] : v[0];
-    v[0] = keep + __shfl_xor(send, 2);
-  }
-  return v[0] + __shfl_xor(v[0], 1);
+  const bool up = lane & 2;
+  const float send = up ? v[0] : v[1], keep = up ? v[1] : v[0];
+  v[0] = keep + dpp<DPP_XOR2>(send);
+  return v[0] + dpp<DPP_XOR1>(v[0]);
 }
 __device__ __forceinline__ int sum_index(int lane) {
   return 8 * ((lane >> 4) & 1) + 4 * ((lane >> 3) & 1) + 2 * ((lane >> 2) & 1) + ((lane >> 1) & 1);
@@ -118,6 +164,21 @@ __device__ __forceinline__ void split8(const float (&x)[8], bf16x8& hi, bf16x8& 
   for (int i = 0; i < 4; ++i) bf2_split(x[2 * i], x[2 * i + 1], h[i], o[i]);
   __builtin_memcpy(&hi, h, 16);
   __builtin_memcpy(&lo, o, 16);
+}
+// Rows 16 gp .. 16 gp + 15 of an accumulator tile, eight consecutive rows per
+// lane (those + 8 in the upper lanes), split into bf16 hi and lo.
+__device__ __forceinline__ SplitBf8 split_rows(const f32x16& acc, int gp) {
+  float v[8];
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    uint32_t x = __float_as_uint(acc[8 * gp + i]), y = __float_as_uint(acc[8 * gp + 4 + i]);
+    swap_halves(x, y);
+    v[i] = __uint_as_float(x);
+    v[4 + i] = __uint_as_float(y);
+  }
+  SplitBf8 s;
+  split8(v, s.hi, s.lo);
+  return s;
 }
 __device__ __forceinline__ SplitBf8 split_bf8(const float (&x)[8]) {
   SplitBf8 s;

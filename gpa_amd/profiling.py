@@ -112,7 +112,7 @@ def kernel_timer():
 
 def _prep(k, v, c, tokens, dtype):
     e, km = _tag(dtype), _kmax(k)
-    return (f"gdn_prep_frag<{km}>" if _mfma(k, dtype) else f"gdn_prep_mfma<{e},{km}>",
+    return (f"gdn_prep_frag<{km},true>" if _mfma(k, dtype) else f"gdn_prep_mfma<{e},{km}>",
             (4 * c * k + 2 * c * v + c * c / 3) * tokens)
 
 
@@ -152,6 +152,8 @@ def _chunk_bwd(k, v, c, tokens, dtype, read):
     flop = 4 * k * v + 4 * c * v + 4 * c * k + 2 * c * c
     if read:
         flop += 2 * k * v + 2 * c * v + 6 * c * k
+    if _mfma(k, dtype) and v % 8 == 0:  # (16-byte aligned rows, as the module's are)
+        return f"gdn_chunk_bwd_frag<{km},{'true' if read else 'false'}>", flop * tokens
     mfma_chunk = k % 4 == 0 and not (km == 256 and e == "f32")
     return f"{'gdn_chunk_bwd_mfma' if mfma_chunk else 'gdn_chunk_bwd'}<{e},{km}>", flop * tokens
 

@@ -35,7 +35,7 @@ ENTRIES = {"gpa_decode_step": 0, "gpa_route_forward": 1, "gpa_route_backward": 2
 SOURCES = ["gpa_decode.hip", "route_reader.hip", "level_mix.hip", "gdn_token.hip", "level_token.hip",
            "product_read.hip", "slot_gates.hip", "moment_scan.hip",
            "quad_features.hip", "gdn_scan.hip", "gdn_prep_mfma.hip", "gdn_state_mfma.hip", "gdn_out_mfma.hip",
-           "gdn_chunk_bwd_mfma.hip"]
+           "gdn_chunk_bwd_mfma.hip", "gdn_chunk_bwd_frag.hip"]
 # Test-side sources of the host build: stand-ins for kernels it does not emulate.
 HOST_SOURCES = ["strip_absent.cpp"]
 

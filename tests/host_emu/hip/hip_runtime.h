@@ -178,19 +178,18 @@ inline emu_pair emu_permlane_swap(uint32_t x, uint32_t y, int n) {
 }
 #define __builtin_amdgcn_permlane32_swap(x, y, a, b) emu_permlane_swap(x, y, 32)
 #define __builtin_amdgcn_permlane16_swap(x, y, a, b) emu_permlane_swap(x, y, 16)
-// The DPP control in use: row_ror:8, the value of lane l ^ 8.
-inline uint32_t emu_row_ror8(uint32_t x) {
+// The DPP controls in use: row_ror:8, row_half_mirror, quad_perm [3,2,1,0],
+// [2,3,0,1] and [1,0,3,2], the value of lane l ^ 8, 7, 3, 2, 1.
+template <int C>
+inline uint32_t emu_mov_dpp(uint32_t x) {
+  static_assert(C == 0x128 || C == 0x141 || C == 0x1b || C == 0x4e || C == 0xb1, "DPP control");
   float f;
   memcpy(&f, &x, 4);
-  f = __shfl_xor(f, 8);
+  f = __shfl_xor(f, C == 0x128 ? 8 : C == 0x141 ? 7 : C == 0x1b ? 3 : C == 0x4e ? 2 : 1);
   memcpy(&x, &f, 4);
   return x;
 }
-#define __builtin_amdgcn_mov_dpp(x, ctrl, rm, bm, bc) (static_assert_dpp<ctrl>(), emu_row_ror8(x))
-template <int C>
-inline void static_assert_dpp() {
-  static_assert(C == 0x128, "row_ror:8 only");
-}
+#define __builtin_amdgcn_mov_dpp(x, ctrl, rm, bm, bc) emu_mov_dpp<ctrl>(x)
 
 // Dynamic LDS: an allocation of exactly the launch's size per workgroup.
 extern char* emu_dynamic_lds;
