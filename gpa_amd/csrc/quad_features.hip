@@ -8,7 +8,7 @@
 // as 16-byte rows of a transposed, zero-padded copy (the caller prepares it:
 // the weights are parameters, a few hundred KB).  Wave w owns the column
 // blocks w, w + 4 of both products, so a and b of an element meet in one
-// lane's accumulators; row sums go through half-wave shuffles and LDS.
+// lane's accumulators; row sums go through the half-wave and LDS.
 //
 // The backward recomputes the forward, forms dz through the two
 // normalisations, da = (dz b) c and db = dz (c a) rounded to E, and
@@ -18,6 +18,8 @@
 // batched GEMM the caller runs) and one partial sum of dc per workgroup.
 #include <hip/hip_runtime.h>
 
+#include <initializer_list>
+
 #include "mfma_tiles.h"
 
 namespace gpa {
@@ -25,28 +27,34 @@ namespace {
 
 constexpr int QT = 256;   // threads per workgroup (4 waves)
 constexpr int QR = 32;    // rows per workgroup
-constexpr int QMAXB = 2;  // column blocks per wave (dim <= 256)
+// (column blocks per wave, QB: 1 up to 128 columns, else 2)
 
 __host__ __device__ inline int qpad(int d) { return (d + 31) / 32 * 32; }
 __device__ __forceinline__ int qmin(int a, int b) { return a < b ? a : b; }
 
+// LDS: rows of u, and for the backward of x, dout (then dx) and [da | db], each
+// row padded by 16 bytes; per-row scalars.
 template <typename E>
 struct QLayout {
   int DP, NB, ULD, DLD;
-  E* u;        // [32][ULD]  unit(x) rows
-  E* dab;      // [32][DLD]  d(a) | d(b) rows (backward)
-  float* nrm;  // [32] ||x||_eps = sqrt(sum x^2 + 1e-12)
-  float* xn;   // [32] sqrt(sum x^2)
-  float* part; // [3][8][32] per-block row partial sums
-  float* row;  // [3][32] row totals
-  float* wsum; // [4] per-wave partial of dc
+  E* u;         // [32][ULD] unit(x) rows, then the output rows (out, dx)
+  E* x;         // [32][ULD] raw rows, zeros past dim and past the last row
+  E* g;         // [32][ULD] dout rows, the same, in dab's place until dab is formed
+  E* dab;       // [32][DLD] d(a) | d(b) rows
+  float* nrm;   // [32] ||x||_eps = sqrt(sum x^2 + 1e-12)
+  float* xn;    // [32] sqrt(sum x^2)
+  float* part;  // [8][32] per-block row partial sums
+  float* ra;    // [32] row factors of the phase at hand
+  float* rb;
+  float* dn;    // [32] d ||x||_eps / ||x||_eps
+  float* wsum;  // [4] per-wave partial of dc
 };
 
 template <typename E>
 __host__ __device__ inline size_t q_lds_bytes(int dim, bool backward) {
   const int DP = qpad(dim), ULD = DP + 16 / (int)sizeof(E), DLD = 2 * DP + 16 / (int)sizeof(E);
-  size_t b = (size_t)QR * ULD * sizeof(E) + (backward ? (size_t)QR * DLD * sizeof(E) : 0);
-  return b + (2 * QR + 3 * 8 * QR + 3 * QR + 4) * sizeof(float);
+  const size_t b = (size_t)QR * ULD * sizeof(E) * (backward ? 2 : 1) + (backward ? (size_t)QR * DLD * sizeof(E) : 0);
+  return b + (5 * QR + 8 * QR + 4) * sizeof(float);
 }
 
 template <typename E>
@@ -56,49 +64,135 @@ __device__ QLayout<E> q_layout(char* smem, int dim, bool backward) {
   L.NB = L.DP / 32;
   L.ULD = L.DP + 16 / (int)sizeof(E);
   L.DLD = 2 * L.DP + 16 / (int)sizeof(E);
-  char* p = smem;
-  L.u = reinterpret_cast<E*>(p);
-  p += (size_t)QR * L.ULD * sizeof(E);
-  L.dab = reinterpret_cast<E*>(p);
-  if (backward) p += (size_t)QR * L.DLD * sizeof(E);
-  float* f = reinterpret_cast<float*>(p);
+  E* e = reinterpret_cast<E*>(smem);
+  L.u = e;
+  e += QR * L.ULD;
+  L.x = L.g = L.dab = e;
+  if (backward) {
+    L.g = L.dab = L.x + QR * L.ULD;
+    e = L.dab + QR * L.DLD;
+  }
+  float* f = reinterpret_cast<float*>(e);
   L.nrm = f;
   L.xn = f + QR;
-  L.part = f + 2 * QR;
-  L.row = L.part + 3 * 8 * QR;
-  L.wsum = L.row + 3 * QR;
+  L.ra = f + 2 * QR;
+  L.rb = f + 3 * QR;
+  L.dn = f + 4 * QR;
+  L.part = f + 5 * QR;
+  L.wsum = f + 13 * QR;
   return L;
 }
 
-// Rows r0 .. r0+31 of head h: u into LDS (zero past dim and past the last row),
-// ||x|| and ||x||_eps per row.
+// One 16-byte piece of a row of E.
 template <typename E>
-__device__ void q_rows(const gpa_quad_problem& p, int h, int r0, QLayout<E>& L) {
-  const int tid = threadIdx.x, row = tid / 8, part = tid % 8, D = p.dim;
-  const int grow = qmin(r0 + row, p.rows - 1);
-  const E* xr = reinterpret_cast<const E*>(p.x) + (int64_t)grow * p.row_stride + (int64_t)h * D;
-  float xv[32];
+struct QPiece {
+  static constexpr int N = 16 / sizeof(E);
+  E v[N];
+};
+// Elements d .. of a row (zeros past dim), in one 16-byte load when VEC.
+template <typename E, bool VEC>
+__device__ __forceinline__ QPiece<E> q_load(const E* row, int d, int dim) {
+  QPiece<E> x;
+  if constexpr (VEC) {
+    const uint4 w = *reinterpret_cast<const uint4*>(row + (d < dim ? d : 0));
+    __builtin_memcpy(&x, &w, 16);
+  } else {
 #pragma unroll
-  for (int i = 0; i < 32; ++i) xv[i] = to_f32(xr[qmin(part + 8 * i, D - 1)]);
+    for (int e = 0; e < QPiece<E>::N; ++e) x.v[e] = row[qmin(d + e, dim - 1)];
+  }
+  return x;
+}
+template <typename E>
+__device__ __forceinline__ void q_put(E* dst, const QPiece<E>& x) {
+  uint4 w;
+  __builtin_memcpy(&w, &x, 16);
+  *reinterpret_cast<uint4*>(dst) = w;
+}
+template <typename E, bool VEC>
+__device__ __forceinline__ void q_store(E* row, int d, int dim, const E* src) {
+  if constexpr (VEC) {
+    if (d < dim) *reinterpret_cast<uint4*>(row + d) = *reinterpret_cast<const uint4*>(src);
+  } else {
+#pragma unroll
+    for (int e = 0; e < QPiece<E>::N; ++e)
+      if (d + e < dim) row[d + e] = src[e];
+  }
+}
+
+// Rows r0 .. r0+31 of head h: u into LDS (zero past dim and past the last row)
+// and, with ROWS, the raw rows and dout's, u also to `uo`; ||x|| and ||x||_eps per
+// row.  Thread t holds the 16-byte pieces t%8, t%8 + 8, ... of row t/8; every load is
+// issued before the first use.
+template <typename E, bool VEC, bool ROWS>
+__device__ void q_rows(const gpa_quad_problem& p, const E* dout, E* uo, int h, int r0, QLayout<E>& L) {
+  constexpr int N = QPiece<E>::N, PM = 256 / (8 * N);
+  const int tid = threadIdx.x, row = tid / 8, part = tid % 8, D = p.dim;
   const bool live = r0 + row < p.rows;
+  const int grow = live ? r0 + row : p.rows - 1;
+  const E* xr = reinterpret_cast<const E*>(p.x) + (int64_t)grow * p.row_stride + (int64_t)h * D;
+  QPiece<E> xv[PM], gv[ROWS ? PM : 1];
+#pragma unroll
+  for (int i = 0; i < PM; ++i) xv[i] = q_load<E, VEC>(xr, (part + 8 * i) * N, D);
+  if constexpr (ROWS)
+#pragma unroll
+    for (int i = 0; i < PM; ++i)
+      gv[i] = q_load<E, VEC>(dout + ((int64_t)grow * p.heads + h) * D, (part + 8 * i) * N, D);
   float ss = 0.f;
 #pragma unroll
-  for (int i = 0; i < 32; ++i) {
-    xv[i] = (live && part + 8 * i < D) ? xv[i] : 0.f;
-    ss += xv[i] * xv[i];
-  }
+  for (int i = 0; i < PM; ++i)
+#pragma unroll
+    for (int e = 0; e < N; ++e) {
+      const bool ok = live && (part + 8 * i) * N + e < D;
+      if (!ok) xv[i].v[e] = from_f32<E>(0.f);
+      if constexpr (ROWS)
+        if (!ok) gv[i].v[e] = from_f32<E>(0.f);
+      const float x = to_f32(xv[i].v[e]);
+      ss += x * x;
+    }
   ss += __shfl_xor(ss, 1, 64);
   ss += __shfl_xor(ss, 2, 64);
   ss += __shfl_xor(ss, 4, 64);
   const float n = sqrtf(ss), den = fmaxf(n, 1e-6f);
 #pragma unroll
-  for (int i = 0; i < 32; ++i) {
-    const int d = part + 8 * i;
-    if (d < L.DP) L.u[row * L.ULD + d] = from_f32<E>(xv[i] / den);
+  for (int i = 0; i < PM; ++i) {
+    const int d = (part + 8 * i) * N;
+    if (d >= L.DP) continue;
+    if constexpr (ROWS) {
+      q_put(L.x + row * L.ULD + d, xv[i]);
+      q_put(L.g + row * L.ULD + d, gv[i]);
+    }
+#pragma unroll
+    for (int e = 0; e < N; ++e) xv[i].v[e] = from_f32<E>(to_f32(xv[i].v[e]) / den);
+    q_put(L.u + row * L.ULD + d, xv[i]);
+    if constexpr (ROWS)
+      if (live) q_store<E, VEC>(uo + ((int64_t)h * p.rows + r0 + row) * L.DP, d, L.DP, xv[i].v);
   }
   if (part == 0) {
     L.nrm[row] = sqrtf(ss + 1e-12f);
     L.xn[row] = n;
+  }
+}
+
+// Rows in LDS (from `src`, `ld` apart) to `width` elements of the live rows of
+// dst, `stride` apart.
+template <typename E, bool VEC>
+__device__ __forceinline__ void q_rows_out(const gpa_quad_problem& p, int r0, E* dst, int64_t stride, int width,
+                                           const E* src, int ld) {
+  constexpr int N = QPiece<E>::N;
+  const int row = threadIdx.x / 8;
+  if (r0 + row < p.rows)
+    for (int d = (threadIdx.x % 8) * N; d < width; d += 8 * N)
+      q_store<E, VEC>(dst + row * stride, d, width, src + row * ld + d);
+}
+
+// A per-row array at a lane's accumulator rows.
+__device__ __forceinline__ void q_at_rows(const float* a, float (&x)[16]) {
+  const int hi = (threadIdx.x & 63) >> 5;
+#pragma unroll
+  for (int g = 0; g < 4; ++g) {
+    const f32x4 v = *reinterpret_cast<const f32x4*>(a + 8 * g + 4 * hi);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) x[4 * g + i] = v[i];
   }
 }
 
@@ -135,166 +229,151 @@ __device__ __forceinline__ void q_products(const gpa_quad_problem& p, int h, int
 }
 
 // Row sums of a lane's 16 accumulator-layout values over the block's 32
-// columns, into part[slot][cb][row].
-__device__ __forceinline__ void q_row_part(float (&v)[16], float* part, int slot, int cb) {
+// columns, into part[cb][row].
+__device__ __forceinline__ void q_row_part(float (&v)[16], float* part, int cb) {
   const int l = threadIdx.x & 63;
   const float s = tile_row_sum(v, l);
-  if ((l & 1) == 0) part[(slot * 8 + cb) * QR + acc_row(sum_index(l), l >> 5)] = s;
+  if ((l & 1) == 0) part[cb * QR + acc_row(sum_index(l), l >> 5)] = s;
+}
+__device__ __forceinline__ float q_row_total(const float* part, int nb, int r) {
+  float s = 0.f;
+  for (int cb = 0; cb < nb; ++cb) s += part[cb * QR + r];
+  return s;
 }
 
-// row[slot][r] = sum over the column blocks of part[slot][.][r] (threads 0..31).
-__device__ __forceinline__ void q_row_total(float* part, float* row, int slot, int nb) {
-  const int t = threadIdx.x;
-  if (t < QR) {
-    float s = 0.f;
-    for (int cb = 0; cb < nb; ++cb) s += part[(slot * 8 + cb) * QR + t];
-    row[slot * QR + t] = s;
-  }
-}
-
+// z (and a, b) at a wave's elements of column block cb; its squares' row sums.
 template <typename E>
+__device__ __forceinline__ void q_z(const gpa_quad_problem& p, int h, int cb, const QLayout<E>& L, float c,
+                                    float (&z)[16], float (&av)[16], float (&bv)[16]) {
+  const int l = threadIdx.x & 63;
+  f32x16 acc_a, acc_b;
+  q_products<E>(p, h, cb, L, acc_a, acc_b);
+  float zz[16];
+#pragma unroll
+  for (int r = 0; r < 16; ++r) {
+    av[r] = round_as<E>(acc_a[r]);
+    bv[r] = round_as<E>(acc_b[r]);
+    z[r] = to_f32(L.u[acc_row(r, l >> 5) * L.ULD + cb * 32 + (l & 31)]) + (c * av[r]) * bv[r];
+    zz[r] = z[r] * z[r];
+  }
+  q_row_part(zz, L.part, cb);
+}
+
+// Rows move between HBM and LDS in 16-byte pieces, a row per 8 lanes, and the
+// per-row factors of an elementwise phase (roots, reciprocals) are formed once per
+// row by 32 threads.  Bound: HBM (the backward moves 6 rows of dim per row); element-
+// wise 2-byte accesses and a root and up to four divisions per element before.
+// bf16, 8192 rows x 16 heads x 128: forward 67 -> 50 us, backward 210 -> 95 us.
+// VEC: dim a whole number of 16-byte pieces, every row on a 16-byte boundary.
+template <typename E, bool VEC, int QB>
 __global__ __launch_bounds__(QT) void quad_fwd(gpa_quad_problem p) {
-  HIP_DYNAMIC_SHARED(char, smem)
+  extern __shared__ __align__(16) char smem[];
   const int h = blockIdx.y, r0 = blockIdx.x * QR, w = threadIdx.x >> 6, l = threadIdx.x & 63;
   QLayout<E> L = q_layout<E>(smem, p.dim, false);
-  q_rows<E>(p, h, r0, L);
-  __syncthreads();
+  q_rows<E, VEC, false>(p, nullptr, nullptr, h, r0, L);
+  lds_barrier();
   const float c = p.gain[h];
-  float z[QMAXB][16];
+  float z[QB][16];
 #pragma unroll
-  for (int bi = 0; bi < QMAXB; ++bi) {
-    const int cb = w + 4 * bi;
-    if (cb >= L.NB) break;
-    f32x16 acc_a, acc_b;
-    q_products<E>(p, h, cb, L, acc_a, acc_b);
-    float zz[16];
-#pragma unroll
-    for (int r = 0; r < 16; ++r) {
-      const int row = acc_row(r, l >> 5), col = cb * 32 + (l & 31);
-      const float a = round_as<E>(acc_a[r]), b = round_as<E>(acc_b[r]);
-      z[bi][r] = to_f32(L.u[row * L.ULD + col]) + (c * a) * b;
-      zz[r] = z[bi][r] * z[bi][r];
-    }
-    q_row_part(zz, L.part, 0, cb);
+  for (int bi = 0; bi < QB; ++bi) {
+    if (w + 4 * bi >= L.NB) break;
+    float a[16], b[16];
+    q_z<E>(p, h, w + 4 * bi, L, c, z[bi], a, b);
   }
-  __syncthreads();
-  q_row_total(L.part, L.row, 0, L.NB);
-  __syncthreads();
-  E* out = reinterpret_cast<E*>(p.out);
+  lds_barrier();
+  if (threadIdx.x < QR)
+    L.ra[threadIdx.x] = L.nrm[threadIdx.x] / fmaxf(sqrtf(q_row_total(L.part, L.NB, threadIdx.x)), 1e-6f);
+  lds_barrier();
+  float f[16];
+  q_at_rows(L.ra, f);
 #pragma unroll
-  for (int bi = 0; bi < QMAXB; ++bi) {
+  for (int bi = 0; bi < QB; ++bi) {
     const int cb = w + 4 * bi;
     if (cb >= L.NB) break;
 #pragma unroll
-    for (int r = 0; r < 16; ++r) {
-      const int row = acc_row(r, l >> 5), col = cb * 32 + (l & 31);
-      const float zn = fmaxf(sqrtf(L.row[row]), 1e-6f);
-      if (r0 + row < p.rows && col < p.dim)
-        out[((int64_t)(r0 + row) * p.heads + h) * p.dim + col] = from_f32<E>(z[bi][r] / zn * L.nrm[row]);
-    }
+    for (int r = 0; r < 16; ++r) L.u[acc_row(r, l >> 5) * L.ULD + cb * 32 + (l & 31)] = from_f32<E>(z[bi][r] * f[r]);
   }
+  lds_barrier();
+  q_rows_out<E, VEC>(p, r0, reinterpret_cast<E*>(p.out) + ((int64_t)r0 * p.heads + h) * p.dim, (int64_t)p.heads * p.dim,
+                     p.dim, L.u, L.ULD);
 }
 
-template <typename E>
+template <typename E, bool VEC, int QB>
 __global__ __launch_bounds__(QT) void quad_bwd(gpa_quad_problem p, gpa_quad_grads g) {
-  HIP_DYNAMIC_SHARED(char, smem)
-  const int h = blockIdx.y, r0 = blockIdx.x * QR, w = threadIdx.x >> 6, l = threadIdx.x & 63;
+  extern __shared__ __align__(16) char smem[];
+  const int h = blockIdx.y, r0 = blockIdx.x * QR, w = threadIdx.x >> 6, l = threadIdx.x & 63, t = threadIdx.x;
   const int D = p.dim;
   QLayout<E> L = q_layout<E>(smem, D, true);
-  q_rows<E>(p, h, r0, L);
-  __syncthreads();
+  q_rows<E, VEC, true>(p, reinterpret_cast<const E*>(g.dout), reinterpret_cast<E*>(g.u), h, r0, L);
+  lds_barrier();
   const float c = p.gain[h];
-  float z[QMAXB][16], av[QMAXB][16], bv[QMAXB][16];
+  float z[QB][16], av[QB][16], bv[QB][16], gv[QB][16];
+  auto at = [&](int r, int cb) { return acc_row(r, l >> 5) * L.ULD + cb * 32 + (l & 31); };
 #pragma unroll
-  for (int bi = 0; bi < QMAXB; ++bi) {
+  for (int bi = 0; bi < QB; ++bi) {
     const int cb = w + 4 * bi;
     if (cb >= L.NB) break;
-    f32x16 acc_a, acc_b;
-    q_products<E>(p, h, cb, L, acc_a, acc_b);
-    float zz[16];
+    q_z<E>(p, h, cb, L, c, z[bi], av[bi], bv[bi]);
 #pragma unroll
-    for (int r = 0; r < 16; ++r) {
-      const int row = acc_row(r, l >> 5), col = cb * 32 + (l & 31);
-      av[bi][r] = round_as<E>(acc_a[r]);
-      bv[bi][r] = round_as<E>(acc_b[r]);
-      z[bi][r] = to_f32(L.u[row * L.ULD + col]) + (c * av[bi][r]) * bv[bi][r];
-      zz[r] = z[bi][r] * z[bi][r];
-    }
-    q_row_part(zz, L.part, 0, cb);
+    for (int r = 0; r < 16; ++r) gv[bi][r] = to_f32(L.g[at(r, cb)]);
   }
-  __syncthreads();
-  q_row_total(L.part, L.row, 0, L.NB);
-  __syncthreads();
+  lds_barrier();
+  float zt = 0.f;
+  if (t < QR) zt = sqrtf(q_row_total(L.part, L.NB, t));
+  lds_barrier();
   // out = unit(z) nrm: d nrm = sum g unit(z), d unit(z) = g nrm; the
-  // normalisation backward needs sum d unit(z) . z per row.
-  const E* dout = reinterpret_cast<const E*>(g.dout);
-  float gv[QMAXB][16];
+  // normalisation backward needs sum d unit(z) . z = nrm sum g z per row.
 #pragma unroll
-  for (int bi = 0; bi < QMAXB; ++bi) {
+  for (int bi = 0; bi < QB; ++bi) {
     const int cb = w + 4 * bi;
     if (cb >= L.NB) break;
+    float gz[16];
 #pragma unroll
-    for (int r = 0; r < 16; ++r) {
-      const int row = acc_row(r, l >> 5), col = cb * 32 + (l & 31);
-      gv[bi][r] = to_f32(dout[((int64_t)qmin(r0 + row, p.rows - 1) * p.heads + h) * D + qmin(col, D - 1)]);
-    }
-    float s1[16], s2[16];
-#pragma unroll
-    for (int r = 0; r < 16; ++r) {
-      const int row = acc_row(r, l >> 5), col = cb * 32 + (l & 31);
-      if (!(r0 + row < p.rows && col < D)) gv[bi][r] = 0.f;
-      const float zn = fmaxf(sqrtf(L.row[row]), 1e-6f);
-      s1[r] = gv[bi][r] * (z[bi][r] / zn);
-      s2[r] = gv[bi][r] * L.nrm[row] * z[bi][r];
-    }
-    q_row_part(s1, L.part, 1, cb);
-    q_row_part(s2, L.part, 2, cb);
+    for (int r = 0; r < 16; ++r) gz[r] = gv[bi][r] * z[bi][r];
+    q_row_part(gz, L.part, cb);
   }
-  __syncthreads();
-  q_row_total(L.part, L.row, 1, L.NB);
-  q_row_total(L.part, L.row, 2, L.NB);
-  __syncthreads();
+  lds_barrier();
+  if (t < QR) {  // dz = g ra - z rb
+    const float gz = q_row_total(L.part, L.NB, t), n = L.nrm[t];
+    const float i = zt > 1e-6f ? 1.f / zt : 1e6f;
+    L.ra[t] = n * i;
+    L.rb[t] = zt > 1e-6f ? n * gz * i * i * i : 0.f;
+    L.dn[t] = gz / fmaxf(zt, 1e-6f) / n;
+  }
+  lds_barrier();
   // dz, then da = (dz b) c, db = dz (c a) in E; du starts as dz rounded to E.
-  float du0[QMAXB][16];
   float dc = 0.f;
-  E* uo = reinterpret_cast<E*>(g.u);
-  E* dabo = reinterpret_cast<E*>(g.dab);
+  {
+    float ra[16], rb[16];
+    q_at_rows(L.ra, ra);
+    q_at_rows(L.rb, rb);
 #pragma unroll
-  for (int bi = 0; bi < QMAXB; ++bi) {
-    const int cb = w + 4 * bi;
-    if (cb >= L.NB) break;
+    for (int bi = 0; bi < QB; ++bi) {
+      const int cb = w + 4 * bi;
+      if (cb >= L.NB) break;
 #pragma unroll
-    for (int r = 0; r < 16; ++r) {
-      const int row = acc_row(r, l >> 5), col = cb * 32 + (l & 31);
-      const float zt = sqrtf(L.row[row]);
-      const float du = gv[bi][r] * L.nrm[row];
-      float dz;
-      if (zt > 1e-6f) dz = du / zt - z[bi][r] * (L.row[2 * QR + row] / (zt * zt * zt));
-      else dz = du / 1e-6f;
-      const float t1 = dz * bv[bi][r];
-      dc += t1 * av[bi][r];
-      const E da = from_f32<E>(t1 * c), db = from_f32<E>(dz * (c * av[bi][r]));
-      L.dab[row * L.DLD + col] = da;
-      L.dab[row * L.DLD + L.DP + col] = db;
-      du0[bi][r] = round_as<E>(dz);
-      if (r0 + row < p.rows) {
-        const int64_t hr = (int64_t)h * p.rows + r0 + row;
-        dabo[hr * 2 * L.DP + col] = da;
-        dabo[hr * 2 * L.DP + L.DP + col] = db;
-        uo[hr * L.DP + col] = L.u[row * L.ULD + col];
+      for (int r = 0; r < 16; ++r) {
+        const float dz = gv[bi][r] * ra[r] - z[bi][r] * rb[r];
+        const float t1 = dz * bv[bi][r];
+        dc += t1 * av[bi][r];
+        E* d = L.dab + acc_row(r, l >> 5) * L.DLD + cb * 32 + (l & 31);
+        d[0] = from_f32<E>(t1 * c);
+        d[L.DP] = from_f32<E>(dz * (c * av[bi][r]));
+        z[bi][r] = round_as<E>(dz);
       }
     }
   }
   dc = sum64(dc);
   if (l == 0) L.wsum[w] = dc;
-  __syncthreads();
-  if (threadIdx.x == 0) g.dgain[(int64_t)blockIdx.x * p.heads + h] = L.wsum[0] + L.wsum[1] + L.wsum[2] + L.wsum[3];
+  lds_barrier();
+  if (t == 0) g.dgain[(int64_t)blockIdx.x * p.heads + h] = L.wsum[0] + L.wsum[1] + L.wsum[2] + L.wsum[3];
+  q_rows_out<E, VEC>(p, r0, reinterpret_cast<E*>(g.dab) + ((int64_t)h * p.rows + r0) * 2 * L.DP, 2 * L.DP, 2 * L.DP, L.dab,
+                     L.DLD);
   // du = dz + da L^T + db R^T: contraction over the 2 DP columns of [da | db];
   // the B operand of output column k is row k of w = [L | R] (contiguous).
   const E* wk = reinterpret_cast<const E*>(p.w);
-  float dun[QMAXB][16];
 #pragma unroll
-  for (int bi = 0; bi < QMAXB; ++bi) {
+  for (int bi = 0; bi < QB; ++bi) {
     const int cb = w + 4 * bi;
     if (cb >= L.NB) break;
     f32x16 acc_l, acc_r;
@@ -319,43 +398,35 @@ __global__ __launch_bounds__(QT) void quad_bwd(gpa_quad_problem p, gpa_quad_grad
         mma8(acc_r, ld_c(d, L.DLD, lr, L.DP + c0), *reinterpret_cast<const f32x4*>(wf + L.DP + c0));
       }
     }
-    // x of the same elements, for unit(x)'s backward
-    const E* x = reinterpret_cast<const E*>(p.x);
-    float xv[16], s3[16];
+    float s3[16];
 #pragma unroll
     for (int r = 0; r < 16; ++r) {
-      const int row = acc_row(r, l >> 5), col = cb * 32 + lr;
-      xv[r] = to_f32(x[(int64_t)qmin(r0 + row, p.rows - 1) * p.row_stride + (int64_t)h * D + qmin(col, D - 1)]);
+      av[bi][r] = to_f32(L.x[at(r, cb)]);
+      z[bi][r] = round_as<E>(z[bi][r] + round_as<E>(acc_l[r]) + round_as<E>(acc_r[r]));
+      s3[r] = z[bi][r] * av[bi][r];
     }
-#pragma unroll
-    for (int r = 0; r < 16; ++r) {
-      const int row = acc_row(r, l >> 5), col = cb * 32 + lr;
-      if (!(r0 + row < p.rows && col < D)) xv[r] = 0.f;
-      dun[bi][r] = round_as<E>(du0[bi][r] + round_as<E>(acc_l[r]) + round_as<E>(acc_r[r]));
-      s3[r] = dun[bi][r] * xv[r];
-      av[bi][r] = xv[r];  // keep x for dx
-    }
-    q_row_part(s3, L.part, 0, cb);
+    q_row_part(s3, L.part, cb);
   }
-  __syncthreads();
-  q_row_total(L.part, L.row, 0, L.NB);
-  __syncthreads();
-  E* dx = reinterpret_cast<E*>(g.dx);
+  lds_barrier();
+  if (t < QR) {  // dx = du ra - x rb, through unit(x) and ||x||_eps
+    const float n = L.xn[t], i = n > 1e-6f ? 1.f / n : 1e6f;
+    L.ra[t] = i;
+    L.rb[t] = (n > 1e-6f ? q_row_total(L.part, L.NB, t) * i * i * i : 0.f) - L.dn[t];
+  }
+  lds_barrier();
+  float ra[16], rb[16];
+  q_at_rows(L.ra, ra);
+  q_at_rows(L.rb, rb);
 #pragma unroll
-  for (int bi = 0; bi < QMAXB; ++bi) {
+  for (int bi = 0; bi < QB; ++bi) {
     const int cb = w + 4 * bi;
     if (cb >= L.NB) break;
 #pragma unroll
-    for (int r = 0; r < 16; ++r) {
-      const int row = acc_row(r, l >> 5), col = cb * 32 + (l & 31);
-      const float n = L.xn[row], x = av[bi][r];
-      float d;
-      if (n > 1e-6f) d = dun[bi][r] / n - x * (L.row[row] / (n * n * n));
-      else d = dun[bi][r] / 1e-6f;
-      d += L.row[QR + row] * x / L.nrm[row];  // through ||x||_eps
-      if (r0 + row < p.rows && col < D) dx[((int64_t)(r0 + row) * p.heads + h) * D + col] = from_f32<E>(d);
-    }
+    for (int r = 0; r < 16; ++r) L.u[at(r, cb)] = from_f32<E>(z[bi][r] * ra[r] - av[bi][r] * rb[r]);
   }
+  lds_barrier();
+  q_rows_out<E, VEC>(p, r0, reinterpret_cast<E*>(g.dx) + ((int64_t)r0 * p.heads + h) * D, (int64_t)p.heads * D, D, L.u,
+                     L.ULD);
 }
 
 int check_quad(const gpa_quad_problem* pp) {
@@ -371,13 +442,39 @@ int check_quad(const gpa_quad_problem* pp) {
   return 0;
 }
 
-template <typename K>
-int q_lds_attr(K kernel, size_t bytes) {
-  if (bytes <= 65536) return 0;
-  if (hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize,
-                          (int)bytes) != hipSuccess)
+template <typename K, typename... A>
+int q_launch(K kernel, const gpa_quad_problem& p, size_t lds, hipStream_t stream, A... args) {
+  if (lds > 65536 && hipFuncSetAttribute(reinterpret_cast<const void*>(kernel),
+                                         hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds) != hipSuccess)
     return fail(GPA_HIP_EHIP, "hipFuncSetAttribute(max dynamic LDS) failed");
+  const dim3 grid((unsigned)((p.rows + QR - 1) / QR), (unsigned)p.heads);
+  hipLaunchKernelGGL(kernel, grid, dim3(QT), lds, stream, p, args...);
   return 0;
+}
+
+// Every row of these buffers starts on a 16-byte boundary and is a whole
+// number of 16-byte pieces.
+template <typename E>
+bool q_vec(const gpa_quad_problem& p, std::initializer_list<const void*> buffers) {
+  const int n = 16 / (int)sizeof(E);
+  bool ok = p.dim % n == 0 && p.row_stride % n == 0;
+  for (const void* b : buffers) ok = ok && reinterpret_cast<uintptr_t>(b) % 16 == 0;
+  return ok;
+}
+
+template <typename E>
+int q_forward(const gpa_quad_problem& p, hipStream_t stream) {
+  const size_t lds = q_lds_bytes<E>(p.dim, false);
+  const bool vec = q_vec<E>(p, {p.x, p.out});
+  if (p.dim <= 128) return q_launch(vec ? quad_fwd<E, true, 1> : quad_fwd<E, false, 1>, p, lds, stream);
+  return q_launch(vec ? quad_fwd<E, true, 2> : quad_fwd<E, false, 2>, p, lds, stream);
+}
+template <typename E>
+int q_backward(const gpa_quad_problem& p, const gpa_quad_grads& g, hipStream_t stream) {
+  const size_t lds = q_lds_bytes<E>(p.dim, true);
+  const bool vec = q_vec<E>(p, {p.x, g.dout, g.dx, g.u, g.dab});
+  if (p.dim <= 128) return q_launch(vec ? quad_bwd<E, true, 1> : quad_bwd<E, false, 1>, p, lds, stream, g);
+  return q_launch(vec ? quad_bwd<E, true, 2> : quad_bwd<E, false, 2>, p, lds, stream, g);
 }
 
 }  // namespace
@@ -386,18 +483,9 @@ int q_lds_attr(K kernel, size_t bytes) {
 extern "C" int gpa_quad_features_forward(const gpa_quad_problem* problem, hipStream_t stream) {
   using namespace gpa;
   if (int rc = check_quad(problem)) return rc;
-  const gpa_quad_problem& p = *problem;
-  if (!p.out) return fail(GPA_HIP_EINVAL, "quad features: out required");
-  const dim3 grid((unsigned)((p.rows + QR - 1) / QR), (unsigned)p.heads);
-  if (p.dtype == GPA_DTYPE_BF16) {
-    const size_t lds = q_lds_bytes<bf16_t>(p.dim, false);
-    if (int rc = q_lds_attr(quad_fwd<bf16_t>, lds)) return rc;
-    hipLaunchKernelGGL((quad_fwd<bf16_t>), grid, dim3(QT), lds, stream, p);
-  } else {
-    const size_t lds = q_lds_bytes<float>(p.dim, false);
-    if (int rc = q_lds_attr(quad_fwd<float>, lds)) return rc;
-    hipLaunchKernelGGL((quad_fwd<float>), grid, dim3(QT), lds, stream, p);
-  }
+  if (!problem->out) return fail(GPA_HIP_EINVAL, "quad features: out required");
+  if (int rc = problem->dtype == GPA_DTYPE_BF16 ? q_forward<bf16_t>(*problem, stream) : q_forward<float>(*problem, stream))
+    return rc;
   return check_launch("gpa_quad_features_forward");
 }
 
@@ -407,16 +495,8 @@ extern "C" int gpa_quad_features_backward(const gpa_quad_problem* problem, const
   if (int rc = check_quad(problem)) return rc;
   if (!grads || !grads->dout || !grads->dx || !grads->u || !grads->dab || !grads->dgain)
     return fail(GPA_HIP_EINVAL, "quad features backward: dout, dx, u, dab and dgain required");
-  const gpa_quad_problem& p = *problem;
-  const dim3 grid((unsigned)((p.rows + QR - 1) / QR), (unsigned)p.heads);
-  if (p.dtype == GPA_DTYPE_BF16) {
-    const size_t lds = q_lds_bytes<bf16_t>(p.dim, true);
-    if (int rc = q_lds_attr(quad_bwd<bf16_t>, lds)) return rc;
-    hipLaunchKernelGGL((quad_bwd<bf16_t>), grid, dim3(QT), lds, stream, p, *grads);
-  } else {
-    const size_t lds = q_lds_bytes<float>(p.dim, true);
-    if (int rc = q_lds_attr(quad_bwd<float>, lds)) return rc;
-    hipLaunchKernelGGL((quad_bwd<float>), grid, dim3(QT), lds, stream, p, *grads);
-  }
+  if (int rc = problem->dtype == GPA_DTYPE_BF16 ? q_backward<bf16_t>(*problem, *grads, stream)
+                                                : q_backward<float>(*problem, *grads, stream))
+    return rc;
   return check_launch("gpa_quad_features_backward");
 }
