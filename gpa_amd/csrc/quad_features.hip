@@ -429,6 +429,30 @@ __global__ __launch_bounds__(QT) void quad_bwd(gpa_quad_problem p, gpa_quad_grad
                      L.ULD);
 }
 
+// The two weight layouts from the float32 parameters [H][D][D], a 32 x 32 tile per
+// workgroup: wt transposed through LDS, w (may be null) as read; zeros past D.
+// One launch in place of a stack, a cast, a pad and two strided copies (19 us each
+// at 16 heads x 128).
+template <typename E>
+__global__ __launch_bounds__(QT) void quad_pack(const float* left, const float* right, E* wt, E* w, int D) {
+  __shared__ float tile[32][33];
+  const int DP = qpad(D), NB = DP / 32, h = blockIdx.y >> 1, p = blockIdx.y & 1;
+  const int k0 = (int)(blockIdx.x / NB) * 32, n0 = (int)(blockIdx.x % NB) * 32, c = threadIdx.x % 32, r0 = threadIdx.x / 32;
+  const float* src = (p ? right : left) + (int64_t)h * D * D;
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const int k = k0 + r0 + 8 * i, n = n0 + c;
+    const bool ok = k < D && n < D;
+    const float x = src[ok ? (int64_t)k * D + n : 0];
+    tile[r0 + 8 * i][c] = ok ? x : 0.f;
+    if (w) w[((int64_t)h * DP + k) * 2 * DP + p * DP + n] = from_f32<E>(ok ? x : 0.f);
+  }
+  __syncthreads();
+#pragma unroll
+  for (int i = 0; i < 4; ++i)
+    wt[(((int64_t)h * 2 + p) * DP + n0 + r0 + 8 * i) * DP + k0 + c] = from_f32<E>(tile[c][r0 + 8 * i]);
+}
+
 int check_quad(const gpa_quad_problem* pp) {
   if (!pp) return fail(GPA_HIP_EINVAL, "quad features: null problem");
   const gpa_quad_problem& p = *pp;
@@ -499,4 +523,37 @@ extern "C" int gpa_quad_features_backward(const gpa_quad_problem* problem, const
                                                 : q_backward<float>(*problem, *grads, stream))
     return rc;
   return check_launch("gpa_quad_features_backward");
+}
+
+extern "C" int gpa_quad_pack_weights(const float* left, const float* right, int32_t heads, int32_t dim, int32_t dtype,
+                                     void* wt, void* w, hipStream_t stream) {
+  using namespace gpa;
+  if (!left || !right || !wt || heads < 1 || heads > 32767 || dim < 1 || dim > GPA_QUAD_MAX_DIM)
+    return fail(GPA_HIP_EINVAL, "quad pack: left, right, wt required; heads 1..32767, dim 1..GPA_QUAD_MAX_DIM");
+  if (dtype != GPA_DTYPE_F32 && dtype != GPA_DTYPE_BF16) return fail(GPA_HIP_EUNSUPPORTED, "quad pack: dtype");
+  const int nb = qpad(dim) / 32;
+  const dim3 grid(nb * nb, 2 * heads);
+  if (dtype == GPA_DTYPE_BF16)
+    hipLaunchKernelGGL((quad_pack<bf16_t>), grid, dim3(QT), 0, stream, left, right, static_cast<bf16_t*>(wt),
+                       static_cast<bf16_t*>(w), dim);
+  else
+    hipLaunchKernelGGL((quad_pack<float>), grid, dim3(QT), 0, stream, left, right, static_cast<float*>(wt),
+                       static_cast<float*>(w), dim);
+  return check_launch("gpa_quad_pack_weights");
+}
+
+extern "C" int gpa_quad_weight_grads(const gpa_quad_problem* problem, const void* u, const void* dab, float* dleft,
+                                     float* dright, hipStream_t stream) {
+  using namespace gpa;
+  if (int rc = check_quad(problem)) return rc;
+  const gpa_quad_problem& p = *problem;
+  if (p.dtype != GPA_DTYPE_BF16) return fail(GPA_HIP_EUNSUPPORTED, "quad weight grads: bf16 only");
+  if (!u || !dab || !dleft || !dright) return fail(GPA_HIP_EINVAL, "quad weight grads: u, dab, dleft and dright required");
+  const int dp = qpad(p.dim);
+  const int64_t hs = (int64_t)p.rows * dp;
+  const bf16_t* b = static_cast<const bf16_t*>(dab);
+  const TnProduct products[2] = {{u, dp, hs, dp, b, 2 * dp, 2 * hs, dp, dleft},
+                                 {u, dp, hs, dp, b + dp, 2 * dp, 2 * hs, dp, dright}};
+  if (int rc = launch_tn_products(products, 2, p.heads, p.rows, true, stream)) return rc;
+  return check_launch("gpa_quad_weight_grads");
 }

@@ -170,6 +170,16 @@ int main(int argc, char** argv) {
       rc = 0;
       break;
     }
+    case 24: {
+      const int32_t* a = reinterpret_cast<const int32_t*>(blobs.at(0).data());
+      rc = gpa_quad_pack_weights(static_cast<float*>(raw.at(0)), static_cast<float*>(raw.at(1)), a[0], a[1], a[2],
+                                 raw.at(2), raw.at(3), nullptr);
+      break;
+    }
+    case 25:
+      rc = gpa_quad_weight_grads(reinterpret_cast<gpa_quad_problem*>(blobs.at(0).data()), raw.at(0), raw.at(1),
+                                 static_cast<float*>(raw.at(2)), static_cast<float*>(raw.at(3)), nullptr);
+      break;
     case 23:
       value = gpa_gdn_path(reinterpret_cast<gpa_gdn_problem*>(blobs.at(0).data()));
       rc = 0;
