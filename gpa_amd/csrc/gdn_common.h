@@ -143,6 +143,26 @@ __device__ __forceinline__ void kernarg_copy(T& dst, const __attribute__((addres
   for (int i = 0; i < (int)(sizeof(T) / 4); ++i) d[i] = s[i];
 }
 
+// A pointer copied out of the argument segment word by word, known to point to
+// global memory (uniform): its accesses are then global ones.  A flat access also
+// counts as an LDS operation, so every LDS wait would wait for it.  (The empty
+// statement keeps the compiler from folding the two casts away.)  The 256-key state
+// packs stay on flat accesses: as global ones they need more registers than there
+// are (16 streams x 32 chunks: 202 -> 214 us forward, 244 -> 251 us backward).
+template <typename T>
+__device__ __forceinline__ void to_global(T*& p) {
+  __attribute__((address_space(1))) T* g = (__attribute__((address_space(1))) T*)p;
+  asm volatile("" : "+s"(g));
+  p = (T*)g;
+}
+__device__ __forceinline__ void to_global(gpa_operand& o) { to_global(o.ptr); }
+template <typename... T>
+__device__ __forceinline__ void all_global(T&... p) {
+  (to_global(p), ...);
+}
+__device__ __forceinline__ void to_global(gpa_gdn_problem& p) {
+  all_global(p.q, p.k, p.v, p.g, p.beta, p.s0);
+}
 // MFMA launchers for the bf16 state recurrences (gdn_state_mfma.hip); they
 // return nonzero if the width is not built.
 template <int KM>

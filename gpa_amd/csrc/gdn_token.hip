@@ -46,6 +46,10 @@ __global__ __launch_bounds__(SNT) void gdn_token_step_pack(TokenPack pk) {
   gpa_operand out;
   kernarg_copy(p, &kp->p[pi]);
   kernarg_copy(out, &kp->out[pi]);
+  to_global(p);
+  to_global(out);
+  float* fin = kp->fin[pi];
+  to_global(fin);
   __shared__ union {
     TokenLds<4> c4;
     TokenLds<8> c8;
@@ -53,9 +57,9 @@ __global__ __launch_bounds__(SNT) void gdn_token_step_pack(TokenPack pk) {
   } lds;
   const int wg = (int)blockIdx.x - kp->wg0[pi], ni = kp->ni[pi];
   const gpa_token_slot none{};
-  if (ni == 4) token_run<E, 4>(p, kp->fin[pi], out, wg, threadIdx.x, lds.c4, none);
-  else if (ni == 8) token_run<E, 8>(p, kp->fin[pi], out, wg, threadIdx.x, lds.c8, none);
-  else token_run<E, 16>(p, kp->fin[pi], out, wg, threadIdx.x, lds.c16, none);
+  if (ni == 4) token_run<E, 4>(p, fin, out, wg, threadIdx.x, lds.c4, none);
+  else if (ni == 8) token_run<E, 8>(p, fin, out, wg, threadIdx.x, lds.c8, none);
+  else token_run<E, 16>(p, fin, out, wg, threadIdx.x, lds.c16, none);
 }
 
 template <typename E>

@@ -217,20 +217,20 @@ __device__ __forceinline__ uint4 pack_bf8(const float (&x)[8]) {
 }
 
 // r0 = softmax(base + gain tanh z) of a workgroup's RR rows, rounded to E,
-// with 32 lanes per row (8 columns each) and 8 rows per pass (VEC rows):
+// with 32 lanes per row (8 columns each), RR / VP rows per pass (VEC rows):
 // written to the saved rows sr0 and, when A is given, to the LDS tile
-// A [RR][lda] (zero beyond M, up to kM).
-template <typename E>
+// A [RR][lda] (zero beyond M, up to kM), in float or bf16.
+template <typename E, int VP = VPASS, typename AT = float>
 __device__ __forceinline__ void rows_r0_vec(const gpa_route_problem& p, const Rows& rows, int row0, int h,
-                                            E* sr0, float* A, int lda, int kM) {
+                                            E* sr0, AT* A, int lda, int kM) {
   const int M = p.slots, R = p.batch * p.tokens, tid = threadIdx.x;
   const int c = 8 * (tid & 31), rsub = tid >> 5;
   const bool on = c < M;
-  float bv[VPASS][8];
-  uint4 mv[VPASS][GPA_ROUTE_MAX_INCOMING];
+  float bv[VP][8];
+  uint4 mv[VP][GPA_ROUTE_MAX_INCOMING];
 #pragma unroll
-  for (int i = 0; i < VPASS; ++i) {
-    const int r = row0 + rsub + 8 * i, rr = r < R ? r : R - 1;
+  for (int i = 0; i < VP; ++i) {
+    const int r = row0 + rsub + RR / VP * i, rr = r < R ? r : R - 1;
     if (on) {
       const float* bp = reinterpret_cast<const float*>(p.base.ptr) + rows.at(p.base, rr, h) + c;
       const f32x4 x0 = *reinterpret_cast<const f32x4*>(bp), x1 = *reinterpret_cast<const f32x4*>(bp + 4);
@@ -249,8 +249,8 @@ __device__ __forceinline__ void rows_r0_vec(const gpa_route_problem& p, const Ro
 #pragma unroll
   for (int e = 0; e < GPA_ROUTE_MAX_INCOMING; ++e) ew[e] = e < p.incoming ? p.edge_weight[e * p.heads + h] : 0.f;
 #pragma unroll
-  for (int i = 0; i < VPASS; ++i) {
-    const int row = rsub + 8 * i, r = row0 + row;
+  for (int i = 0; i < VP; ++i) {
+    const int row = rsub + RR / VP * i, r = row0 + row;
     float v[8];
 #pragma unroll
     for (int e = 0; e < 8; ++e) v[e] = on ? bv[i][e] : 0.f;
@@ -294,8 +294,12 @@ __device__ __forceinline__ void rows_r0_vec(const gpa_route_problem& p, const Ro
 #pragma unroll
     for (int j = 0; j < 8; ++j) v[j] = (valid && on) ? round_as<E>(v[j] / sm) : 0.f;
     if (A && c < kM) {
-      *reinterpret_cast<f32x4*>(&A[row * lda + c]) = f32x4{v[0], v[1], v[2], v[3]};
-      *reinterpret_cast<f32x4*>(&A[row * lda + c + 4]) = f32x4{v[4], v[5], v[6], v[7]};
+      if constexpr (std::is_same<AT, float>::value) {
+        *reinterpret_cast<f32x4*>(&A[row * lda + c]) = f32x4{v[0], v[1], v[2], v[3]};
+        *reinterpret_cast<f32x4*>(&A[row * lda + c + 4]) = f32x4{v[4], v[5], v[6], v[7]};
+      } else {
+        *reinterpret_cast<uint4*>(&A[row * lda + c]) = pack_bf8(v);
+      }
     }
     if (valid && on) *reinterpret_cast<uint4*>(sr0 + (int64_t)r * M + c) = pack_bf8(v);
   }
@@ -436,10 +440,7 @@ __device__ __forceinline__ void rows_bwd_vec(const gpa_route_problem& p, const g
 }
 
 // The forward of RR rows (row0 ..) of head h of one problem.
-// NW waves: the row phases and the q staging run on the first RNT threads,
-// the product tiles are spread over all NW waves (the packed one-token read
-// uses 8, so that the 32 rows of a wide level walk half as many tiles per wave).
-template <typename E, bool VEC, int NW = RW>
+template <typename E, bool VEC>
 __device__ __forceinline__ void route_fwd_run(const gpa_route_problem& p, int h, int row0) {
   using W = typename Wt<E>::type;
   HIP_DYNAMIC_SHARED(float, lds)
@@ -456,9 +457,7 @@ __device__ __forceinline__ void route_fwd_run(const gpa_route_problem& p, int h,
   E* shd = reinterpret_cast<E*>(p.hd) + (int64_t)h * R * M;
 
   // ---- r0 = softmax(base + gain tanh z)
-  if (NW > RW && tid >= RNT) {
-    // the row phase runs on the first RNT threads
-  } else if constexpr (VEC) {
+  if constexpr (VEC) {
     rows_r0_vec<E>(p, rows, row0, h, sr0, A, lda, kM);
   } else {
     const int row = tid >> 3, part = tid & 7, r = row0 + row;
@@ -481,7 +480,7 @@ __device__ __forceinline__ void route_fwd_run(const gpa_route_problem& p, int h,
   // ---- h1 = r0 U, gelu(h1) -> Hs
   {
     const W* ut = reinterpret_cast<const W*>(p.up_t) + (int64_t)h * pad32(2 * M) * kM;
-    for (int t = wave; t < pad32(2 * M) / 32; t += NW) {
+    for (int t = wave; t < pad32(2 * M) / 32; t += RW) {
       f32x16 acc = {};
       tile_gemm(acc, A, lda, ut, kM, kM, 32 * t, lane);
 #pragma unroll
@@ -504,7 +503,7 @@ __device__ __forceinline__ void route_fwd_run(const gpa_route_problem& p, int h,
     const W* dt = reinterpret_cast<const W*>(p.down_t) + (int64_t)h * pad32(M) * k2M;
     const float g = p.mlp_gain[h];
     E* route = reinterpret_cast<E*>(p.route.ptr);
-    for (int t = wave; t < pad32(M) / 32; t += NW) {
+    for (int t = wave; t < pad32(M) / 32; t += RW) {
       f32x16 acc = {};
       tile_gemm(acc, Hs, ldh, dt, k2M, k2M, 32 * t, lane);
 #pragma unroll
@@ -526,31 +525,27 @@ __device__ __forceinline__ void route_fwd_run(const gpa_route_problem& p, int h,
 
   // ---- rsa_update: r1 <- round(r1 / clamp(sum |r1|, .25, 4)) in A and the route output
   if (p.rsa) {
-    if (!(NW > RW && tid >= RNT)) {
-      const int row = tid >> 3, part = tid & 7, r = row0 + row;
-      float s = 0.f;
+    const int row = tid >> 3, part = tid & 7, r = row0 + row;
+    float s = 0.f;
 #pragma unroll
-      for (int i = 0; i < RPER; ++i)
-        if (part + 8 * i < M) s += fabsf(A[row * lda + part + 8 * i]);
-      const float l = fminf(fmaxf(sum8(s), .25f), 4.f);
-      E* route = reinterpret_cast<E*>(p.route.ptr);
+    for (int i = 0; i < RPER; ++i)
+      if (part + 8 * i < M) s += fabsf(A[row * lda + part + 8 * i]);
+    const float l = fminf(fmaxf(sum8(s), .25f), 4.f);
+    E* route = reinterpret_cast<E*>(p.route.ptr);
 #pragma unroll
-      for (int i = 0; i < RPER; ++i) {
-        const int m = part + 8 * i;
-        if (m < M) {
-          const float x = round_as<E>(A[row * lda + m] / l);
-          A[row * lda + m] = x;
-          if (r < R) route[rows.at(p.route, r, h) + m] = from_f32<E>(x);
-        }
+    for (int i = 0; i < RPER; ++i) {
+      const int m = part + 8 * i;
+      if (m < M) {
+        const float x = round_as<E>(A[row * lda + m] / l);
+        A[row * lda + m] = x;
+        if (r < R) route[rows.at(p.route, r, h) + m] = from_f32<E>(x);
       }
     }
     __syncthreads();
   }
 
   // ---- q -> Hs
-  if (NW > RW && tid >= RNT) {
-    // the q staging runs on the first RNT threads
-  } else if constexpr (VEC) {
+  if constexpr (VEC) {
     const int c = 8 * (tid & 31), rsub = tid >> 5;
     uint4 qv[VPASS];
 #pragma unroll
@@ -587,7 +582,7 @@ __device__ __forceinline__ void route_fwd_run(const gpa_route_problem& p, int h,
     const W* rt = reinterpret_cast<const W*>(p.rs_t) + (int64_t)h * pad32(M) * kM;
     const W* qt = reinterpret_cast<const W*>(p.qs_t) + (int64_t)h * pad32(M) * kD;
     E* qo = reinterpret_cast<E*>(p.qo.ptr);
-    for (int t = wave; t < pad32(M) / 32; t += NW) {
+    for (int t = wave; t < pad32(M) / 32; t += RW) {
       f32x16 a3 = {}, a4 = {};
       tile_gemm(a3, A, lda, rt, kM, kM, 32 * t, lane);
       tile_gemm(a4, Hs, ldh, qt, kD, kD, 32 * t, lane);
@@ -640,14 +635,231 @@ __device__ __forceinline__ int route_pack_entry(RoutePackPtr kp, gpa_route_probl
   return pi;
 }
 
-// bf16 with 16-byte rows (the one-token decode path), 8 waves per workgroup.
-constexpr int RPACK_W = 8;
+// Weights of one 32-column tile, 128 contraction columns per batch: loaded as
+// whole 128-byte pieces of the tile's rows (8 rows per instruction; as fragments
+// an instruction would touch 32 rows for 32 bytes each, and the address path, not
+// the memory, sets the pace), turned into fragments through 4 KB of LDS of the
+// wave's own, 16-byte pieces swizzled by row.  Columns past the width are loaded
+// from column 0 and not used.
+typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+struct RouteBatch {
+  u32x4 lo[4], hi[4];  // columns 0..63, 64..127
+  // rows: the tile's first row; ld: its row length (the contraction width)
+  __device__ __forceinline__ void load(const bf16_t* rows, int k0, int ld, int lane) {
+    const int k = k0 + 8 * (lane & 7), ka = k < ld ? k : 0, kb = k + 64 < ld ? k + 64 : 0;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) lo[i] = *reinterpret_cast<const u32x4*>(rows + (8 * i + (lane >> 3)) * ld + ka);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) hi[i] = *reinterpret_cast<const u32x4*>(rows + (8 * i + (lane >> 3)) * ld + kb);
+  }
+  __device__ __forceinline__ void mma(f32x16& acc, const bf16_t* a, int k0, int k16, u32x4* buf, int lane) const {
+    if (k0 < k16) half(lo, acc, a, k0, k16, buf, lane);
+    if (k0 + 64 < k16) half(hi, acc, a, k0 + 64, k16, buf, lane);
+  }
+  static __device__ __forceinline__ void half(const u32x4 (&v)[4], f32x16& acc, const bf16_t* a, int k0, int k16,
+                                              u32x4* buf, int lane) {
+    const int li = lane & 31, hh = lane >> 5, r8 = lane >> 3;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) buf[(8 * i + r8) * 8 + ((lane ^ r8) & 7)] = v[i];
+    __builtin_amdgcn_wave_barrier();  // one wave's LDS operations run in order
+    u32x4 x[4];
+#pragma unroll
+    for (int s = 0; s < 4; ++s) x[s] = buf[li * 8 + ((2 * s + hh) ^ (li & 7))];
+    __builtin_amdgcn_wave_barrier();
+#pragma unroll
+    for (int s = 0; s < 4; ++s) {
+      bf16x8 w;
+      __builtin_memcpy(&w, &x[s], 16);
+      if (k0 + 16 * s < k16) mma_bf16(acc, *reinterpret_cast<const bf16x8*>(a + k0 + 16 * s), w);
+    }
+  }
+};
+
+// LDS of the packed read (bytes): r0 then r1, gelu(h1), q, and the scaled direct
+// term, all bf16 (exact: each is rounded to the activation type), and the waves'
+// fragment buffers.
+__host__ __device__ inline size_t route_pack_lds(int M, int Dk) {
+  const int kM = (M + 15) / 16 * 16, k2M = (2 * M + 15) / 16 * 16, kD = (Dk + 15) / 16 * 16, M32 = (M + 31) / 32 * 32;
+  return (size_t)2 * RR * (kM + 8 + k2M + 8 + kD + 8 + M32 + 8) + 16 * 4096;
+}
+
+// The one-token read (bf16, 16-byte rows), 16 waves per 32-row workgroup; the
+// bits of route_fwd.  A workgroup reads every weight of its head and level once
+// (0.8 MB at 256 slots, 128 keys) and the four products depend on one another,
+// so what counts is that the weights are on their way before the rows are:
+// every wave has the first 16 fragments of its next product in flight across the
+// barrier before it, and refills a batch as soon as its MFMAs have taken it.  The
+// direct term q W_qs runs on the waves that have no tile of hd.  Rows past
+// the call's are computed (their MFMA rows are there anyway) but skip the
+// elementwise work.  4 levels x 16 heads, (128,128,128,256) slots: 22.7 us at 1
+// row, 41 us at 64 (41 and 52 with 8 waves, flat loads and each batch of fragments
+// loaded where it is used; 31 and 47 with 16 waves and the early loads alone).
+constexpr int RPACK_W = 16;
 __global__ __launch_bounds__(64 * RPACK_W) void route_fwd_pack(RoutePack pk) {
+  typedef bf16_t E;
+  HIP_DYNAMIC_SHARED(float, lds)
+  __shared__ int row_b[RR], row_t[RR];
   const RoutePackPtr kp = (RoutePackPtr)__builtin_amdgcn_kernarg_segment_ptr();
   gpa_route_problem p;
   const int pi = route_pack_entry(kp, p);
-  const int local = (int)blockIdx.x - kp->wg0[pi], nt = kp->tiles[pi];
-  route_fwd_run<bf16_t, true, RPACK_W>(p, local / nt, (local % nt) * RR);
+  all_global(p.up_t, p.down_t, p.rs_t, p.qs_t, p.r0, p.h1, p.hd, p.qr, p.qdir, p.gain, p.mlp_gain, p.edge_weight,
+             p.base.ptr, p.q.ptr, p.route.ptr, p.qo.ptr);
+#pragma unroll
+  for (int e = 0; e < GPA_ROUTE_MAX_INCOMING; ++e) to_global(p.msg[e].ptr);
+  const int local = (int)blockIdx.x - kp->wg0[pi], nt = kp->tiles[pi], h = local / nt, row0 = (local % nt) * RR;
+  const int M = p.slots, Dk = p.key_dim, R = p.batch * p.tokens;
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), li = lane & 31, hh = lane >> 5;
+  const int kM = pad16(M), k2M = pad16(2 * M), kD = pad16(Dk), T1 = pad32(2 * M) / 32, T2 = pad32(M) / 32;
+  const int lda = kM + 8, ldh = k2M + 8, ldq = kD + 8, ldd = 32 * T2 + 8;
+  bf16_t* A = reinterpret_cast<bf16_t*>(lds);  // r0, then r1  [RR][lda]
+  bf16_t* Hs = A + RR * lda;                   // gelu(h1)     [RR][ldh]
+  bf16_t* Qs = Hs + RR * ldh;                  // q            [RR][ldq]
+  bf16_t* Ds = Qs + RR * ldq;                  // round(query_scale q W_qs)  [RR][ldd]
+  const bf16_t* ar = A + li * lda + 8 * hh;
+  const bf16_t* hr = Hs + li * ldh + 8 * hh;
+  const bf16_t* qr = Qs + li * ldq + 8 * hh;
+  u32x4* buf = reinterpret_cast<u32x4*>(Ds + RR * ldd) + 256 * wave;  // this wave's fragments
+  // weight rows of this wave's tiles (a tile past the last reads the last)
+  auto tile_row = [&](const void* w, int rows32, int k16, int t) {
+    t = t < rows32 / 32 ? t : rows32 / 32 - 1;
+    return reinterpret_cast<const bf16_t*>(w) + ((int64_t)h * rows32 + 32 * t) * k16;
+  };
+  const int td = wave - (RPACK_W - RMAX / 32);  // direct-term tile: waves 8 ..
+  const bf16_t* wu = tile_row(p.up_t, 32 * T1, kM, wave);
+  const bf16_t* wd = tile_row(p.down_t, 32 * T2, k2M, wave);
+  const bf16_t* wr = tile_row(p.rs_t, 32 * T2, kM, wave);
+  const bf16_t* wq = tile_row(p.qs_t, 32 * T2, kD, td < 0 ? 0 : td);
+  RouteBatch b0, b1;
+  b0.load(wu, 0, kM, lane);
+  b1.load(wu, 128, kM, lane);
+  const Rows rows = make_rows(row_b, row_t, row0, R, p.tokens);
+  E* sr0 = reinterpret_cast<E*>(p.r0) + (int64_t)h * R * M;
+  E* sh1 = reinterpret_cast<E*>(p.h1) + (int64_t)h * R * 2 * M;
+  E* shd = reinterpret_cast<E*>(p.hd) + (int64_t)h * R * M;
+  auto live = [&](int i) { return row0 + acc_row(i, 0) < R; };  // accumulator register i holds a row of the call
+
+  // ---- r0 = softmax(base + gain tanh z), q to LDS
+  {
+    const int c = 8 * (tid & 31), row = tid >> 5, r = row0 + row;
+    const bool ok = c < Dk && r < R;
+    const uint4 qv = *reinterpret_cast<const uint4*>(reinterpret_cast<const bf16_t*>(p.q.ptr) +
+                                                     rows.at(p.q, r < R ? r : R - 1, h) + (ok ? c : 0));
+    rows_r0_vec<E, 1, bf16_t>(p, rows, row0, h, sr0, A, lda, kM);
+    if (c < kD) *reinterpret_cast<uint4*>(Qs + row * ldq + c) = ok ? qv : make_uint4(0, 0, 0, 0);
+  }
+  lds_barrier();
+
+  // ---- h1 = r0 U, gelu(h1) -> Hs
+  f32x16 acc = {};
+  b0.mma(acc, ar, 0, kM, buf, lane);
+  b1.mma(acc, ar, 128, kM, buf, lane);
+  if (td >= 0) {
+    b0.load(wq, 0, kD, lane);
+    b1.load(wq, 128, kD, lane);
+  } else {
+    b0.load(wd, 0, k2M, lane);
+    b1.load(wd, 128, k2M, lane);
+  }
+  if (wave < T1) {
+    const int col = 32 * wave + li;
+#pragma unroll
+    for (int i = 0; i < 16; ++i) {
+      if (!live(i)) continue;
+      const int row = acc_row(i, hh), r = row0 + row;
+      if (col < 2 * M) {
+        const float h1 = round_as<E>(acc[i]);
+        if (r < R) sh1[(int64_t)r * 2 * M + col] = from_f32<E>(h1);
+        Hs[row * ldh + col] = from_f32<E>(gelu(h1));
+      } else if (col < k2M) {
+        Hs[row * ldh + col] = from_f32<E>(0.f);
+      }
+    }
+  }
+  // ---- the direct term (waves 8 ..): round(query_scale round(q W_qs)) -> Ds
+  if (td >= 0) {
+    f32x16 a4 = {};
+    b0.mma(a4, qr, 0, kD, buf, lane);
+    b1.mma(a4, qr, 128, kD, buf, lane);
+    if (td < T2)
+#pragma unroll
+      for (int i = 0; i < 16; ++i)
+        if (live(i)) Ds[acc_row(i, hh) * ldd + 32 * td + li] = from_f32<E>(p.query_scale * round_as<E>(a4[i]));
+  }
+  lds_barrier();
+
+  // ---- hd = gelu(h1) D, r1 = r0 + mlp_gain hd -> A and the route output
+  E* route = reinterpret_cast<E*>(p.route.ptr);
+  if (td < 0) {
+    f32x16 c = {};
+    b0.mma(c, hr, 0, k2M, buf, lane);
+    b0.load(wd, 256, k2M, lane);
+    b1.mma(c, hr, 128, k2M, buf, lane);
+    b1.load(wd, 384, k2M, lane);
+    b0.mma(c, hr, 256, k2M, buf, lane);
+    b0.load(wr, 0, kM, lane);
+    b1.mma(c, hr, 384, k2M, buf, lane);
+    b1.load(wr, 128, kM, lane);
+    const float g = p.mlp_gain[h];
+    const int col = 32 * wave + li;
+    if (wave < T2 && col < M)
+#pragma unroll
+      for (int i = 0; i < 16; ++i) {
+        if (!live(i)) continue;
+        const int row = acc_row(i, hh), r = row0 + row;
+        const float hd = round_as<E>(c[i]);
+        const E r1 = from_f32<E>(to_f32(A[row * lda + col]) + g * hd);
+        A[row * lda + col] = r1;
+        if (r < R) {
+          shd[(int64_t)r * M + col] = from_f32<E>(hd);
+          if (!p.rsa) route[rows.at(p.route, r, h) + col] = r1;
+        }
+      }
+  }
+  lds_barrier();
+
+  // ---- rsa_update: r1 <- round(r1 / clamp(sum |r1|, .25, 4)) in A and the route output
+  if (p.rsa) {
+    if (tid < RNT) {
+      const int row = tid >> 3, part = tid & 7, r = row0 + row;
+      float s = 0.f;
+#pragma unroll
+      for (int i = 0; i < RPER; ++i)
+        if (part + 8 * i < M) s += fabsf(to_f32(A[row * lda + part + 8 * i]));
+      const float l = fminf(fmaxf(sum8(s), .25f), 4.f);
+#pragma unroll
+      for (int i = 0; i < RPER; ++i) {
+        const int m = part + 8 * i;
+        if (m < M) {
+          const E x = from_f32<E>(to_f32(A[row * lda + m]) / l);
+          A[row * lda + m] = x;
+          if (r < R) route[rows.at(p.route, r, h) + m] = x;
+        }
+      }
+    }
+    lds_barrier();
+  }
+
+  // ---- qo = r1 W_rs + the direct term
+  if (td < 0) {
+    f32x16 a3 = {};
+    b0.mma(a3, ar, 0, kM, buf, lane);
+    b1.mma(a3, ar, 128, kM, buf, lane);
+    E* qo = reinterpret_cast<E*>(p.qo.ptr);
+    const int col = 32 * wave + li;
+    if (wave < T2 && col < M)
+#pragma unroll
+      for (int i = 0; i < 16; ++i) {
+        const int row = acc_row(i, hh), r = row0 + row;
+        if (!live(i) || r >= R) continue;
+        const E dir = Ds[row * ldd + col];
+        if (p.balanced) {  // both halves saved; route_mix_fwd forms qo from their unit rows
+          reinterpret_cast<E*>(p.qr)[((int64_t)h * R + r) * M + col] = from_f32<E>(a3[i]);
+          reinterpret_cast<E*>(p.qdir)[((int64_t)h * R + r) * M + col] = dir;
+        } else {
+          qo[rows.at(p.qo, r, h) + col] = from_f32<E>(round_as<E>(a3[i]) + to_f32(dir));
+        }
+      }
+  }
 }
 
 // ---------------------------------------------------------------- rsa_update and balanced_bridge rows
@@ -882,7 +1094,7 @@ __global__ __launch_bounds__(RNT) void route_rows16(gpa_route_problem p) {
   const int h = rtile.h, row0 = rtile.tile * RR;
   __shared__ int row_b[RR], row_t[RR];
   const Rows rows = make_rows(row_b, row_t, row0, R, p.tokens);
-  rows_r0_vec<bf16_t>(p, rows, row0, h, reinterpret_cast<bf16_t*>(p.r0) + (int64_t)h * R * M, nullptr, 0, 0);
+  rows_r0_vec<bf16_t>(p, rows, row0, h, reinterpret_cast<bf16_t*>(p.r0) + (int64_t)h * R * M, static_cast<float*>(nullptr), 0, 0);
 }
 
 constexpr int GM_BM = 128;           // rows per tile
@@ -2201,7 +2413,7 @@ extern "C" int gpa_route_forward_many(const gpa_route_problem* problems, int32_t
     pk.wg0[i] = total;
     pk.tiles[i] = (p.batch * p.tokens + RR - 1) / RR;
     total += pk.tiles[i] * p.heads;
-    lds = std::max(lds, fwd_lds(p));
+    lds = std::max(lds, route_pack_lds(p.slots, p.key_dim));
   }
   if (int rc = set_lds(route_fwd_pack, lds)) return rc;
   hipLaunchKernelGGL(route_fwd_pack, dim3(total), dim3(64 * RPACK_W), lds, stream, pk);

@@ -99,6 +99,7 @@ __global__ __launch_bounds__(256) void token_logits_pack(LogitsPack pk) {
     if ((int)blockIdx.x >= kp->wg0[i]) pi = i;
   gpa_token_logits_problem p;
   kernarg_copy(p, &kp->p[pi]);
+  all_global(p.raw.ptr, p.write.ptr, p.count0, p.gain, p.scale, p.logits, p.count, p.local);
   const int row = ((int)blockIdx.x - kp->wg0[pi]) * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63;
   if (row >= p.batch * p.heads) return;
   token_logits_row<E>(p, row / p.heads, row % p.heads, lane);

@@ -161,6 +161,8 @@ inline uint32_t emu_perm(uint32_t a, uint32_t b, uint32_t sel) {
 #define __builtin_amdgcn_mfma_f32_32x32x2f32(a, b, c, x, y, z) emu_mfma_32x32x2_f32(a, b, c)
 #define __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, x, y, z) emu_mfma_16x16x4_f32(a, b, c)
 
+// In-wave ordering of LDS accesses: the wave's threads meet here.
+#define __builtin_amdgcn_wave_barrier() emu_wave_barrier[threadIdx.x / 64]->arrive_and_wait()
 // v_permlane32_swap / v_permlane16_swap: the upper half (odd 16-lane rows) of
 // the first operand trades places with the lower half (even rows) of the second.
 struct emu_pair {
