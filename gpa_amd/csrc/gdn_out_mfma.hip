@@ -336,14 +336,16 @@ __global__ __launch_bounds__(ONT) void gdn_prep_q(gpa_gdn_problem p, gpa_gdn_sav
 #pragma unroll
     for (int i = 0; i < NI; ++i) {
       const int d = lane + 64 * i;
+      const float yq = round_as<E>(xq[j][i] / dq);
       if (d < K) {
-        const float yq = round_as<E>(xq[j][i] / dq);
         if (MF) reinterpret_cast<bf16_t*>(sv.qn)[rows_off(s, n, nch, r, K) + d] = from_f32<bf16_t>(yq);
         else sv.qn[rows_off(s, n, nch, r, K) + d] = yq;
-        if (MF) {  // Qn^T fragment (d/32, r/16), lane d%32 + 32 ((r/8) % 2), element r % 8
-          const int rb = d >> 5, cs = r >> 4, ln = (d & 31) + 32 * ((r >> 3) & 1);
-          qcol[((rb * 4 + cs) * 64 + ln) * 8 + (r & 7)] = (__bf16)yq;
-        }
+      }
+      // Qn^T fragment (d/32, r/16), lane d%32 + 32 ((r/8) % 2), element r % 8: whole
+      // 32-key tiles, zero past K (the chunk backward multiplies the padding too)
+      if (MF && d < (K + 31) / 32 * 32) {
+        const int rb = d >> 5, cs = r >> 4, ln = (d & 31) + 32 * ((r >> 3) & 1);
+        qcol[((rb * 4 + cs) * 64 + ln) * 8 + (r & 7)] = (__bf16)yq;
       }
     }
   }
