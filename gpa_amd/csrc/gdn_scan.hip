@@ -209,144 +209,170 @@ __global__ __launch_bounds__(NT) void gdn_state_fwd(gpa_gdn_problem p, gpa_gdn_s
       if (kb + j < K) sv.final[(int64_t)s * K * V + (int64_t)(kb + j) * V + v] = S[j % VEC][j / VEC];
 }
 
-// ---------------------------------------------------------------------------
-// The chunk-parallel reads of the float32 path on v_mfma_f32_16x16x4f32
-// (gdn_out_fwd, gdn_dd0; also bf16 scans whose keys or values the bf16 MFMA kernels
-// do not take): one workgroup per (chunk, stream), wave w owns 16 positions and
-// works alone, without barriers.  Its 16 rows of P (or of P^T) are formed in
-// accumulators, pass through LDS of its own into operand order, and multiply
-// value-major D, S_n or the dO rows, whose operands are plain 16-byte reads.  Only
-// the causal tiles of P are formed.  Bound: the waves' MFMA chains; 32 streams x 16
-// chunks, 64 x 96: read 23 us, gradient 17 us (56 and 40 as scalar FMA
-// products over LDS tiles).
-constexpr int PLD = R + 4;  // row pitch of a wave's P rows
-
-// Rows 16 w + 4 q + r (accumulator order) of P, or of P^T with TRANS, into the
-// wave's LDS rows: P_tu = e^{G_t-G_u} Qn_t . Kn_u, u <= t.
-template <int KM, bool FULL, bool TRANS>
-__device__ __forceinline__ void wave_p_rows(float* ps, const float* own, const float* other, const float* gam, int w,
-                                            int col, int q, int K) {
-  f32x4 x[KM / 16];
-  load_rows<KM, FULL>(x, own, 16 * w + col, q, K);
-  const f32x4 go = *reinterpret_cast<const f32x4*>(gam + 16 * w + 4 * q);
+// P = causal e^{G_t-G_s} Qn Kn^T into p_s ([R][LDR]); uses two R x KS slices.
+template <int KM>
+__device__ void build_p(float* p_s, float* a_s, float* b_s, const float* qn, const float* kn,
+                        const float* gam_s, int K) {
+  const int tid = threadIdx.x, ty = tid / 16, tx = tid % 16;
+  float acc[4][4] = {};
+  for (int k0 = 0; k0 < KM; k0 += KS) {
+    __syncthreads();
+    stage_rows(a_s, qn, K, k0, nullptr);
+    stage_rows(b_s, kn, K, k0, nullptr);
+    __syncthreads();
+    for (int kk = 0; kk < KS; ++kk) {
+      float a[4], c[4];
 #pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    if (TRANS ? i < w : i > w) continue;  // (uniform) no tile on this side of the diagonal
-    f32x4 y[KM / 16], acc = {0.f, 0.f, 0.f, 0.f};
-    load_rows<KM, FULL>(y, other, 16 * i + col, q, K);
-    const float gu = gam[16 * i + col];
+      for (int i = 0; i < 4; ++i) a[i] = a_s[(4 * ty + i) * LDS_ + kk];
 #pragma unroll
-    for (int g = 0; g < KM / 16; ++g)
-      if (16 * g < K) mma16(acc, x[g], y[g]);
+      for (int j = 0; j < 4; ++j) c[j] = b_s[(tx + 16 * j) * LDS_ + kk];
 #pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      const int a = 16 * w + 4 * q + r, c = 16 * i + col;  // own row, other row
-      const bool live = TRANS ? a <= c : c <= a;
-      const float e = __expf(live ? (TRANS ? gu - go[r] : go[r] - gu) : 0.f);
-      ps[(4 * q + r) * PLD + c] = live ? e * acc[r] : 0.f;
+      for (int i = 0; i < 4; ++i)
+#pragma unroll
+        for (int j = 0; j < 4; ++j) acc[i][j] += a[i] * c[j];
     }
   }
-  __builtin_amdgcn_wave_barrier();  // one wave's LDS operations run in order
+#pragma unroll
+  for (int i = 0; i < 4; ++i)
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      const int t = 4 * ty + i, u = tx + 16 * j;
+      p_s[t * LDR + u] = (u <= t) ? __expf(gam_s[t] - gam_s[u]) * acc[i][j] : 0.f;
+    }
+  __syncthreads();
 }
 
-// gdn_out_fwd: O = diag(e^G) Qn S_n + P D.
-template <typename E, int KM, bool FULL>
+// ---------------------------------------------------------------------------
+// gdn_out_fwd: O = diag(e^G) Qn S_n + P D, one block per (chunk, stream).
+template <typename E, int KM>
 __global__ __launch_bounds__(NT) void gdn_out_fwd(gpa_gdn_problem p, gpa_gdn_saved sv, gpa_operand out,
                                                    int nch) {
-  __shared__ __align__(16) float p_s[NT / 64][16 * PLD];
+  extern __shared__ float smem[];
+  float* p_s = smem;              // [R][LDR]
+  float* a_s = p_s + R * LDR;     // [R][LDS_]
+  float* b_s = a_s + R * LDS_;    // [R][LDS_]  (also KS x 64 state slice)
+  float* gam_s = b_s + R * LDS_;  // [R]
   const int n = blockIdx.x, s = blockIdx.y, b = s / p.heads, h = s % p.heads;
-  const int K = p.kdim, V = p.vdim, tid = threadIdx.x, w = __builtin_amdgcn_readfirstlane(tid / 64);
-  const int col = tid % 16, q = tid % 64 / 16;
-  const float* gam = sv.gam + rows_off(s, n, nch, 0, 1);
+  const int K = p.kdim, V = p.vdim, tid = threadIdx.x, ty = tid / 16, tx = tid % 16;
+  if (tid < R) gam_s[tid] = sv.gam[rows_off(s, n, nch, 0, 1) + tid];
+  __syncthreads();
   const float* qn = sv.qn + rows_off(s, n, nch, 0, K);
-  float* ps = p_s[w];
-  wave_p_rows<KM, FULL, false>(ps, qn, sv.kn + rows_off(s, n, nch, 0, K), gam, w, col, q, K);
-  f32x4 qr[KM / 16], pr[4], eg = *reinterpret_cast<const f32x4*>(gam + 16 * w + 4 * q);
-  load_rows<KM, FULL>(qr, qn, 16 * w + col, q, K);
-#pragma unroll
-  for (int i = 0; i < 4; ++i)
-    pr[i] = i <= w ? *reinterpret_cast<const f32x4*>(ps + col * PLD + 16 * i + 4 * q) : f32x4{0.f, 0.f, 0.f, 0.f};
-  int tok[4];
-#pragma unroll
-  for (int r = 0; r < 4; ++r) {
-    eg[r] = __expf(eg[r]);
-    tok[r] = token_at(p, n, 16 * w + 4 * q + r);
-  }
+  build_p<KM>(p_s, a_s, b_s, qn, sv.kn + rows_off(s, n, nch, 0, K), gam_s, K);
   const float* st = sv.states + state_off(s, n, nch, K, V);
   const float* dl = sv.delta + vc_off(s, n, nch, V);
-  E* o = reinterpret_cast<E*>(out.ptr) + op_base(out, b, h);
-  for (int v0 = 0; v0 < V; v0 += 16) {
-    const int v = v0 + col, vc = v < V ? v : V - 1;
-    f32x4 s4[KM / 16], d4[4], acc = {0.f, 0.f, 0.f, 0.f};
+  for (int v0 = 0; v0 < V; v0 += 64) {
+    float acc[4][4] = {};
+    for (int k0 = 0; k0 < KM; k0 += KS) {
+      __syncthreads();
+      stage_rows(a_s, qn, K, k0, nullptr);
+      for (int idx = tid; idx < KS * 64; idx += NT) {
+        const int kk = idx % KS, c = idx / KS;
+        b_s[kk * LDS_ + c] = (k0 + kk < K && v0 + c < V) ? st[(int64_t)(v0 + c) * K + k0 + kk] : 0.f;
+      }
+      __syncthreads();
+      for (int kk = 0; kk < KS; ++kk) {
+        float a[4], c[4];
 #pragma unroll
-    for (int g = 0; g < KM / 16; ++g) s4[g] = row4<FULL>(st + (int64_t)vc * K, 16 * g + 4 * q, K);
+        for (int i = 0; i < 4; ++i) a[i] = a_s[(4 * ty + i) * LDS_ + kk];
 #pragma unroll
-    for (int i = 0; i < 4; ++i) d4[i] = *reinterpret_cast<const f32x4*>(dl + (int64_t)vc * R + 16 * i + 4 * q);
+        for (int j = 0; j < 4; ++j) c[j] = b_s[kk * LDS_ + tx + 16 * j];
 #pragma unroll
-    for (int g = 0; g < KM / 16; ++g)
-      if (16 * g < K) mma16(acc, qr[g], s4[g]);
-    acc *= eg;
+        for (int i = 0; i < 4; ++i)
 #pragma unroll
-    for (int i = 0; i < 4; ++i)
-      if (i <= w) mma16(acc, pr[i], d4[i]);
+          for (int j = 0; j < 4; ++j) acc[i][j] += a[i] * c[j];
+      }
+    }
 #pragma unroll
-    for (int r = 0; r < 4; ++r)
-      if (tok[r] >= 0 && v < V) o[(int64_t)tok[r] * out.st + v] = from_f32<E>(acc[r]);
+    for (int i = 0; i < 4; ++i) {
+      const float e = __expf(gam_s[4 * ty + i]);
+#pragma unroll
+      for (int j = 0; j < 4; ++j) acc[i][j] *= e;
+    }
+    __syncthreads();
+    for (int idx = tid; idx < R * 64; idx += NT) {
+      const int u = idx % R, c = idx / R;
+      b_s[u * LDS_ + c] = v0 + c < V ? dl[(int64_t)(v0 + c) * R + u] : 0.f;
+    }
+    __syncthreads();
+    for (int u = 0; u < R; ++u) {
+      float a[4], c[4];
+#pragma unroll
+      for (int i = 0; i < 4; ++i) a[i] = p_s[(4 * ty + i) * LDR + u];
+#pragma unroll
+      for (int j = 0; j < 4; ++j) c[j] = b_s[u * LDS_ + tx + 16 * j];
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+#pragma unroll
+        for (int j = 0; j < 4; ++j) acc[i][j] += a[i] * c[j];
+    }
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const int t = token_at(p, n, 4 * ty + i);
+      if (t < 0) continue;
+      E* o = reinterpret_cast<E*>(out.ptr) + op_base(out, b, h) + (int64_t)t * out.st;
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        const int v = v0 + tx + 16 * j;
+        if (v < V) o[v] = from_f32<E>(acc[i][j]);
+      }
+    }
   }
 }
 
+// ---------------------------------------------------------------------------
 // gdn_dd0: dd0 = P^T dO (the part of dD not carried by the state), and
 // o = diag(e^G) dO, both value-major [V][R] per chunk.
-template <typename E, int KM, bool FULL>
+template <typename E, int KM>
 __global__ __launch_bounds__(NT) void gdn_dd0(gpa_gdn_problem p, gpa_gdn_saved sv, gpa_gdn_grads gr,
                                                int nch) {
-  __shared__ __align__(16) float p_s[NT / 64][16 * PLD];
+  extern __shared__ float smem[];
+  float* p_s = smem;
+  float* a_s = p_s + R * LDR;
+  float* b_s = a_s + R * LDS_;
+  float* gam_s = b_s + R * LDS_;
   const int n = blockIdx.x, s = blockIdx.y, b = s / p.heads, h = s % p.heads;
-  const int K = p.kdim, V = p.vdim, tid = threadIdx.x, w = __builtin_amdgcn_readfirstlane(tid / 64);
-  const int col = tid % 16, q = tid % 64 / 16, t0 = 16 * w + 4 * q;
-  const float* gam = sv.gam + rows_off(s, n, nch, 0, 1);
-  float* ps = p_s[w];
-  wave_p_rows<KM, FULL, true>(ps, sv.kn + rows_off(s, n, nch, 0, K), sv.qn + rows_off(s, n, nch, 0, K), gam, w, col, q, K);
-  f32x4 pr[4], eg = *reinterpret_cast<const f32x4*>(gam + t0);
-#pragma unroll
-  for (int i = 0; i < 4; ++i)
-    pr[i] = i >= w ? *reinterpret_cast<const f32x4*>(ps + col * PLD + 16 * i + 4 * q) : f32x4{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-  for (int r = 0; r < 4; ++r) eg[r] = __expf(eg[r]);
-  // dd0 and o are value-major for the float32 state kernels and in fragment order
-  // (ufrag_idx, whole 32-column strips, zero past V) for the MFMA ones (bf16, K a
-  // multiple of 16); four consecutive rows are contiguous in both.
+  const int K = p.kdim, V = p.vdim, tid = threadIdx.x, ty = tid / 16, tx = tid % 16;
+  if (tid < R) gam_s[tid] = sv.gam[rows_off(s, n, nch, 0, 1) + tid];
+  __syncthreads();
+  build_p<KM>(p_s, a_s, b_s, sv.qn + rows_off(s, n, nch, 0, K), sv.kn + rows_off(s, n, nch, 0, K), gam_s, K);
+  // dd0 and o are value-major for the FMA state kernels and in fragment order
+  // (ufrag_idx) for the MFMA ones (bf16, K a multiple of 16).
   const bool frag = std::is_same<E, bf16_t>::value && K % 16 == 0;
-  const int VP = frag ? ufrag_v(V) : V;
   float* d0 = gr.dd0 + (frag ? ufrag_off(s, n, nch, V) : vc_off(s, n, nch, V));
   float* om = gr.o + (frag ? ufrag_off(s, n, nch, V) : vc_off(s, n, nch, V));
-  const E* dout = reinterpret_cast<const E*>(gr.dout.ptr) + op_base(gr.dout, b, h);
-  int64_t row[16];  // this lane's dO rows (clamped to token 0), bit r of `real` set where there is one
-  uint32_t real = 0;
+  auto at = [&](int v, int r) -> int64_t { return frag ? ufrag_elem(v, r) : (int64_t)v * R + r; };
+  for (int v0 = 0; v0 < V; v0 += 64) {
+    __syncthreads();
+    for (int idx = tid; idx < R * 64; idx += NT) {
+      const int r = idx / 64, c = idx % 64;
+      const int t = token_at(p, n, r);
+      b_s[r * LDS_ + c] = (t >= 0 && v0 + c < V) ? op_load<E>(gr.dout, b, h, t, v0 + c) : 0.f;
+    }
+    __syncthreads();
+    for (int idx = tid; idx < R * 64; idx += NT) {
+      const int r = idx % R, c = idx / R;
+      if (v0 + c < V) om[at(v0 + c, r)] = __expf(gam_s[r]) * b_s[r * LDS_ + c];
+      else if (frag && v0 + c < ufrag_v(V)) om[at(v0 + c, r)] = 0.f;
+    }
+    float acc[4][4] = {};
+    for (int u = 0; u < R; ++u) {  // acc[t'][v] += P[u][t'] dO[u][v]
+      float a[4], c[4];
 #pragma unroll
-  for (int r = 0; r < 16; ++r) {
-    const int t = token_at(p, n, 16 * (r / 4) + 4 * q + r % 4);
-    row[r] = (int64_t)(t >= 0 ? t : 0) * gr.dout.st;
-    real |= t >= 0 ? 1u << r : 0u;
-  }
-  for (int v0 = 0; v0 < VP; v0 += 16) {
-    const int v = v0 + col, vc = v < V ? v : V - 1;
-    E raw[16];
+      for (int i = 0; i < 4; ++i) a[i] = p_s[u * LDR + 4 * ty + i];
 #pragma unroll
-    for (int r = 0; r < 16; ++r) raw[r] = dout[row[r] + vc];
-    f32x4 x[4], acc = {0.f, 0.f, 0.f, 0.f};
+      for (int j = 0; j < 4; ++j) c[j] = b_s[u * LDS_ + tx + 16 * j];
 #pragma unroll
-    for (int r = 0; r < 16; ++r) x[r / 4][r % 4] = (real >> r & 1) && v < V ? to_f32(raw[r]) : 0.f;
+      for (int i = 0; i < 4; ++i)
 #pragma unroll
-    for (int i = 0; i < 4; ++i)
-      if (i >= w) mma16(acc, pr[i], x[i]);
-    f32x4 mine = x[0];
+        for (int j = 0; j < 4; ++j) acc[i][j] += a[i] * c[j];
+    }
 #pragma unroll
-    for (int i = 1; i < 4; ++i) mine = i == w ? x[i] : mine;
-    if (v < VP) {
-      const int64_t at = frag ? ufrag_elem(v, t0) : (int64_t)v * R + t0;
-      *reinterpret_cast<f32x4*>(d0 + at) = acc;
-      *reinterpret_cast<f32x4*>(om + at) = eg * mine;
+    for (int j = 0; j < 4; ++j) {
+      const int v = v0 + tx + 16 * j;  // four consecutive rows are contiguous in both layouts
+      if (v < V)
+        *reinterpret_cast<float4*>(&d0[at(v, 4 * ty)]) = make_float4(acc[0][j], acc[1][j], acc[2][j], acc[3][j]);
+      else if (frag && v < ufrag_v(V))
+        *reinterpret_cast<float4*>(&d0[at(v, 4 * ty)]) = make_float4(0.f, 0.f, 0.f, 0.f);
     }
   }
 }
@@ -456,39 +482,6 @@ __global__ __launch_bounds__(NT) void gdn_state_bwd(gpa_gdn_problem p, gpa_gdn_s
 #pragma unroll
     for (int j = 0; j < 4 * VEC; ++j)
       if (kb + j < K) gr.ds0[(int64_t)s * K * V + (int64_t)(kb + j) * V + v] = S[j % VEC][j / VEC];
-}
-
-// P = causal e^{G_t-G_s} Qn Kn^T into p_s ([R][LDR]); uses two R x KS slices.
-template <int KM>
-__device__ void build_p(float* p_s, float* a_s, float* b_s, const float* qn, const float* kn,
-                        const float* gam_s, int K) {
-  const int tid = threadIdx.x, ty = tid / 16, tx = tid % 16;
-  float acc[4][4] = {};
-  for (int k0 = 0; k0 < KM; k0 += KS) {
-    __syncthreads();
-    stage_rows(a_s, qn, K, k0, nullptr);
-    stage_rows(b_s, kn, K, k0, nullptr);
-    __syncthreads();
-    for (int kk = 0; kk < KS; ++kk) {
-      float a[4], c[4];
-#pragma unroll
-      for (int i = 0; i < 4; ++i) a[i] = a_s[(4 * ty + i) * LDS_ + kk];
-#pragma unroll
-      for (int j = 0; j < 4; ++j) c[j] = b_s[(tx + 16 * j) * LDS_ + kk];
-#pragma unroll
-      for (int i = 0; i < 4; ++i)
-#pragma unroll
-        for (int j = 0; j < 4; ++j) acc[i][j] += a[i] * c[j];
-    }
-  }
-#pragma unroll
-  for (int i = 0; i < 4; ++i)
-#pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      const int t = 4 * ty + i, u = tx + 16 * j;
-      p_s[t * LDR + u] = (u <= t) ? __expf(gam_s[t] - gam_s[u]) * acc[i][j] : 0.f;
-    }
-  __syncthreads();
 }
 
 // ---------------------------------------------------------------------------
@@ -1071,9 +1064,9 @@ int fwd_state(const gpa_gdn_problem& p, const gpa_gdn_saved& sv, int nch, hipStr
 template <typename E, int KM>
 int fwd_out(const gpa_gdn_problem& p, const gpa_gdn_saved& sv, gpa_operand out, int nch, hipStream_t st) {
   if (use_mfma<E>(p) && p.vdim <= GPA_OUT_MFMA_MAX_V) return launch_out_mfma<KM>(p, sv, out, nch, st);
-  const dim3 grid(nch, p.batch * p.heads);
-  if (p.kdim % 16 == 0) hipLaunchKernelGGL((gdn_out_fwd<E, KM, true>), grid, dim3(NT), 0, st, p, sv, out, nch);
-  else hipLaunchKernelGGL((gdn_out_fwd<E, KM, false>), grid, dim3(NT), 0, st, p, sv, out, nch);
+  const dim3 grid_c(nch, p.batch * p.heads), block(NT);
+  const size_t lds_out = sizeof(float) * (R * LDR + 2 * R * LDS_ + R);
+  hipLaunchKernelGGL((gdn_out_fwd<E, KM>), grid_c, block, lds_out, st, p, sv, out, nch);
   return GPA_HIP_OK;
 }
 
@@ -1091,9 +1084,9 @@ gpa_gdn_grads effective_grads(const gpa_gdn_problem& p, gpa_gdn_grads gr) {
 template <typename E, int KM>
 int bwd_dd0(const gpa_gdn_problem& p, const gpa_gdn_saved& sv, const gpa_gdn_grads& gr, int nch, hipStream_t st) {
   if (use_mfma<E>(p) && p.vdim <= GPA_OUT_MFMA_MAX_V) return launch_dd0_mfma<KM>(p, sv, gr, nch, st);
-  const dim3 grid(nch, p.batch * p.heads);
-  if (p.kdim % 16 == 0) hipLaunchKernelGGL((gdn_dd0<E, KM, true>), grid, dim3(NT), 0, st, p, sv, gr, nch);
-  else hipLaunchKernelGGL((gdn_dd0<E, KM, false>), grid, dim3(NT), 0, st, p, sv, gr, nch);
+  const dim3 grid_c(nch, p.batch * p.heads), block(NT);
+  const size_t lds = sizeof(float) * (R * LDR + 2 * R * LDS_ + R);
+  hipLaunchKernelGGL((gdn_dd0<E, KM>), grid_c, block, lds, st, p, sv, gr, nch);
   return GPA_HIP_OK;
 }
 

@@ -32,27 +32,3 @@ def test_float32_state_matches_recurrence(case):
     errs = [_rel(a, b) for a, b in zip((*got, *dg), (*want, *dr))]
     print(case, errs)
     assert max(errs) < 1e-5, errs
-
-
-# (T, K, V, chunk, offset): bf16 calls of the float32 read kernels (gdn_out_fwd, gdn_dd0),
-# values above 256 with fragment-ordered gradients, and key widths off 16.
-READS = [(70, 48, 264, 64, 5), (20, 20, 17, 8, 3), (65, 80, 290, 64, 0), (130, 130, 40, 64, 63)]
-
-
-@pytest.mark.parametrize("case", READS, ids=lambda c: "T{}K{}V{}C{}o{}".format(*c))
-def test_bf16_calls_of_the_float32_reads(case):
-    """Bound: the scan tests' 2e-2, inputs and results rounded to bf16 at 2^-9."""
-    from gpa_amd.ops import gdn_scan_hip
-    t, kd, vd, chunk, offset = case
-    inputs = _inputs(2, t, 2, kd, vd, torch.bfloat16, seed=23)
-    leaves = [x.to(DEV).requires_grad_() for x in inputs]
-    refs = [x.double().requires_grad_() for x in inputs]
-    got = gdn_scan_hip(*leaves, chunk=chunk, offset=offset)
-    want = _oracle_segments_autograd(refs[:3], *refs[3:], chunk, offset)
-    gen = torch.Generator().manual_seed(3)
-    grads = [torch.randn(x.shape, generator=gen).to(torch.bfloat16) for x in want]
-    dg = torch.autograd.grad(got, leaves, [w.to(DEV, x.dtype) for w, x in zip(grads, got)])
-    dr = torch.autograd.grad(want, refs, [w.double() for w in grads])
-    errs = [_rel(a, b) for a, b in zip((*got, *dg), (*want, *dr))]
-    print(case, errs)
-    assert max(errs) < 2e-2, errs
