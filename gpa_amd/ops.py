@@ -48,6 +48,43 @@ def _in_use_here(*tensors):
             t.record_stream(stream)
 
 
+def _pieces(base, width, sizes):
+    """Addresses of consecutive buffers of the given element counts in one
+    allocation (None for 0).  Every size is a multiple of 64 elements."""
+    at = base.data_ptr() if base is not None else None
+    out = []
+    for n in sizes:
+        out.append(at if n else None)
+        at = at + width * n if n else at
+    return out
+
+
+def _layout(rows, kd, vd, mfma, read):
+    """Element counts of a scan's saved float32 buffers (kn, qn, w, u, delta,
+    tri, gam, bet) and bf16 fragments (wrow, wcol, krow, kcol, qcol; MFMA path
+    only), layouts of include/gpa_hip.h.  Each kind is one allocation, cut here:
+    a buffer of its own costs the host 3 us, and a scan of one block, whose kernels take
+    49 us, took 62 with them.  U is
+    value-major [S,N,V,64] on the FMA path, on the MFMA path in fragment order
+    over ceil(V/32) whole 32-column strips."""
+    f32 = (rows * kd, rows * kd if read else 0, 0 if mfma else rows * kd,
+           rows * (-(-vd // 32) * 32 if mfma else vd), rows * vd, rows * _lib.CHUNK_ROWS, rows, rows)
+    if not mfma:
+        return f32, (0,) * 5
+    row, col = 2 * (kd // 16) * rows * 8, (kd + 31) // 32 * 4 * rows * 8
+    return f32, (2 * row, 2 * col, row, col, col if read else 0)
+
+
+def _saved(inter, layout, qn=None, qcol=None):
+    """The library's record of a scan's saved intermediates (work, frag,
+    states, final); qn and qcol of a late read are tensors of their own."""
+    work, frag, states, final = inter
+    kn, own_qn, *rest = _pieces(work, 4, layout[0])
+    *frags, own_qcol = _pieces(frag, 2, layout[1])
+    return _lib.Saved(kn, own_qn if qn is None else qn.data_ptr(), *rest, states.data_ptr(), final.data_ptr(),
+                      *frags, own_qcol if qcol is None else qcol.data_ptr())
+
+
 class _Group:
     """One scan group's forward: its problem, saved intermediates (layouts of
     include/gpa_hip.h) and outputs."""
@@ -65,45 +102,29 @@ class _Group:
         mfma = lib.gpa_gdn_path(self.prob) == 1
         chunks = bsz * heads * nch
         rows = chunks * _lib.CHUNK_ROWS
+        layout = _layout(rows, kd, vd, mfma, q is not None)
         f32 = dict(device=dev, dtype=torch.float32)
-        b16 = dict(device=dev, dtype=torch.bfloat16)
-        kn = torch.empty(rows * kd, **f32)
-        qn = torch.empty(rows * kd, **f32) if q is not None else None
-        w = torch.empty(rows * kd, **f32) if not mfma else None
-        # U: value-major [S,N,V,64] on the FMA path; on the MFMA path fragment
-        # order over ceil(V/32) whole 32-column strips (include/gpa_hip.h).
-        u = torch.empty(rows * (-(-vd // 32) * 32 if mfma else vd), **f32)
-        delta = torch.empty(rows * vd, **f32)
-        tri = torch.empty(rows * _lib.CHUNK_ROWS, **f32)
-        gam = torch.empty(rows, **f32)
-        bet = torch.empty(rows, **f32)
+        work = torch.empty(sum(layout[0]), **f32)
+        frag = torch.empty(sum(layout[1]), device=dev, dtype=torch.bfloat16) if mfma else None
         self.states = torch.empty(bsz, heads, nch, vd, kd, **f32)   # value-major chunk-start states
         self.final = torch.empty(bsz, heads, kd, vd, **f32)
-        frags = [None] * 5
-        if mfma:
-            k16, rb = kd // 16, (kd + 31) // 32
-            frags = [torch.empty(chunks * 2 * k16 * 64 * 16, **b16),   # wrow
-                     torch.empty(chunks * rb * 4 * 64 * 16, **b16),    # wcol
-                     torch.empty(chunks * 2 * k16 * 64 * 8, **b16),    # krow
-                     torch.empty(chunks * rb * 4 * 64 * 8, **b16),     # kcol
-                     torch.empty(chunks * rb * 4 * 64 * 8, **b16) if q is not None else None]  # qcol
         self.out = torch.empty(bsz, tokens, heads, vd, device=dev, dtype=k.dtype) if q is not None else None
-        self.inter = (kn, qn, w, u, delta, tri, gam, bet, self.states, self.final, *frags)
-        self.saved = _lib.Saved(*(_ptr(t) for t in self.inter))
+        inter = (work, frag, self.states, self.final)
+        self.saved = _saved(inter, layout)
         self.geom = (chunk, offset, nch, q is not None, s0 is not None, mfma)
         self.timing_args = (kd, vd, chunk, tokens * bsz * heads, k.dtype, q is not None)
-        self.tensors = (q, k, v, g, beta, s0f) + self.inter
+        self.tensors = (q, k, v, g, beta, s0f) + inter
         self.token = None
         if box is not None:  # a late read will use these intermediates
             box.args = (k, v, g, beta, s0f, chunk, offset, nch)
-            box.saved = (kn, w, u, delta, tri, gam, bet, self.states, self.final, *frags)
+            box.saved = inter
             self.token = torch.zeros(1, device=dev)
 
     def outputs(self):
         return self.out, self.states, self.final, self.token
 
 
-_N_SAVED = 21  # tensors a group saves: q, k, v, g, beta, s0 and its 15 intermediates
+_N_SAVED = 10  # tensors a group saves: q, k, v, g, beta, s0 and work, frag, states, final
 
 
 class _GroupGrad:
@@ -112,14 +133,14 @@ class _GroupGrad:
     def __init__(self, saved_tensors, geom, box, dout, dstates, dfinal, needs_dq: bool):
         _in_use_here(dout, dstates, dfinal)
         chunk, offset, nch, has_q, has_s0, mfma = geom
-        (q, k, v, g, beta, s0f, kn, qn, w, u, delta, tri, gam, bet, states, final, *frags) = saved_tensors
+        q, k, v, g, beta, s0f, *inter = saved_tensors
+        qn = qcol = None
         self.box = box
         self.late = box is not None and box.dout is not None
         if self.late:  # the late read's gradient joins this backward as its read
-            q, qn, dout = box.q, box.qn, box.dout
-            frags[4] = box.qcol
+            q, qn, qcol, dout = box.q, box.qn, box.qcol, box.dout
             has_q = True
-            _in_use_here(q, qn, dout, box.qcol)
+            _in_use_here(q, qn, dout, qcol)
         bsz, tokens, heads, kd = k.shape
         vd = v.shape[-1]
         dev = k.device
@@ -131,11 +152,10 @@ class _GroupGrad:
         # dd0 and o: value-major on the FMA path, fragment order over whole
         # 32-column strips on the MFMA path (like u).
         vcols = -(-vd // 32) * 32 if mfma else vd
-        dd0 = torch.empty(rows * vcols, **f32) if want_read else None
-        obuf = torch.empty(rows * vcols, **f32) if want_read else None
-        ddelta = torch.empty(rows * vd, **f32)
-        dhend = torch.empty(bsz * heads * nch * kd * vd, **f32)
-        dw = torch.empty(rows * kd, **f32)
+        read = rows * vcols if want_read else 0
+        sizes = (read, read, rows * vd, -(-bsz * heads * nch * kd * vd // 64) * 64, rows * kd)
+        scratch = torch.empty(sum(sizes), **f32)
+        dd0, obuf, ddelta, dhend, dw = _pieces(scratch, 4, sizes)
         act = dict(device=dev, dtype=k.dtype)  # the kernels round dq, dk, dv to the activation type
         dq = torch.empty(bsz, tokens, heads, kd, **act) if has_q else None
         dk = torch.empty(bsz, tokens, heads, kd, **act)
@@ -146,9 +166,10 @@ class _GroupGrad:
         dstates = dstates.float().contiguous() if dstates is not None else None
         dfinal = dfinal.float().contiguous() if dfinal is not None else None
         self.prob = _problem(q, k, v, g, beta, s0f, chunk, offset)
-        self.saved = _lib.Saved(*(_ptr(t) for t in (kn, qn, w, u, delta, tri, gam, bet, states, final, *frags)))
+        # (the scan's own read, not a late one, has qn and qcol in its buffers)
+        self.saved = _saved(inter, _layout(rows, kd, vd, mfma, geom[3]), qn, qcol)
         self.grads = _lib.Grads(_lib.operand(dout if want_read else None), _ptr(dstates), _ptr(dfinal),
-                                _ptr(dd0), _ptr(obuf), ddelta.data_ptr(), dhend.data_ptr(), dw.data_ptr(),
+                                dd0, obuf, ddelta, dhend, dw,
                                 _lib.operand(dq), _lib.operand(dk), _lib.operand(dv),
                                 _lib.operand(dg), _lib.operand(db), ds0.data_ptr())
         # Every buffer the library reads or writes stays referenced until the
@@ -156,7 +177,7 @@ class _GroupGrad:
         # does not return (ds0 without an initial state, dq of a late read) is
         # still written, and memory dropped early would be handed to the next
         # group's buffers of a packed call before the kernels run.
-        self.keep = (dout, dstates, dfinal, dd0, obuf, ddelta, dhend, dw, q, qn, frags[4], dq, ds0)
+        self.keep = (*saved_tensors, dout, dstates, dfinal, scratch, q, qn, qcol, dq, ds0)
         self.timing_args = (kd, vd, chunk, tokens * bsz * heads, k.dtype, want_read)
         self.inj = dstates is not None
         dq_out = dq if (has_q and not self.late and needs_dq) else None
@@ -313,8 +334,7 @@ class _GDNRead(torch.autograd.Function):
             raise ValueError("gdn_scan_deferred: the read of a scan can be taken once")
         k, v, g, beta, s0f, chunk, offset, nch = box.args
         inter = box.saved
-        kn, w, u, delta, tri, gam, bet, states, final, *frags = inter
-        _in_use_here(q, k, v, g, beta, s0f, kn, delta, gam, states, frags[3])
+        _in_use_here(q, k, v, g, beta, s0f, *inter[:3])
         bsz, tokens, heads, kd = k.shape
         vd = v.shape[-1]
         dev = k.device
@@ -323,9 +343,9 @@ class _GDNRead(torch.autograd.Function):
         qcol = torch.empty(chunks * ((kd + 31) // 32) * 4 * 64 * 8, device=dev, dtype=torch.bfloat16)
         out = torch.empty(bsz, tokens, heads, vd, device=dev, dtype=k.dtype)
         prob = _problem(q, k, v, g, beta, s0f, chunk, offset)
-        saved = _read_saved(inter, qn, qcol)
+        saved = _saved(inter, _layout(chunks * _lib.CHUNK_ROWS, kd, vd, True, False), qn, qcol)
         _lib.check(lib.gpa_gdn_read(prob, saved, _lib.operand(out), _lib.stream_handle(dev)), "gpa_gdn_read")
-        ctx.box, ctx.geom = box, (chunk, offset)
+        ctx.box, ctx.geom = box, (chunk, offset, nch)
         ctx.save_for_backward(q, qn, qcol, k, v, g, beta, s0f, *inter)
         box.args = box.saved = None
         return out
@@ -335,25 +355,18 @@ class _GDNRead(torch.autograd.Function):
         lib = _lib.load()
         box = ctx.box
         q, qn, qcol, k, v, g, beta, s0f, *inter = ctx.saved_tensors
-        chunk, offset = ctx.geom
+        chunk, offset, nch = ctx.geom
+        bsz, _, heads, kd = k.shape
+        rows = bsz * heads * nch * _lib.CHUNK_ROWS
         dout = dout.to(k.dtype).contiguous()
         dq = torch.empty(q.shape, device=q.device, dtype=torch.float32)
         prob = _problem(q, k, v, g, beta, s0f, chunk, offset)
-        saved = _read_saved(inter, qn, qcol)
+        saved = _saved(inter, _layout(rows, kd, v.shape[-1], True, False), qn, qcol)
         _lib.check(lib.gpa_gdn_read_backward(prob, saved, _lib.operand(dout), _lib.operand(dq),
                                              _lib.stream_handle(q.device)), "gpa_gdn_read_backward")
         # the scan's backward takes the read's gradient as its own read
         box.q, box.qn, box.qcol, box.dout = q, qn, qcol, dout
         return dq.to(q.dtype), torch.zeros(1, device=q.device), None
-
-
-def _read_saved(inter, qn, qcol):
-    """The scan's saved intermediates (kn, w, u, delta, tri, gam, bet,
-    states, final, wrow, wcol, krow, kcol, qcol) with the read's qn and qcol."""
-    kn, w, u, delta, tri, gam, bet, states, final, *frags = inter
-    frags = list(frags)
-    frags[4] = qcol
-    return _lib.Saved(*(_ptr(t) for t in (kn, qn, w, u, delta, tri, gam, bet, states, final, *frags)))
 
 
 def gdn_scan_hip(q: Tensor | None, k: Tensor, v: Tensor, g: Tensor, beta: Tensor, s0: Tensor | None,
