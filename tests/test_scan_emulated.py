@@ -9,7 +9,8 @@ when K is not a multiple of 4), the bfloat16 FMA path (K not a multiple of
 16) and the bfloat16 MFMA path above 128 keys (gdn_state_fwd_mfma / gdn_state_bwd_mfma at 256 keys, with K
 below and at the tile), with chunk offsets, ragged last chunks and tiny
 shapes.  Every global access of those kernels is checked against the exact
-extent of the buffer it addresses; the results are held to the GPU tests'
+extent of its allocation (a scan's float32 intermediates, fragments and backward
+scratch are one each); the results are held to the GPU tests'
 bar: relative L2 1e-4 in float32, 2e-2 in bfloat16.  The bfloat16 scans of
 at most 128 keys take the strip state kernels, which the host build does not
 emulate (their LDS loads are inline global_load_lds); the GPU tests cover
