@@ -64,8 +64,8 @@ def _layout(rows, kd, vd, mfma, read):
     tri, gam, bet) and bf16 fragments (wrow, wcol, krow, kcol, qcol; MFMA path
     only), layouts of include/gpa_hip.h.  Each kind is one allocation, cut here:
     a buffer of its own costs the host 3 us; the forward of 130 tokens, 16 heads
-    128 x 256, 62 -> 49 us.  U is value-major [S,N,V,64] on the FMA path, on the MFMA path in fragment order
-    over ceil(V/32) whole 32-column strips."""
+    128 x 256, 62 -> 49 us.  U is value-major [S,N,V,64] on the FMA path, on the
+    MFMA path in fragment order over ceil(V/32) whole 32-column strips."""
     f32 = (rows * kd, rows * kd if read else 0, 0 if mfma else rows * kd,
            rows * (-(-vd // 32) * 32 if mfma else vd), rows * vd, rows * _lib.CHUNK_ROWS, rows, rows)
     if not mfma:
