@@ -436,8 +436,8 @@ __global__ __launch_bounds__(QT) void quad_bwd(gpa_quad_problem p, gpa_quad_grad
 template <typename E>
 __global__ __launch_bounds__(QT) void quad_pack(const float* left, const float* right, E* wt, E* w, int D) {
   __shared__ float tile[32][33];
-  const int DP = qpad(D), NB = DP / 32, h = blockIdx.y >> 1, p = blockIdx.y & 1;
-  const int k0 = (int)(blockIdx.x / NB) * 32, n0 = (int)(blockIdx.x % NB) * 32, c = threadIdx.x % 32, r0 = threadIdx.x / 32;
+  const int DP = qpad(D), NB = DP / 32, h = blockIdx.y, p = blockIdx.x & 1, tb = blockIdx.x >> 1;
+  const int k0 = tb / NB * 32, n0 = tb % NB * 32, c = threadIdx.x % 32, r0 = threadIdx.x / 32;
   const float* src = (p ? right : left) + (int64_t)h * D * D;
 #pragma unroll
   for (int i = 0; i < 4; ++i) {
@@ -528,11 +528,11 @@ extern "C" int gpa_quad_features_backward(const gpa_quad_problem* problem, const
 extern "C" int gpa_quad_pack_weights(const float* left, const float* right, int32_t heads, int32_t dim, int32_t dtype,
                                      void* wt, void* w, hipStream_t stream) {
   using namespace gpa;
-  if (!left || !right || !wt || heads < 1 || heads > 32767 || dim < 1 || dim > GPA_QUAD_MAX_DIM)
-    return fail(GPA_HIP_EINVAL, "quad pack: left, right, wt required; heads 1..32767, dim 1..GPA_QUAD_MAX_DIM");
+  if (!left || !right || !wt || heads < 1 || heads > 65535 || dim < 1 || dim > GPA_QUAD_MAX_DIM)
+    return fail(GPA_HIP_EINVAL, "quad pack: left, right, wt required; heads 1..65535, dim 1..GPA_QUAD_MAX_DIM");
   if (dtype != GPA_DTYPE_F32 && dtype != GPA_DTYPE_BF16) return fail(GPA_HIP_EUNSUPPORTED, "quad pack: dtype");
   const int nb = qpad(dim) / 32;
-  const dim3 grid(nb * nb, 2 * heads);
+  const dim3 grid(2 * nb * nb, heads);
   if (dtype == GPA_DTYPE_BF16)
     hipLaunchKernelGGL((quad_pack<bf16_t>), grid, dim3(QT), 0, stream, left, right, static_cast<bf16_t*>(wt),
                        static_cast<bf16_t*>(w), dim);

@@ -23,6 +23,18 @@ def _pad(d: int) -> int:
     return -(-d // 32) * 32
 
 
+def _check_parameters(x: Tensor, left: Tensor, right: Tensor, gain: Tensor) -> None:
+    """The kernels address both matrices and the gain by x's [.., heads, dim]."""
+    heads, dim = x.shape[-2:]
+    for name, w in (("left", left), ("right", right)):
+        if tuple(w.shape) != (heads, dim, dim) or w.device != x.device:
+            raise _lib.HipBackendError(f"quadratic features: {name} must be [{heads}, {dim}, {dim}] on {x.device}, "
+                                       f"got {list(w.shape)} on {w.device}")
+    if gain.numel() != heads or gain.device != x.device:
+        raise _lib.HipBackendError(f"quadratic features: one gain per head ({heads}) on {x.device} needed, "
+                                   f"got {gain.numel()} on {gain.device}")
+
+
 def _weights(left: Tensor, right: Tensor, dtype: torch.dtype, backward: bool):
     """wt [H][2][DP][DP] (wt[h][p][n][k] = W_p[h][k][n]) and, for the backward, w
     [H][DP][2DP] (w[h][k][p*DP + n] = W_p[h][k][n]), zero-padded, in `dtype`."""
@@ -51,6 +63,7 @@ def _problem(x: Tensor, wt: Tensor, w: Tensor | None, gain: Tensor, out: Tensor 
 class _QuadFeatures(torch.autograd.Function):
     @staticmethod
     def forward(ctx, x, left, right, gain):
+        _check_parameters(x, left, right, gain)
         lib = _lib.load()
         wt, w = _weights(left, right, x.dtype, False)
         gain = gain.float().contiguous()

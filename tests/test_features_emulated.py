@@ -5,7 +5,8 @@ the oracle's restatement of the reference's map (oracle.reference
 gradients of x and of every parameter, float32 (1e-5 / 1e-4) and bfloat16
 (2e-2), for widths below, at and above one 32-column block (8, 32, 40, 128,
 256), partial row tiles and a zero row.  Every access of the kernels is
-bounds-checked here before they run on a GPU.
+bounds-checked here before they run on a GPU.  Parameters that do not fit x's
+heads, width or device are refused before any kernel runs.
 """
 import math
 
@@ -57,3 +58,25 @@ def test_quad_features_match_oracle(host, rows, heads, dim, dtype):
     tol = (1e-5, 1e-4) if dtype == torch.float32 else (2e-2, 3e-2)
     for i, (name, a, r) in enumerate(zip(("out", "dx", "dleft", "dright", "dgain"), got, want)):
         assert _rel(a, r) < tol[min(i, 1)], (name, _rel(a, r))
+
+
+@pytest.mark.parametrize("wrong", [dict(right=(1, 8, 8)), dict(left=(1, 8, 8)), dict(left=(1, 8, 8), right=(1, 8, 8)),
+                                   dict(right=(2, 8, 4)), dict(left=(2, 4, 8)), dict(right=(2, 64)),
+                                   dict(left=(3, 8, 8), right=(3, 8, 8)), dict(gain=(1,))], ids=str)
+def test_quad_features_refuse_parameters_of_other_shapes(host, wrong):
+    """The kernels address the matrices and the gain by x's heads and width:
+    parameters that hold fewer values would be read past their end."""
+    from gpa_amd import _lib
+    shapes = {**dict(left=(2, 8, 8), right=(2, 8, 8), gain=(2,)), **wrong}
+    x = torch.randn(5, 2, 8)
+    with pytest.raises(_lib.HipBackendError, match="quadratic features"):
+        features._QuadFeatures.apply(x, *(torch.randn(shapes[n]) for n in ("left", "right", "gain")))
+
+
+@pytest.mark.parametrize("name", ["left", "right", "gain"])
+def test_quad_features_refuse_parameters_on_another_device(host, name):
+    from gpa_amd import _lib
+    params = dict(left=torch.randn(2, 8, 8), right=torch.randn(2, 8, 8), gain=torch.randn(2))
+    params[name] = params[name].to("meta")
+    with pytest.raises(_lib.HipBackendError, match="quadratic features"):
+        features._QuadFeatures.apply(torch.randn(5, 2, 8), *params.values())

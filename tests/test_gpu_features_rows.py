@@ -16,3 +16,22 @@ pytestmark = pytest.mark.gpu
                                             ((97,), 1, 250), ((700,), 3, 64)])
 def test_quad_features_at_row_and_block_edges(lead, heads, dim, dtype):
     check(lead, heads, dim, dtype)
+
+
+def test_quad_features_of_many_heads():
+    """Heads up to the launch limit of 65535 (one workgroup row per head): the
+    weight layouts, which take two matrices per head, included.  Forward against
+    the oracle at test_gpu_features.py's float32 bound."""
+    from gpa_amd.module import QuadraticFeatures
+    from oracle import reference as ref
+    from tests.test_gpu_features import _rel
+    heads, dim = 65535, 2
+    torch.manual_seed(0)
+    many = QuadraticFeatures(1, dim)
+    many.left, many.right = (torch.nn.Parameter(torch.randn(heads, dim, dim)) for _ in range(2))
+    many.gain_raw = torch.nn.Parameter(torch.randn(heads))
+    x = torch.randn(3, heads, dim)
+    with torch.no_grad():
+        want = ref.quadratic_features(many, x)
+        got = many.cuda()(x.cuda())
+    assert _rel(got, want) < 1e-5
