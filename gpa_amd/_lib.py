@@ -12,7 +12,7 @@ import torch
 
 HERE = os.path.dirname(os.path.abspath(__file__))
 LIB_PATH = os.path.join(HERE, "libgpa_hip.so")
-ABI_VERSION = 32
+ABI_VERSION = 33
 DECODE_MAX_LEVELS = 4
 DECODE_MAX_EDGES = 12
 DECODE_MAX_WIDTH = 256
@@ -273,7 +273,8 @@ EXPORTS = {
     "gpa_quad_features_forward": ([ctypes.POINTER(QuadProblem), c_vp], ctypes.c_int),
     "gpa_quad_features_backward": ([ctypes.POINTER(QuadProblem), ctypes.POINTER(QuadGrads), c_vp], ctypes.c_int),
     "gpa_quad_pack_weights": ([c_vp, c_vp, c_i32, c_i32, c_i32, c_vp, c_vp, c_vp], ctypes.c_int),
-    "gpa_quad_weight_grads": ([ctypes.POINTER(QuadProblem), c_vp, c_vp, c_vp, c_vp, c_vp], ctypes.c_int),
+    "gpa_quad_grad_partials": ([ctypes.POINTER(QuadProblem)], c_i64),
+    "gpa_quad_weight_grads": ([ctypes.POINTER(QuadProblem), c_vp, c_vp, c_vp, c_vp, c_vp, c_vp], ctypes.c_int),
     "gpa_sum_many": ([c_vp, ctypes.POINTER(c_vp), c_i32, c_i64, c_i32, c_vp], ctypes.c_int),
 }
 

@@ -64,7 +64,10 @@ namespace gpa {
 // Up to four products C[h] = sum over the R rows r of A[h][r]^T B[h][r]
 // (float32 [heads][a_width][b_width], cleared first), rounded to bf16 values
 // when bf16: row r of head h of A sits at a + h * a_hs + r * a_rs (elements).
-// The bf16 path runs them as one MFMA launch (route_reader.hip).
+// The bf16 path runs them as one MFMA launch (route_reader.hip) over spans of the
+// rows.  The spans' tiles are added to C with float atomics, in any order, or, with
+// `partials` (tn_partials floats; 16-byte aligned bf16 operands), kept apart and
+// added in the order of the rows: a result that repeats.
 struct TnProduct {
   const void* a;
   int64_t a_rs, a_hs;
@@ -74,5 +77,7 @@ struct TnProduct {
   int b_width;
   float* c;
 };
-int launch_tn_products(const TnProduct* products, int n, int heads, int rows, bool bf16, hipStream_t stream);
+int launch_tn_products(const TnProduct* products, int n, int heads, int rows, bool bf16, hipStream_t stream,
+                       float* partials = nullptr);
+int64_t tn_partials(const TnProduct* products, int n, int heads, int rows);
 }  // namespace gpa

@@ -542,18 +542,39 @@ extern "C" int gpa_quad_pack_weights(const float* left, const float* right, int3
   return check_launch("gpa_quad_pack_weights");
 }
 
-extern "C" int gpa_quad_weight_grads(const gpa_quad_problem* problem, const void* u, const void* dab, float* dleft,
-                                     float* dright, hipStream_t stream) {
+namespace gpa {
+namespace {
+// dW_p[h] = sum over the rows of u^T da (p = 0), u^T db (p = 1).
+struct QuadProducts {
+  TnProduct p[2];
+  QuadProducts(const gpa_quad_problem& q, const void* u, const void* dab, float* dleft, float* dright) {
+    const int dp = qpad(q.dim);
+    const int64_t hs = (int64_t)q.rows * dp;
+    const bf16_t* b = static_cast<const bf16_t*>(dab);
+    p[0] = {u, dp, hs, dp, b, 2 * dp, 2 * hs, dp, dleft};
+    p[1] = {u, dp, hs, dp, b ? b + dp : b, 2 * dp, 2 * hs, dp, dright};
+  }
+};
+}  // namespace
+}  // namespace gpa
+
+extern "C" int64_t gpa_quad_grad_partials(const gpa_quad_problem* problem) {
+  using namespace gpa;
+  if (check_quad(problem)) return -1;
+  const QuadProducts q(*problem, nullptr, nullptr, nullptr, nullptr);
+  return tn_partials(q.p, 2, problem->heads, problem->rows);
+}
+
+extern "C" int gpa_quad_weight_grads(const gpa_quad_problem* problem, const void* u, const void* dab, float* partials,
+                                     float* dleft, float* dright, hipStream_t stream) {
   using namespace gpa;
   if (int rc = check_quad(problem)) return rc;
-  const gpa_quad_problem& p = *problem;
-  if (p.dtype != GPA_DTYPE_BF16) return fail(GPA_HIP_EUNSUPPORTED, "quad weight grads: bf16 only");
-  if (!u || !dab || !dleft || !dright) return fail(GPA_HIP_EINVAL, "quad weight grads: u, dab, dleft and dright required");
-  const int dp = qpad(p.dim);
-  const int64_t hs = (int64_t)p.rows * dp;
-  const bf16_t* b = static_cast<const bf16_t*>(dab);
-  const TnProduct products[2] = {{u, dp, hs, dp, b, 2 * dp, 2 * hs, dp, dleft},
-                                 {u, dp, hs, dp, b + dp, 2 * dp, 2 * hs, dp, dright}};
-  if (int rc = launch_tn_products(products, 2, p.heads, p.rows, true, stream)) return rc;
+  if (problem->dtype != GPA_DTYPE_BF16) return fail(GPA_HIP_EUNSUPPORTED, "quad weight grads: bf16 only");
+  if (!u || !dab || !partials || !dleft || !dright)
+    return fail(GPA_HIP_EINVAL, "quad weight grads: u, dab, partials, dleft and dright required");
+  for (const void* x : {u, dab, (const void*)partials, (const void*)dleft, (const void*)dright})
+    if (reinterpret_cast<uintptr_t>(x) % 16) return fail(GPA_HIP_EINVAL, "quad weight grads: buffers on 16-byte boundaries");
+  const QuadProducts q(*problem, u, dab, dleft, dright);
+  if (int rc = launch_tn_products(q.p, 2, problem->heads, problem->rows, true, stream, partials)) return rc;
   return check_launch("gpa_quad_weight_grads");
 }

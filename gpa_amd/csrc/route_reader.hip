@@ -2027,7 +2027,8 @@ __global__ void round_in_place(float* c, int64_t n) {
 // that LDS holds [column][token] and each MFMA operand is one 16-byte read.
 // With a 72-element pitch and lanes ordered row block first, the writes and
 // the reads both touch 16 distinct 4-bank groups per 16 lanes.  Partial tiles
-// of the spans are added into C (cleared first) with float atomics.
+// of the spans are added into C (cleared first) with float atomics, or (PART) stored
+// in a copy of C per span.
 constexpr int GT = 128;         // output tile
 constexpr int GK = 64;          // rows per slab
 constexpr int GP = GK + 8;      // LDS pitch (bf16)
@@ -2043,9 +2044,10 @@ struct WJob {
 struct WJobs {
   WJob j0, j1, j2, j3;
   int span, R, tiles, heads, n;  // tiles of all four products, workgroups
+  int64_t span_elems;            // elements of all four products (PART: from one span's C to the next)
 };
 
-
+template <bool PART>
 __global__ __launch_bounds__(GNT, 4) void route_wgrad16(WJobs js) {
   HIP_DYNAMIC_SHARED(uint16_t, glds)
   const int logical = xcd_logical(blockIdx.x, js.n);
@@ -2133,7 +2135,7 @@ __global__ __launch_bounds__(GNT, 4) void route_wgrad16(WJobs js) {
     }
     __syncthreads();
   }
-  float* c = J.c + (int64_t)h * J.a.width * J.b.width;
+  float* c = J.c + (PART ? span_idx * js.span_elems : 0) + (int64_t)h * J.a.width * J.b.width;
 #pragma unroll
   for (int u = 0; u < 2; ++u)
 #pragma unroll
@@ -2141,7 +2143,11 @@ __global__ __launch_bounds__(GNT, 4) void route_wgrad16(WJobs js) {
 #pragma unroll
       for (int r = 0; r < 16; ++r) {
         const int i = i0 + wi + 32 * u + acc_row(r, lane >> 5), j = j0 + wj + 32 * v + fr;
-        if (i < J.a.width && j < J.b.width) atomicAdd(&c[(int64_t)i * J.b.width + j], acc[u][v][r]);
+        if (i < J.a.width && j < J.b.width) {
+          float* at = &c[(int64_t)i * J.b.width + j];
+          if (PART) *at = acc[u][v][r];
+          else atomicAdd(at, acc[u][v][r]);
+        }
       }
 }
 
@@ -2155,6 +2161,34 @@ __global__ void fill_or_round4(FourBufs b) {
 #pragma unroll
   for (int q = 0; q < 4; ++q)
     for (int64_t i = first; i < b.n[q]; i += step) b.c[q][i] = ROUND ? round_as<bf16_t>(b.c[q][i]) : 0.f;
+}
+
+// C = the spans' copies added in the order of the spans, rounded to bf16 values.
+// (Every product's elements are a multiple of 64: widths are multiples of 8.)
+// Bound: the copies' bytes, from the Infinity Cache where they fit.
+__global__ __launch_bounds__(256) void sum_spans4(FourBufs b, const float* part, int spans, int64_t span_elems) {
+  const int64_t step = 4 * (int64_t)gridDim.x * blockDim.x, first = 4 * ((int64_t)blockIdx.x * blockDim.x + threadIdx.x);
+#pragma unroll
+  for (int q = 0; q < 4; ++q) {
+    for (int64_t i = first; i < b.n[q]; i += step) {
+      f32x4 sum = {0.f, 0.f, 0.f, 0.f};
+      const float* src = part + i;
+      for (int s0 = 0; s0 < spans; s0 += 8) {  // eight loads in flight
+        f32x4 x[8];
+#pragma unroll
+        for (int s = 0; s < 8; ++s)
+          x[s] = *reinterpret_cast<const f32x4*>(src + (s0 + s < spans ? s0 + s : s0) * span_elems);
+#pragma unroll
+        for (int s = 0; s < 8; ++s)
+          if (s0 + s < spans) sum += x[s];
+      }
+      f32x4 r;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) r[e] = round_as<bf16_t>(sum[e]);
+      *reinterpret_cast<f32x4*>(b.c[q] + i) = r;
+    }
+    part += b.n[q];
+  }
 }
 
 // 16-byte loads need 8-element aligned columns, strides and base.
@@ -2468,7 +2502,27 @@ extern "C" int gpa_route_backward(const gpa_route_problem* problem, const gpa_ro
 }
 
 namespace gpa {
-int launch_tn_products(const TnProduct* products, int np, int H, int R, bool bf, hipStream_t stream) {
+// Row spans: enough workgroups for the whole chip, each span whole slabs.
+static int tn_spans(int tiles, int H, int R, int& span) {
+  const int slabs = (R + GK - 1) / GK, per_span_wgs = tiles * H;
+  int spans = (G_WGS + per_span_wgs - 1) / per_span_wgs;
+  spans = spans < 1 ? 1 : spans > slabs ? slabs : spans;
+  span = GK * ((slabs + spans - 1) / spans);
+  return (R + span - 1) / span;
+}
+static int tn_tiles(const TnProduct& p) { return ((p.a_width + GT - 1) / GT) * ((p.b_width + GT - 1) / GT); }
+
+int64_t tn_partials(const TnProduct* products, int np, int H, int R) {
+  int tiles = 0, span;
+  int64_t elems = 0;
+  for (int q = 0; q < np; ++q) {
+    tiles += tn_tiles(products[q]);
+    elems += (int64_t)H * products[q].a_width * products[q].b_width;
+  }
+  return tn_spans(tiles, H, R, span) * elems;
+}
+
+int launch_tn_products(const TnProduct* products, int np, int H, int R, bool bf, hipStream_t stream, float* partials) {
   if (np < 1 || np > 4) return fail(GPA_HIP_EINVAL, "tn products: 1 to 4 products");
   struct Job {
     TnOperand a, b;
@@ -2483,27 +2537,28 @@ int launch_tn_products(const TnProduct* products, int np, int H, int R, bool bf,
   if (fast) {
     WJob w[4] = {};  // unused products have no tiles
     FourBufs fb = {};
-    int tiles = 0;
+    int tiles = 0, span;
+    int64_t total = 0;
     for (int q = 0; q < np; ++q) {
-      const int ti = (jobs[q].a.width + GT - 1) / GT, tj = (jobs[q].b.width + GT - 1) / GT;
-      w[q] = {jobs[q].a, jobs[q].b, jobs[q].c, tj, ti * tj};
+      w[q] = {jobs[q].a, jobs[q].b, partials ? partials + total : jobs[q].c, (jobs[q].b.width + GT - 1) / GT,
+              tn_tiles(products[q])};
       fb.c[q] = jobs[q].c;
       fb.n[q] = (int64_t)H * jobs[q].a.width * jobs[q].b.width;
-      tiles += ti * tj;
+      tiles += w[q].tiles;
+      total += fb.n[q];
     }
-    // Row spans: enough workgroups for the whole chip, each span whole slabs.
-    const int slabs = (R + GK - 1) / GK, per_span_wgs = tiles * H;
-    int spans = (G_WGS + per_span_wgs - 1) / per_span_wgs;
-    spans = spans < 1 ? 1 : spans > slabs ? slabs : spans;
-    const int span = GK * ((slabs + spans - 1) / spans);
-    spans = (R + span - 1) / span;
-    const int n = tiles * H * spans;
-    const WJobs js{w[0], w[1], w[2], w[3], span, R, tiles, H, n};
-    if (int rc = set_lds(route_wgrad16, G_LDS)) return rc;
-    const int64_t total = fb.n[0] + fb.n[1] + fb.n[2] + fb.n[3];
+    const int spans = tn_spans(tiles, H, R, span), n = tiles * H * spans;
+    const WJobs js{w[0], w[1], w[2], w[3], span, R, tiles, H, n, total};
     const dim3 fgrid((unsigned)((total + 1023) / 1024 < 2048 ? (total + 1023) / 1024 : 2048));
+    if (partials) {
+      if (int rc = set_lds(route_wgrad16<true>, G_LDS)) return rc;
+      hipLaunchKernelGGL(route_wgrad16<true>, dim3(n), dim3(GNT), G_LDS, stream, js);
+      hipLaunchKernelGGL(sum_spans4, fgrid, dim3(256), 0, stream, fb, partials, spans, total);
+      return GPA_HIP_OK;
+    }
+    if (int rc = set_lds(route_wgrad16<false>, G_LDS)) return rc;
     hipLaunchKernelGGL(fill_or_round4<false>, fgrid, dim3(256), 0, stream, fb);
-    hipLaunchKernelGGL(route_wgrad16, dim3(n), dim3(GNT), G_LDS, stream, js);
+    hipLaunchKernelGGL(route_wgrad16<false>, dim3(n), dim3(GNT), G_LDS, stream, js);
     hipLaunchKernelGGL(fill_or_round4<true>, fgrid, dim3(256), 0, stream, fb);
     return GPA_HIP_OK;
   }

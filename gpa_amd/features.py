@@ -91,9 +91,11 @@ class _QuadFeatures(torch.autograd.Function):
                    "gpa_quad_features_backward")
         # dW_p = u^T d(u W_p), in the activation type
         if x.dtype == torch.bfloat16:
-            dleft, dright = (torch.empty(heads, dp, dp, device=x.device, dtype=torch.float32) for _ in range(2))
-            _lib.check(lib.gpa_quad_weight_grads(prob, u.data_ptr(), dab.data_ptr(), dleft.data_ptr(),
-                                                 dright.data_ptr(), _lib.stream_handle(x.device)),
+            f32 = dict(device=x.device, dtype=torch.float32)
+            partials = torch.empty(lib.gpa_quad_grad_partials(prob), **f32)
+            dleft, dright = (torch.empty(heads, dp, dp, **f32) for _ in range(2))
+            _lib.check(lib.gpa_quad_weight_grads(prob, u.data_ptr(), dab.data_ptr(), partials.data_ptr(),
+                                                 dleft.data_ptr(), dright.data_ptr(), _lib.stream_handle(x.device)),
                        "gpa_quad_weight_grads")
             dleft, dright = dleft[:, :dim, :dim], dright[:, :dim, :dim]
         else:

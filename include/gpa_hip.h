@@ -46,7 +46,7 @@
 extern "C" {
 #endif
 
-#define GPA_HIP_ABI_VERSION 32
+#define GPA_HIP_ABI_VERSION 33
 #define GPA_CHUNK_ROWS 64   /* rows per stored chunk; chunk <= 64 */
 #define GPA_MAX_KDIM 256    /* key width of a scan (the reduced dimension) */
 #define GPA_MAX_VDIM 1024   /* value width of a scan */
@@ -722,7 +722,10 @@ int gpa_moment_scan_many(const gpa_moment_problem *problems, int32_t n, hipStrea
  * gpa_quad_pack_weights makes the two weight copies from contiguous float32
  * parameters [heads][dim][dim] (w may be NULL: forward only).
  * gpa_quad_weight_grads (bf16) forms both weight gradients from the backward's
- * u and d(a)|d(b): float32 [heads][DP][DP], sums rounded to bf16. */
+ * u and d(a)|d(b): float32 [heads][DP][DP], sums rounded to bf16.  Spans of the rows
+ * are summed apart in `partials`, gpa_quad_grad_partials(problem) floats (-1 for a
+ * problem that no entry point takes), then in the order of the rows: equal calls give
+ * equal bits.  Its buffers start on 16-byte boundaries. */
 #define GPA_QUAD_MAX_DIM 256
 
 typedef struct gpa_quad_problem {
@@ -744,8 +747,9 @@ int gpa_quad_features_forward(const gpa_quad_problem *problem, hipStream_t strea
 int gpa_quad_features_backward(const gpa_quad_problem *problem, const gpa_quad_grads *grads, hipStream_t stream);
 int gpa_quad_pack_weights(const float *left, const float *right, int32_t heads, int32_t dim, int32_t dtype, void *wt,
                           void *w, hipStream_t stream);
-int gpa_quad_weight_grads(const gpa_quad_problem *problem, const void *u, const void *dab, float *dleft, float *dright,
-                          hipStream_t stream);
+int64_t gpa_quad_grad_partials(const gpa_quad_problem *problem);
+int gpa_quad_weight_grads(const gpa_quad_problem *problem, const void *u, const void *dab, float *partials, float *dleft,
+                          float *dright, hipStream_t stream);
 
 /* dst = src[0] + ... + src[n-1] elementwise over `count` elements of dtype,
  * accumulated in float32 and rounded once; 1 <= n <= GPA_SUM_MAX, every

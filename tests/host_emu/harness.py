@@ -32,7 +32,7 @@ ENTRIES = {"gpa_decode_step": 0, "gpa_route_forward": 1, "gpa_route_backward": 2
            "gpa_quad_features_forward": 16, "gpa_quad_features_backward": 17, "gpa_gdn_forward": 18,
            "gpa_gdn_backward": 19, "gpa_gdn_forward_many": 20, "gpa_gdn_backward_many": 21,
            "gpa_gdn_nchunks": 22, "gpa_gdn_path": 23,
-           "gpa_quad_pack_weights": 24, "gpa_quad_weight_grads": 25}
+           "gpa_quad_pack_weights": 24, "gpa_quad_weight_grads": 25, "gpa_quad_grad_partials": 26}
 SOURCES = ["gpa_decode.hip", "route_reader.hip", "level_mix.hip", "gdn_token.hip", "level_token.hip",
            "product_read.hip", "slot_gates.hip", "moment_scan.hip",
            "quad_features.hip", "gdn_scan.hip", "gdn_prep_mfma.hip", "gdn_state_mfma.hip", "gdn_out_mfma.hip",
@@ -238,8 +238,11 @@ class HostLib:
     def gpa_quad_pack_weights(self, left, right, heads, dim, dtype, wt, w, stream):
         return self._call("gpa_quad_pack_weights", [(ctypes.c_int32 * 3)(heads, dim, dtype)], [left, right, wt, w])
 
-    def gpa_quad_weight_grads(self, prob, u, dab, dleft, dright, stream):
-        return self._call("gpa_quad_weight_grads", [prob], [u, dab, dleft, dright])
+    def gpa_quad_grad_partials(self, prob):
+        return self._call("gpa_quad_grad_partials", [prob])
+
+    def gpa_quad_weight_grads(self, prob, u, dab, partials, dleft, dright, stream):
+        return self._call("gpa_quad_weight_grads", [prob], [u, dab, partials, dleft, dright])
 
     def gpa_gdn_forward(self, prob, saved, out, timing, stream):
         assert not timing

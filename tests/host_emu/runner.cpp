@@ -178,7 +178,12 @@ int main(int argc, char** argv) {
     }
     case 25:
       rc = gpa_quad_weight_grads(reinterpret_cast<gpa_quad_problem*>(blobs.at(0).data()), raw.at(0), raw.at(1),
-                                 static_cast<float*>(raw.at(2)), static_cast<float*>(raw.at(3)), nullptr);
+                                 static_cast<float*>(raw.at(2)), static_cast<float*>(raw.at(3)),
+                                 static_cast<float*>(raw.at(4)), nullptr);
+      break;
+    case 26:
+      value = gpa_quad_grad_partials(reinterpret_cast<gpa_quad_problem*>(blobs.at(0).data()));
+      rc = 0;
       break;
     case 23:
       value = gpa_gdn_path(reinterpret_cast<gpa_gdn_problem*>(blobs.at(0).data()));

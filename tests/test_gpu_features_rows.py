@@ -18,6 +18,20 @@ def test_quad_features_at_row_and_block_edges(lead, heads, dim, dtype):
     check(lead, heads, dim, dtype)
 
 
+@pytest.mark.parametrize("rows,heads,dim", [(4097, 2, 128), (700, 3, 64), (9000, 1, 200), (30, 2, 40)])
+def test_weight_gradients_repeat(rows, heads, dim):
+    """The bf16 weight gradients add their row spans (1 to 256 of them here) in
+    a fixed order: equal calls give equal bits."""
+    from gpa_amd.module import QuadraticFeatures
+    torch.manual_seed(rows)
+    fm = QuadraticFeatures(heads, dim).cuda()
+    x = torch.randn(rows, heads, dim, device="cuda", dtype=torch.bfloat16, requires_grad=True)
+    w = torch.randn(rows, heads, dim, device="cuda", dtype=torch.bfloat16)
+    grads = [torch.autograd.grad(fm(x), (x, *fm.parameters()), w) for _ in range(6)]
+    for again in grads[1:]:
+        assert all(torch.equal(a, b) for a, b in zip(grads[0], again))
+
+
 def test_quad_features_of_many_heads():
     """Heads up to the launch limit of 65535 (one workgroup row per head): the
     weight layouts, which take two matrices per head, included.  Forward against
