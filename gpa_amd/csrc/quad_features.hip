@@ -38,7 +38,7 @@ template <typename E>
 struct QLayout {
   int DP, NB, ULD, DLD;
   E* u;         // [32][ULD] unit(x) rows, then the output rows (out, dx)
-  E* x;         // [32][ULD] raw rows, zeros past dim and past the last row
+  E* x;         // [32][ULD] raw rows, zeros past dim and past the last row (null: q_raw_in_lds)
   E* g;         // [32][ULD] dout rows, the same, in dab's place until dab is formed
   E* dab;       // [32][DLD] d(a) | d(b) rows
   float* nrm;   // [32] ||x||_eps = sqrt(sum x^2 + 1e-12)
@@ -50,10 +50,19 @@ struct QLayout {
   float* wsum;  // [4] per-wave partial of dc
 };
 
+// Whether the backward keeps the raw rows in LDS: not in float32 above 128 columns, where
+// they would leave one workgroup per compute unit instead of two up to 192 columns
+// (8192 rows x 16 heads, forward and backward: 130 columns 1161 us with them, 869 without,
+// 192 columns 1443 and 1206; 256 columns, one either way, 1826 and 1846); they are read
+// again there.
+template <typename E>
+__host__ __device__ constexpr bool q_raw_in_lds(int dim) { return sizeof(E) == 2 || dim <= 128; }
+
 template <typename E>
 __host__ __device__ inline size_t q_lds_bytes(int dim, bool backward) {
   const int DP = qpad(dim), ULD = DP + 16 / (int)sizeof(E), DLD = 2 * DP + 16 / (int)sizeof(E);
-  const size_t b = (size_t)QR * ULD * sizeof(E) * (backward ? 2 : 1) + (backward ? (size_t)QR * DLD * sizeof(E) : 0);
+  const int rows = backward && q_raw_in_lds<E>(dim) ? 2 : 1;
+  const size_t b = (size_t)QR * ULD * sizeof(E) * rows + (backward ? (size_t)QR * DLD * sizeof(E) : 0);
   return b + (5 * QR + 8 * QR + 4) * sizeof(float);
 }
 
@@ -67,10 +76,14 @@ __device__ QLayout<E> q_layout(char* smem, int dim, bool backward) {
   E* e = reinterpret_cast<E*>(smem);
   L.u = e;
   e += QR * L.ULD;
-  L.x = L.g = L.dab = e;
+  L.x = nullptr;
   if (backward) {
-    L.g = L.dab = L.x + QR * L.ULD;
-    e = L.dab + QR * L.DLD;
+    if (q_raw_in_lds<E>(dim)) {
+      L.x = e;
+      e += QR * L.ULD;
+    }
+    L.g = L.dab = e;
+    e += QR * L.DLD;
   }
   float* f = reinterpret_cast<float*>(e);
   L.nrm = f;
@@ -89,54 +102,76 @@ struct QPiece {
   static constexpr int N = 16 / sizeof(E);
   E v[N];
 };
-// Elements d .. of a row (zeros past dim), in one 16-byte load when VEC.
-template <typename E, bool VEC>
-__device__ __forceinline__ QPiece<E> q_load(const E* row, int d, int dim) {
+template <typename E>
+__device__ __forceinline__ QPiece<E> q_get(const E* src) {
+  const uint4 w = *reinterpret_cast<const uint4*>(src);
   QPiece<E> x;
-  if constexpr (VEC) {
-    const uint4 w = *reinterpret_cast<const uint4*>(row + (d < dim ? d : 0));
-    __builtin_memcpy(&x, &w, 16);
-  } else {
-#pragma unroll
-    for (int e = 0; e < QPiece<E>::N; ++e) x.v[e] = row[qmin(d + e, dim - 1)];
-  }
+  __builtin_memcpy(&x, &w, 16);
   return x;
 }
+__device__ __forceinline__ bool q_aligned(const void* p) { return reinterpret_cast<uintptr_t>(p) % 16 == 0; }
 template <typename E>
 __device__ __forceinline__ void q_put(E* dst, const QPiece<E>& x) {
   uint4 w;
   __builtin_memcpy(&w, &x, 16);
   *reinterpret_cast<uint4*>(dst) = w;
 }
-template <typename E, bool VEC>
-__device__ __forceinline__ void q_store(E* row, int d, int dim, const E* src) {
-  if constexpr (VEC) {
-    if (d < dim) *reinterpret_cast<uint4*>(row + d) = *reinterpret_cast<const uint4*>(src);
-  } else {
+// Rows r0 .. r0+31 of `src`, `stride` apart, to LDS (zero past dim and past the last
+// row), element-wise: a wave per row, a lane per element of 64, so that rows off
+// 16-byte boundaries are read in whole lines too (8192 x 16 rows of 250 bf16, forward and
+// backward: 651 us; 785 with each thread on its own pieces' elements).
+template <typename E>
+__device__ __forceinline__ void q_stage(const gpa_quad_problem& p, const E* src, int64_t stride, int r0,
+                                        const QLayout<E>& L, E* dst) {
+  const int w = threadIdx.x >> 6, l = threadIdx.x & 63, D = p.dim;
+  for (int c = l; c < L.DP; c += 64) {
+    E v[8];
 #pragma unroll
-    for (int e = 0; e < QPiece<E>::N; ++e)
-      if (d + e < dim) row[d + e] = src[e];
+    for (int i = 0; i < 8; ++i) v[i] = src[qmin(r0 + 8 * w + i, p.rows - 1) * stride + qmin(c, D - 1)];
+#pragma unroll
+    for (int i = 0; i < 8; ++i)
+      dst[(8 * w + i) * L.ULD + c] = r0 + 8 * w + i < p.rows && c < D ? v[i] : from_f32<E>(0.f);
   }
 }
 
 // Rows r0 .. r0+31 of head h: u into LDS (zero past dim and past the last row)
-// and, with ROWS, the raw rows and dout's, u also to `uo`; ||x|| and ||x||_eps per
-// row.  Thread t holds the 16-byte pieces t%8, t%8 + 8, ... of row t/8; every load is
-// issued before the first use.
-template <typename E, bool VEC, bool ROWS>
+// and, with ROWS, the raw rows (RAW) and dout's, u also to `uo`; ||x|| and ||x||_eps per
+// row.  Thread t holds the 16-byte pieces t%8, t%8 + 8, ... of row t/8, loaded as such
+// (VEC; every load is issued before the first use) or from the rows in LDS.
+template <typename E, bool VEC, bool ROWS, bool RAW>
 __device__ void q_rows(const gpa_quad_problem& p, const E* dout, E* uo, int h, int r0, QLayout<E>& L) {
   constexpr int N = QPiece<E>::N, PM = 256 / (8 * N);
   const int tid = threadIdx.x, row = tid / 8, part = tid % 8, D = p.dim;
   const bool live = r0 + row < p.rows;
   const int grow = live ? r0 + row : p.rows - 1;
-  const E* xr = reinterpret_cast<const E*>(p.x) + (int64_t)grow * p.row_stride + (int64_t)h * D;
-  QPiece<E> xv[PM], gv[ROWS ? PM : 1];
+  const E* xh = reinterpret_cast<const E*>(p.x) + (int64_t)h * D;
+  const E* gh = ROWS ? dout + (int64_t)h * D : nullptr;
+  const int64_t gs = (int64_t)p.heads * D;
+  constexpr bool PUT = VEC && ROWS;  // the pieces are not in LDS yet
+  QPiece<E> xv[PM], gv[PUT ? PM : 1];
+  if constexpr (VEC) {
 #pragma unroll
-  for (int i = 0; i < PM; ++i) xv[i] = q_load<E, VEC>(xr, (part + 8 * i) * N, D);
-  if constexpr (ROWS)
+    for (int i = 0; i < PM; ++i) {
+      const int d = (part + 8 * i) * N;
+      xv[i] = q_get(xh + grow * p.row_stride + (d < D ? d : 0));
+    }
+    if constexpr (ROWS)
 #pragma unroll
-    for (int i = 0; i < PM; ++i)
-      gv[i] = q_load<E, VEC>(dout + ((int64_t)grow * p.heads + h) * D, (part + 8 * i) * N, D);
+      for (int i = 0; i < PM; ++i) {
+        const int d = (part + 8 * i) * N;
+        gv[i] = q_get(gh + grow * gs + (d < D ? d : 0));
+      }
+  } else {
+    E* raw = RAW ? L.x : L.u;
+    q_stage(p, xh, p.row_stride, r0, L, raw);
+    if constexpr (ROWS) q_stage(p, gh, gs, r0, L, L.g);
+    lds_barrier();
+#pragma unroll
+    for (int i = 0; i < PM; ++i) {
+      const int d = (part + 8 * i) * N;
+      xv[i] = q_get(raw + row * L.ULD + (d < L.DP ? d : 0));
+    }
+  }
   float ss = 0.f;
 #pragma unroll
   for (int i = 0; i < PM; ++i)
@@ -144,7 +179,7 @@ __device__ void q_rows(const gpa_quad_problem& p, const E* dout, E* uo, int h, i
     for (int e = 0; e < N; ++e) {
       const bool ok = live && (part + 8 * i) * N + e < D;
       if (!ok) xv[i].v[e] = from_f32<E>(0.f);
-      if constexpr (ROWS)
+      if constexpr (PUT)
         if (!ok) gv[i].v[e] = from_f32<E>(0.f);
       const float x = to_f32(xv[i].v[e]);
       ss += x * x;
@@ -157,15 +192,18 @@ __device__ void q_rows(const gpa_quad_problem& p, const E* dout, E* uo, int h, i
   for (int i = 0; i < PM; ++i) {
     const int d = (part + 8 * i) * N;
     if (d >= L.DP) continue;
-    if constexpr (ROWS) {
-      q_put(L.x + row * L.ULD + d, xv[i]);
-      q_put(L.g + row * L.ULD + d, gv[i]);
-    }
+    if constexpr (PUT && RAW) q_put(L.x + row * L.ULD + d, xv[i]);
+    if constexpr (PUT) q_put(L.g + row * L.ULD + d, gv[i]);
 #pragma unroll
     for (int e = 0; e < N; ++e) xv[i].v[e] = from_f32<E>(to_f32(xv[i].v[e]) / den);
     q_put(L.u + row * L.ULD + d, xv[i]);
     if constexpr (ROWS)
-      if (live) q_store<E, VEC>(uo + ((int64_t)h * p.rows + r0 + row) * L.DP, d, L.DP, xv[i].v);
+      if (live) {  // (u has whole pieces whatever the width)
+        E* dst = uo + ((int64_t)h * p.rows + r0 + row) * L.DP + d;
+        if (VEC || q_aligned(uo)) q_put(dst, xv[i]);
+        else
+          for (int e = 0; e < N; ++e) dst[e] = xv[i].v[e];
+      }
   }
   if (part == 0) {
     L.nrm[row] = sqrtf(ss + 1e-12f);
@@ -174,15 +212,20 @@ __device__ void q_rows(const gpa_quad_problem& p, const E* dout, E* uo, int h, i
 }
 
 // Rows in LDS (from `src`, `ld` apart) to `width` elements of the live rows of
-// dst, `stride` apart.
-template <typename E, bool VEC>
+// dst, `stride` apart: in 16-byte pieces (vec) or, as in q_stage, element-wise.
+template <typename E>
 __device__ __forceinline__ void q_rows_out(const gpa_quad_problem& p, int r0, E* dst, int64_t stride, int width,
-                                           const E* src, int ld) {
-  constexpr int N = QPiece<E>::N;
-  const int row = threadIdx.x / 8;
-  if (r0 + row < p.rows)
-    for (int d = (threadIdx.x % 8) * N; d < width; d += 8 * N)
-      q_store<E, VEC>(dst + row * stride, d, width, src + row * ld + d);
+                                           const E* src, int ld, bool vec) {
+  if (vec) {
+    constexpr int N = QPiece<E>::N;
+    const int row = threadIdx.x / 8;
+    if (r0 + row < p.rows)
+      for (int d = (threadIdx.x % 8) * N; d < width; d += 8 * N) q_put(dst + row * stride + d, q_get(src + row * ld + d));
+  } else {
+    const int w = threadIdx.x >> 6, l = threadIdx.x & 63;
+    for (int row = 8 * w; row < 8 * w + 8 && r0 + row < p.rows; ++row)
+      for (int c = l; c < width; c += 64) dst[row * stride + c] = src[row * ld + c];
+  }
 }
 
 // A per-row array at a lane's accumulator rows.
@@ -270,7 +313,7 @@ __global__ __launch_bounds__(QT) void quad_fwd(gpa_quad_problem p) {
   extern __shared__ __align__(16) char smem[];
   const int h = blockIdx.y, r0 = blockIdx.x * QR, w = threadIdx.x >> 6, l = threadIdx.x & 63;
   QLayout<E> L = q_layout<E>(smem, p.dim, false);
-  q_rows<E, VEC, false>(p, nullptr, nullptr, h, r0, L);
+  q_rows<E, VEC, false, false>(p, nullptr, nullptr, h, r0, L);
   lds_barrier();
   const float c = p.gain[h];
   float z[QB][16];
@@ -294,8 +337,8 @@ __global__ __launch_bounds__(QT) void quad_fwd(gpa_quad_problem p) {
     for (int r = 0; r < 16; ++r) L.u[acc_row(r, l >> 5) * L.ULD + cb * 32 + (l & 31)] = from_f32<E>(z[bi][r] * f[r]);
   }
   lds_barrier();
-  q_rows_out<E, VEC>(p, r0, reinterpret_cast<E*>(p.out) + ((int64_t)r0 * p.heads + h) * p.dim, (int64_t)p.heads * p.dim,
-                     p.dim, L.u, L.ULD);
+  q_rows_out(p, r0, reinterpret_cast<E*>(p.out) + ((int64_t)r0 * p.heads + h) * p.dim, (int64_t)p.heads * p.dim, p.dim,
+             L.u, L.ULD, VEC);
 }
 
 template <typename E, bool VEC, int QB>
@@ -304,7 +347,8 @@ __global__ __launch_bounds__(QT) void quad_bwd(gpa_quad_problem p, gpa_quad_grad
   const int h = blockIdx.y, r0 = blockIdx.x * QR, w = threadIdx.x >> 6, l = threadIdx.x & 63, t = threadIdx.x;
   const int D = p.dim;
   QLayout<E> L = q_layout<E>(smem, D, true);
-  q_rows<E, VEC, true>(p, reinterpret_cast<const E*>(g.dout), reinterpret_cast<E*>(g.u), h, r0, L);
+  constexpr bool RAW = q_raw_in_lds<E>(128 * QB);
+  q_rows<E, VEC, true, RAW>(p, reinterpret_cast<const E*>(g.dout), reinterpret_cast<E*>(g.u), h, r0, L);
   lds_barrier();
   const float c = p.gain[h];
   float z[QB][16], av[QB][16], bv[QB][16], gv[QB][16];
@@ -367,8 +411,8 @@ __global__ __launch_bounds__(QT) void quad_bwd(gpa_quad_problem p, gpa_quad_grad
   if (l == 0) L.wsum[w] = dc;
   lds_barrier();
   if (t == 0) g.dgain[(int64_t)blockIdx.x * p.heads + h] = L.wsum[0] + L.wsum[1] + L.wsum[2] + L.wsum[3];
-  q_rows_out<E, VEC>(p, r0, reinterpret_cast<E*>(g.dab) + ((int64_t)h * p.rows + r0) * 2 * L.DP, 2 * L.DP, 2 * L.DP, L.dab,
-                     L.DLD);
+  q_rows_out(p, r0, reinterpret_cast<E*>(g.dab) + ((int64_t)h * p.rows + r0) * 2 * L.DP, 2 * L.DP, 2 * L.DP, L.dab, L.DLD,
+             VEC || q_aligned(g.dab));
   // du = dz + da L^T + db R^T: contraction over the 2 DP columns of [da | db];
   // the B operand of output column k is row k of w = [L | R] (contiguous).
   const E* wk = reinterpret_cast<const E*>(p.w);
@@ -399,9 +443,17 @@ __global__ __launch_bounds__(QT) void quad_bwd(gpa_quad_problem p, gpa_quad_grad
       }
     }
     float s3[16];
+    if constexpr (!RAW) {
+      const int col = cb * 32 + lr;
+      const E* xh = reinterpret_cast<const E*>(p.x) + (int64_t)h * D + qmin(col, D - 1);
+#pragma unroll
+      for (int r = 0; r < 16; ++r) av[bi][r] = to_f32(xh[qmin(r0 + acc_row(r, l >> 5), p.rows - 1) * p.row_stride]);
+#pragma unroll
+      for (int r = 0; r < 16; ++r) av[bi][r] = r0 + acc_row(r, l >> 5) < p.rows && col < D ? av[bi][r] : 0.f;
+    }
 #pragma unroll
     for (int r = 0; r < 16; ++r) {
-      av[bi][r] = to_f32(L.x[at(r, cb)]);
+      if constexpr (RAW) av[bi][r] = to_f32(L.x[at(r, cb)]);
       z[bi][r] = round_as<E>(z[bi][r] + round_as<E>(acc_l[r]) + round_as<E>(acc_r[r]));
       s3[r] = z[bi][r] * av[bi][r];
     }
@@ -425,8 +477,7 @@ __global__ __launch_bounds__(QT) void quad_bwd(gpa_quad_problem p, gpa_quad_grad
     for (int r = 0; r < 16; ++r) L.u[at(r, cb)] = from_f32<E>(z[bi][r] * ra[r] - av[bi][r] * rb[r]);
   }
   lds_barrier();
-  q_rows_out<E, VEC>(p, r0, reinterpret_cast<E*>(g.dx) + ((int64_t)r0 * p.heads + h) * D, (int64_t)p.heads * D, D, L.u,
-                     L.ULD);
+  q_rows_out(p, r0, reinterpret_cast<E*>(g.dx) + ((int64_t)r0 * p.heads + h) * D, (int64_t)p.heads * D, D, L.u, L.ULD, VEC);
 }
 
 // The two weight layouts from the float32 parameters [H][D][D], a 32 x 32 tile per

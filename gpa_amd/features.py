@@ -25,12 +25,12 @@ def _pad(d: int) -> int:
 
 def _check_parameters(x: Tensor, left: Tensor, right: Tensor, gain: Tensor) -> None:
     """The kernels address both matrices and the gain by x's [.., heads, dim]."""
-    heads, dim = x.shape[-2:]
+    heads, dim, device = x.shape[-2], x.shape[-1], x.device
     for name, w in (("left", left), ("right", right)):
-        if tuple(w.shape) != (heads, dim, dim) or w.device != x.device:
+        if w.shape != (heads, dim, dim) or w.device != device:
             raise _lib.HipBackendError(f"quadratic features: {name} must be [{heads}, {dim}, {dim}] on {x.device}, "
                                        f"got {list(w.shape)} on {w.device}")
-    if gain.numel() != heads or gain.device != x.device:
+    if gain.numel() != heads or gain.device != device:
         raise _lib.HipBackendError(f"quadratic features: one gain per head ({heads}) on {x.device} needed, "
                                    f"got {gain.numel()} on {gain.device}")
 
@@ -93,11 +93,11 @@ class _QuadFeatures(torch.autograd.Function):
         if x.dtype == torch.bfloat16:
             f32 = dict(device=x.device, dtype=torch.float32)
             partials = torch.empty(lib.gpa_quad_grad_partials(prob), **f32)
-            dleft, dright = (torch.empty(heads, dp, dp, **f32) for _ in range(2))
-            _lib.check(lib.gpa_quad_weight_grads(prob, u.data_ptr(), dab.data_ptr(), partials.data_ptr(),
-                                                 dleft.data_ptr(), dright.data_ptr(), _lib.stream_handle(x.device)),
+            dw = torch.empty(2, heads, dp, dp, **f32)
+            _lib.check(lib.gpa_quad_weight_grads(prob, u.data_ptr(), dab.data_ptr(), partials.data_ptr(), dw.data_ptr(),
+                                                 dw.data_ptr() + 4 * heads * dp * dp, _lib.stream_handle(x.device)),
                        "gpa_quad_weight_grads")
-            dleft, dright = dleft[:, :dim, :dim], dright[:, :dim, :dim]
+            dleft, dright = dw[0, :, :dim, :dim], dw[1, :, :dim, :dim]
         else:
             dw = torch.bmm(u.transpose(1, 2).contiguous(), dab)           # [H, DP, 2DP], contiguous operands
             dleft, dright = dw[:, :dim, :dim], dw[:, :dim, dp:dp + dim]
