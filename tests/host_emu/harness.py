@@ -32,13 +32,14 @@ ENTRIES = {"gpa_decode_step": 0, "gpa_route_forward": 1, "gpa_route_backward": 2
            "gpa_quad_features_forward": 16, "gpa_quad_features_backward": 17, "gpa_gdn_forward": 18,
            "gpa_gdn_backward": 19, "gpa_gdn_forward_many": 20, "gpa_gdn_backward_many": 21,
            "gpa_gdn_nchunks": 22, "gpa_gdn_path": 23,
-           "gpa_quad_pack_weights": 24, "gpa_quad_weight_grads": 25, "gpa_quad_grad_partials": 26}
+           "gpa_quad_pack_weights": 24, "gpa_quad_weight_grads": 25, "gpa_quad_grad_partials": 26,
+           "gpa_gdn_read": 27, "gpa_gdn_read_backward": 28}
 SOURCES = ["gpa_decode.hip", "route_reader.hip", "level_mix.hip", "gdn_token.hip", "level_token.hip",
            "product_read.hip", "slot_gates.hip", "moment_scan.hip",
            "quad_features.hip", "gdn_scan.hip", "gdn_prep_mfma.hip", "gdn_state_mfma.hip", "gdn_out_mfma.hip",
            "gdn_chunk_bwd_mfma.hip", "gdn_chunk_bwd_frag.hip"]
 # Test-side sources of the host build: stand-ins for kernels it does not emulate.
-HOST_SOURCES = ["strip_absent.cpp"]
+HOST_SOURCES = ["strip_reference.cpp"]
 
 
 def compiler() -> str | None:
@@ -260,6 +261,12 @@ class HostLib:
         assert not timing and n == len(probs) == len(saved) == len(grads)
         return self._call("gpa_gdn_backward_many", [probs, saved, grads])
 
+    def gpa_gdn_read(self, prob, saved, out, stream):
+        return self._call("gpa_gdn_read", [prob, saved, out])
+
+    def gpa_gdn_read_backward(self, prob, saved, dout, dq, stream):
+        return self._call("gpa_gdn_read_backward", [prob, saved, dout, dq])
+
     def gpa_gdn_nchunks(self, tokens, offset, chunk):
         return self._call("gpa_gdn_nchunks", [(ctypes.c_int32 * 3)(tokens, offset, chunk)])
 
@@ -277,3 +284,4 @@ def use_host(monkeypatch, host: HostLib) -> None:
     monkeypatch.setattr(_lib, "load", lambda: host)
     monkeypatch.setattr(_lib, "require_device", lambda t: None)
     monkeypatch.setattr(_lib, "stream_handle", lambda d: 0)
+

@@ -181,6 +181,17 @@ int main(int argc, char** argv) {
                                  static_cast<float*>(raw.at(2)), static_cast<float*>(raw.at(3)),
                                  static_cast<float*>(raw.at(4)), nullptr);
       break;
+    case 27:
+      rc = gpa_gdn_read(reinterpret_cast<gpa_gdn_problem*>(blobs.at(0).data()),
+                        reinterpret_cast<gpa_gdn_saved*>(blobs.at(1).data()),
+                        *reinterpret_cast<gpa_operand*>(blobs.at(2).data()), nullptr);
+      break;
+    case 28:
+      rc = gpa_gdn_read_backward(reinterpret_cast<gpa_gdn_problem*>(blobs.at(0).data()),
+                                 reinterpret_cast<gpa_gdn_saved*>(blobs.at(1).data()),
+                                 *reinterpret_cast<gpa_operand*>(blobs.at(2).data()),
+                                 *reinterpret_cast<gpa_operand*>(blobs.at(3).data()), nullptr);
+      break;
     case 26:
       value = gpa_quad_grad_partials(reinterpret_cast<gpa_quad_problem*>(blobs.at(0).data()));
       rc = 0;

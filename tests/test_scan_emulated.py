@@ -1,20 +1,21 @@
 """The chunked GDN scan's kernels (gdn_scan.hip and the prep, 256-key state,
-out / dd0 and chunk-backward MFMA kernels) built for the host and run under
+out / dd0, late-read and chunk-backward MFMA kernels) built for the host and run under
 AddressSanitizer (tests/host_emu/), against the oracle's per-token
 recurrence in float64 (reference ops.py:29-85), on the CPU.
 
 The cases reach the float32 FMA path (state, out and dd0 kernels of
 gdn_scan.hip, the chunk backward on fp32 MFMA, or the FMA chunk backward
 when K is not a multiple of 4), the bfloat16 FMA path (K not a multiple of
-16) and the bfloat16 MFMA path above 128 keys (gdn_state_fwd_mfma / gdn_state_bwd_mfma at 256 keys, with K
-below and at the tile), with chunk offsets, ragged last chunks and tiny
-shapes.  Every global access of those kernels is checked against the exact
-extent of its allocation (a scan's float32 intermediates, fragments and backward
-scratch are one each); the results are held to the GPU tests'
-bar: relative L2 1e-4 in float32, 2e-2 in bfloat16.  The bfloat16 scans of
-at most 128 keys take the strip state kernels, which the host build does not
-emulate (their LDS loads are inline global_load_lds); the GPU tests cover
-them.
+16) and the bfloat16 MFMA path in each key-width class (64, 128 and 256, with
+K below and at the tile; widths, and rows off 16-byte boundaries, that take the
+element-wise loads of the preparation and leave the fragment chunk backward),
+with chunk offsets, ragged last chunks and tiny shapes.  Every global access of
+those kernels is checked against the exact extent of its allocation (a scan's
+float32 intermediates, fragments and backward scratch are one each), and new
+memory is NaN; the results are held to the GPU tests' bar: relative L2 1e-4 in float32, 2e-2 in bfloat16.  The strip state kernels that
+bfloat16 scans of at most 128 keys take are not emulated (their LDS loads are
+inline global_load_lds): a plain recurrence stands in for them
+(host_emu/strip_reference.cpp), and the GPU tests cover them.
 """
 import pytest
 import torch
@@ -33,6 +34,11 @@ CASES = [
     (1, 40, 1, 128, 64, 16, 3, torch.float32),
     (1, 129, 1, 256, 96, 64, 1, torch.bfloat16),
     (1, 70, 1, 192, 128, 64, 5, torch.bfloat16),
+    (1, 9, 1, 16, 8, 8, 3, torch.bfloat16),
+    (1, 70, 1, 48, 20, 64, 5, torch.bfloat16),  # V % 8 != 0: element-wise rows, the general chunk backward
+    (1, 70, 2, 64, 40, 64, 17, torch.bfloat16),
+    (1, 40, 1, 80, 96, 16, 3, torch.bfloat16),
+    (1, 129, 1, 128, 64, 64, 1, torch.bfloat16),
 ]
 IDS = [f"B{c[0]}T{c[1]}H{c[2]}K{c[3]}V{c[4]}C{c[5]}o{c[6]}{str(c[7])[6:]}" for c in CASES]
 
@@ -43,6 +49,10 @@ def host(host_runner, monkeypatch, tmp_path):
     harness.use_host(monkeypatch, harness.HostLib(host_runner, str(tmp_path)))
     # host tensors belong to no stream: nothing to mark as in use
     monkeypatch.setattr(ops, "_in_use_here", lambda *tensors: None)
+    was = torch.are_deterministic_algorithms_enabled(), torch.is_deterministic_algorithms_warn_only_enabled()
+    torch.use_deterministic_algorithms(True, warn_only=True)  # new tensors start as NaN
+    yield
+    torch.use_deterministic_algorithms(was[0], warn_only=was[1])
 
 
 @pytest.mark.parametrize("case", CASES, ids=IDS)
@@ -90,3 +100,44 @@ def test_emulated_scan_backward_matches_autograd_of_recurrence(host, case, with_
     errs = {n: _rel(a.grad, r.grad) for n, a, r in zip(names, leaves, refs) if a is not None}
     print(case, with_q, errs)
     assert all(e < tol for e in errs.values()), errs
+
+
+def _off_boundary(x):
+    """The same values in rows that start 2 bytes past a 16-byte boundary."""
+    wide = torch.zeros(*x.shape[:-1], x.shape[-1] + 9, dtype=x.dtype)
+    wide[..., 1:x.shape[-1] + 1] = x
+    return wide[..., 1:x.shape[-1] + 1]
+
+
+@pytest.mark.parametrize("kd,vd", [(64, 24), (128, 64)])
+def test_emulated_rows_off_boundaries_give_the_same(host, kd, vd):
+    """Element-wise loads of the preparation against its 16-byte loads."""
+    from gpa_amd.ops import gdn_scan_hip
+    q, k, v, g, beta, s0 = _inputs(1, 70, 1, kd, vd, torch.bfloat16, seed=9)
+    want = gdn_scan_hip(q, k, v, g, beta, s0, chunk=64, offset=5)
+    got = gdn_scan_hip(*(_off_boundary(x) for x in (q, k, v)), g, beta, s0, chunk=64, offset=5)
+    assert all(torch.equal(a, b) for a, b in zip(got, want))
+
+
+@pytest.mark.parametrize("kd,vd", [(48, 24), (128, 40), (144, 32)])
+def test_emulated_late_read_matches_the_scan_with_its_read(host, kd, vd):
+    """A read taken after its scan (gpa_gdn_read, gpa_gdn_read_backward, and the
+    scan backward that takes the read's gradient): keys that end inside a 32-key
+    tile leave padding in the query fragments that the chunk backward multiplies."""
+    from gpa_amd.ops import gdn_scan_deferred, gdn_scan_hip
+    inputs = _inputs(1, 21, 1, kd, vd, torch.bfloat16, seed=5)
+    gen = torch.Generator()
+    res = []
+    for late in (False, True):
+        leaves = [x.clone().requires_grad_() for x in inputs]
+        q, rest = leaves[0], leaves[1:]
+        if late:
+            states, final, read = gdn_scan_deferred(*rest, chunk=64, offset=3)
+            out = read(q)
+        else:
+            out, states, final = gdn_scan_hip(q, *rest, chunk=64, offset=3)
+        w = [torch.randn(x.shape, generator=gen.manual_seed(3)).to(x.dtype) for x in (out, states, final)]
+        res.append((out, *torch.autograd.grad((out, states, final), leaves, w)))
+    errs = [_rel(a, b) for a, b in zip(res[1], res[0])]
+    print(kd, errs)
+    assert all(e < 2e-2 for e in errs), errs  # (a NaN fails)
