@@ -112,7 +112,8 @@ def kernel_timer():
 
 def _prep(k, v, c, tokens, dtype):
     e, km = _tag(dtype), _kmax(k)
-    return (f"gdn_prep_frag<{km},true>" if _mfma(k, dtype) else f"gdn_prep_mfma<{e},{km}>",
+    vec = "true" if v % 8 == 0 else "false"  # (16-byte aligned rows, as the module's are)
+    return (f"gdn_prep_frag<{km},{vec}>" if _mfma(k, dtype) else f"gdn_prep_mfma<{e},{km}>",
             (4 * c * k + 2 * c * v + c * c / 3) * tokens)
 
 
@@ -132,7 +133,7 @@ def _state_bwd_name(k, dtype) -> str:
     km = _kmax(k)
     if _mfma(k, dtype):
         return f"gdn_state_bwd_strip<{km}>" if km <= 128 else f"gdn_state_bwd_mfma<{km}>"
-    return f"gdn_state_bwd<{_tag(dtype)},{km}>"
+    return f"gdn_state_bwd<{km}>"
 
 
 def _out(k, v, c, tokens, dtype):
@@ -152,7 +153,7 @@ def _chunk_bwd(k, v, c, tokens, dtype, read):
     flop = 4 * k * v + 4 * c * v + 4 * c * k + 2 * c * c
     if read:
         flop += 2 * k * v + 2 * c * v + 6 * c * k
-    if _mfma(k, dtype) and v % 8 == 0:  # (16-byte aligned rows, as the module's are)
+    if _mfma(k, dtype) and v % 8 == 0:  # (aligned rows)
         return f"gdn_chunk_bwd_frag<{km},{'true' if read else 'false'}>", flop * tokens
     mfma_chunk = k % 4 == 0 and not (km == 256 and e == "f32")
     return f"{'gdn_chunk_bwd_mfma' if mfma_chunk else 'gdn_chunk_bwd'}<{e},{km}>", flop * tokens
@@ -313,10 +314,11 @@ def _ours(kernel: str) -> bool:
 
 def timer_name(kernel: str) -> str:
     """The name `kernel_timer` gives a kernel of a trace: the namespace and
-    spaces dropped, bf16_t written bf16, and the state recurrences grouped by
-    their key width alone (their other template flags select variants)."""
-    n = kernel.replace("gpa::", "").replace("bf16_t", "bf16").replace(" ", "")
-    if n.startswith("gdn_state_") and "<" in n:
+    spaces dropped, bf16_t written bf16 and float f32, and the state recurrences
+    and the MFMA dd0 kernel grouped by their key width alone (their other
+    template parameters select variants)."""
+    n = kernel.replace("gpa::", "").replace("bf16_t", "bf16").replace("float", "f32").replace(" ", "")
+    if n.startswith(("gdn_state_", "gdn_dd0_mfma")) and "<" in n:
         n = n.split(",")[0].rstrip(">") + ">"
     return n
 

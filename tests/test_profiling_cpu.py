@@ -3,6 +3,13 @@
 files whose answers are known, and the bench's reading of the committed
 traffic table."""
 import csv
+import os
+import re
+import shutil
+import subprocess
+
+import pytest
+import torch
 
 import bench
 from gpa_amd import profiling as pf
@@ -29,22 +36,56 @@ def test_timer_name_groups_state_kernels_by_key_width():
     assert pf.timer_name("gpa::gdn_state_fwd_mfma_pack<256, true>") == "gdn_state_fwd_mfma_pack<256>"
 
 
+def _library_kernels():
+    """The scan kernels that the built library holds, by their symbols' names."""
+    from gpa_amd import _lib
+    if not os.path.exists(_lib.LIB_PATH) or not shutil.which("nm"):
+        pytest.skip("needs libgpa_hip.so (python -m gpa_amd.build) and nm")
+    names = subprocess.run(["nm", "-C", _lib.LIB_PATH], capture_output=True, text=True, check=True).stdout
+    return {pf.timer_name(n) for n in re.findall(r"gpa::gdn_\w+<[^()]*>", names)}
+
+
+def test_timed_names_are_those_of_the_kernels_in_the_library():
+    """Event timings and traces are matched by name: every name that the timer
+    gives a launch is an instantiation that exists."""
+    kernels = _library_kernels()
+    for dtype in (torch.float32, torch.bfloat16):
+        for k in (2, 6, 16, 40, 64, 128, 130, 256):
+            for v in (8, 20, 256, 264):
+                rows = [pf._prep(k, v, 64, 1, dtype)[0], pf._state_fwd_name(k, dtype), pf._state_bwd_name(k, dtype),
+                        pf._out(k, v, 64, 1, dtype)[0], pf._dd0(k, v, 64, 1, dtype)[0],
+                        *(pf._chunk_bwd(k, v, 64, 1, dtype, read)[0] for read in (True, False))]
+                assert not [n for n in rows if n not in kernels], (dtype, k, v, rows)
+
+
+def test_timed_names_follow_the_widths():
+    bf, f32 = torch.bfloat16, torch.float32
+    assert pf._prep(128, 64, 64, 1, bf)[0] == pf.timer_name("gpa::gdn_prep_frag<128, true>")
+    assert pf._prep(128, 20, 64, 1, bf)[0] == pf.timer_name("gpa::gdn_prep_frag<128, false>")
+    assert pf._prep(40, 64, 64, 1, bf)[0] == pf.timer_name("gpa::gdn_prep_mfma<gpa::bf16_t, 64>")
+    assert pf._prep(40, 64, 64, 1, f32)[0] == pf.timer_name("gpa::gdn_prep_mfma<float, 64>")
+    assert pf._state_bwd_name(64, f32) == pf.timer_name("gpa::gdn_state_bwd<64, true>")
+    assert pf._state_fwd_name(250, bf) == pf.timer_name("gpa::gdn_state_fwd<256, false>")
+    assert pf._chunk_bwd(128, 64, 64, 1, bf, True)[0] == pf.timer_name("gpa::gdn_chunk_bwd_frag<128, true>")
+    assert pf._chunk_bwd(128, 20, 64, 1, bf, True)[0] == pf.timer_name("gpa::gdn_chunk_bwd_mfma<gpa::bf16_t, 128>")
+
+
 def test_traffic_scales_each_counter_by_the_copy_calibration(tmp_path):
     """A copy of 1 MiB whose FETCH_SIZE reads 512 KiB and WRITE_SIZE 1024 KiB
     gives factors 2 and 1; a kernel whose counters read 100,000 and 50,000
     KiB per dispatch (two dispatches) then moves 200,000 KiB read and 50,000
     KiB written per dispatch (204.8 and 51.2 MB)."""
     copy = "__amd_rocclr_copyBuffer"
-    kern = "void gpa::gdn_prep_mfma<gpa::bf16_t, 128, true>(gpa_gdn_problem, gpa_gdn_saved, int)"
+    kern = "void gpa::gdn_prep_frag<128, true>(gpa_gdn_problem, gpa_gdn_saved, int)"
     cf = _write(tmp_path / "cf.csv", [_row(0, copy, "FETCH_SIZE", 512.0)])
     cw = _write(tmp_path / "cw.csv", [_row(0, copy, "WRITE_SIZE", 1024.0)])
     f = _write(tmp_path / "f.csv", [_row(1, kern, "FETCH_SIZE", 1e5), _row(2, kern, "FETCH_SIZE", 1e5)])
     w = _write(tmp_path / "w.csv", [_row(1, kern, "WRITE_SIZE", 5e4), _row(2, kern, "WRITE_SIZE", 5e4)])
     text = pf.summarize_traffic(f, w, cf, cw, 1 << 20)
     assert "FETCH_SIZE x 2.000, WRITE_SIZE x 1.000" in text
-    row = next(line for line in text.splitlines() if "gdn_prep_mfma" in line)
+    row = next(line for line in text.splitlines() if "gdn_prep_frag" in line)
     cells = [c.strip() for c in row.strip("|").split("|")]
-    assert cells[0] == "`gdn_prep_mfma<bf16,128,true>`" and cells[1] == "2"
+    assert cells[0] == "`gdn_prep_frag<128,true>`" and cells[1] == "2"
     assert cells[2:] == ["100,000.0", "50,000.0", "204.8", "51.2"]
 
 
@@ -63,6 +104,6 @@ def test_stalls_are_shares_of_wave_cycles(tmp_path):
 def test_bench_reads_the_committed_traffic_table():
     """`roofline.traffic` of the dominant kernel comes from the committed PMC
     summary: read plus written MB per launch, in bytes."""
-    got = bench._measured_traffic("gdn_chunk_bwd_mfma<bf16,128>")
+    got = bench._measured_traffic("gdn_chunk_bwd_frag<128,true>")
     assert got is not None and 5e8 < got < 2e9
     assert bench._measured_traffic("no_such_kernel<1>") is None
