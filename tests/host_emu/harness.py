@@ -285,3 +285,22 @@ def use_host(monkeypatch, host: HostLib) -> None:
     monkeypatch.setattr(_lib, "require_device", lambda t: None)
     monkeypatch.setattr(_lib, "stream_handle", lambda d: 0)
 
+
+class SeparateBuffers:
+    """In place of `gpa_amd.ops._pieces`, which cuts a scan's buffers from one
+    allocation per kind: a tensor of exactly its size for each, so that the host
+    run bounds every access by the buffer it addresses.  They start as NaN: a
+    kernel that uses what none has written shows.  The cut allocations are kept,
+    and their addresses with them, so that a later call on one finds its buffers."""
+
+    def __init__(self):
+        self.made = {}
+
+    def __call__(self, base, width, sizes):
+        if base is None:
+            return [None] * len(sizes)
+        _, buffers = self.made.setdefault(base.data_ptr(), (base, [
+            torch.full((n,), float("nan"), dtype=torch.float32 if width == 4 else torch.bfloat16) if n else None
+            for n in sizes]))
+        assert [b.numel() if b is not None else 0 for b in buffers] == list(sizes)
+        return [b.data_ptr() if b is not None else None for b in buffers]

@@ -10,9 +10,10 @@ when K is not a multiple of 4), the bfloat16 FMA path (K not a multiple of
 K below and at the tile; widths, and rows off 16-byte boundaries, that take the
 element-wise loads of the preparation and leave the fragment chunk backward),
 with chunk offsets, ragged last chunks and tiny shapes.  Every global access of
-those kernels is checked against the exact extent of its allocation (a scan's
-float32 intermediates, fragments and backward scratch are one each), and new
-memory is NaN; the results are held to the GPU tests' bar: relative L2 1e-4 in float32, 2e-2 in bfloat16.  The strip state kernels that
+those kernels is checked against the exact extent of the buffer it addresses
+(each of a scan's intermediates, fragments and scratch buffers in a tensor of
+its own), and new memory is NaN; the results are held to the GPU tests' bar:
+relative L2 1e-4 in float32, 2e-2 in bfloat16.  The strip state kernels that
 bfloat16 scans of at most 128 keys take are not emulated (their LDS loads are
 inline global_load_lds): a plain recurrence stands in for them
 (host_emu/strip_reference.cpp), and the GPU tests cover them.
@@ -47,12 +48,33 @@ IDS = [f"B{c[0]}T{c[1]}H{c[2]}K{c[3]}V{c[4]}C{c[5]}o{c[6]}{str(c[7])[6:]}" for c
 def host(host_runner, monkeypatch, tmp_path):
     from gpa_amd import ops
     harness.use_host(monkeypatch, harness.HostLib(host_runner, str(tmp_path)))
+    monkeypatch.setattr(ops, "_pieces", harness.SeparateBuffers())
     # host tensors belong to no stream: nothing to mark as in use
     monkeypatch.setattr(ops, "_in_use_here", lambda *tensors: None)
     was = torch.are_deterministic_algorithms_enabled(), torch.is_deterministic_algorithms_warn_only_enabled()
     torch.use_deterministic_algorithms(True, warn_only=True)  # new tensors start as NaN
     yield
     torch.use_deterministic_algorithms(was[0], warn_only=was[1])
+
+
+def test_every_scan_buffer_is_an_allocation_of_its_size(host, monkeypatch):
+    """What the host run bounds: each intermediate and each scratch buffer ends
+    where its allocation does."""
+    from gpa_amd.ops import gdn_scan_hip
+    seen, locate = set(), harness.HostLib._locate
+
+    def check(self, spans, p):
+        i, at = locate(self, spans, p)
+        seen.add(spans[i][1])
+        assert at == 0, "a buffer inside another's allocation"
+        return i, at
+
+    monkeypatch.setattr(harness.HostLib, "_locate", check)
+    q, k, v, g, beta, s0 = (x.requires_grad_() for x in _inputs(1, 9, 1, 16, 8, torch.bfloat16, seed=1))
+    out, _, final = gdn_scan_hip(q, k, v, g, beta, s0, chunk=64, offset=0)
+    (out.float().sum() + final.sum()).backward()
+    # one chunk of one stream: float32 kn, delta, u (a whole strip) and T, bf16 w and k fragments
+    assert {64 * 16 * 4, 64 * 8 * 4, 64 * 32 * 4, 64 * 64 * 4, 2 * 64 * 16 * 2, 4 * 64 * 16 * 2} <= seen
 
 
 @pytest.mark.parametrize("case", CASES, ids=IDS)
