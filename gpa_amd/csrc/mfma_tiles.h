@@ -46,6 +46,20 @@ __device__ __forceinline__ f32x4 ld_x(const float* m, int ld, int x, int c0) {
   return f32x4{m[c0 * ld + x], m[(c0 + 1) * ld + x], m[(c0 + 2) * ld + x], m[(c0 + 3) * ld + x]};
 }
 
+// The operands of mma16 with the contraction indices in order: its MFMAs are chains of
+// fused multiply-adds over the quarters, so with index c0 + 4 s + l/16 in element s the
+// sum runs over c0, c0 + 1, ...  Where the terms of neighbouring indices cancel (the
+// delta rule's over positions, when keys are nearly parallel), any other order adds up
+// large partial sums first.
+__device__ __forceinline__ f32x4 ld_c_inorder(const float* m, int ld, int x, int c0, int q) {
+  const float* p = m + x * ld + c0 + q;
+  return f32x4{p[0], p[4], p[8], p[12]};
+}
+__device__ __forceinline__ f32x4 ld_x_inorder(const float* m, int ld, int x, int c0, int q) {
+  const float* p = m + (c0 + q) * ld + x;
+  return f32x4{p[0], p[4 * ld], p[8 * ld], p[12 * ld]};
+}
+
 __device__ __forceinline__ int acc_row(int r, int half) { return 8 * (r >> 2) + 4 * half + (r & 3); }
 
 // x of lanes 32..63 trades places with y of lanes 0..31 ...
@@ -59,6 +73,18 @@ __device__ __forceinline__ void swap_quarters(uint32_t& x, uint32_t& y) {
   const auto r = __builtin_amdgcn_permlane16_swap(x, y, false, false);
   x = r[0];
   y = r[1];
+}
+// Elements 4 (l/16) + e of an accumulator column to elements 4 e + l/16 (the B operand of
+// the next product, its indices in order), by an exchange of quarters and elements.
+__device__ __forceinline__ f32x4 acc_inorder(f32x4 x) {
+  uint32_t u[4];
+  __builtin_memcpy(u, &x, 16);
+  swap_halves(u[0], u[2]);
+  swap_halves(u[1], u[3]);
+  swap_quarters(u[0], u[1]);
+  swap_quarters(u[2], u[3]);
+  __builtin_memcpy(&x, u, 16);
+  return x;
 }
 // The value of another lane of the row of 16: l ^ 8, l ^ 7, l ^ 3, l ^ 2, l ^ 1.
 constexpr int DPP_XOR8 = 0x128, DPP_XOR7 = 0x141, DPP_XOR3 = 0x1b, DPP_XOR2 = 0x4e, DPP_XOR1 = 0xb1;

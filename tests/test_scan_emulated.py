@@ -124,6 +124,26 @@ def test_emulated_scan_backward_matches_autograd_of_recurrence(host, case, with_
     assert all(e < tol for e in errs.values()), errs
 
 
+@pytest.mark.parametrize("dtype,kd", [(torch.float32, 16), (torch.float32, 100), (torch.bfloat16, 16)], ids=str)
+def test_emulated_inverse_of_parallel_keys(host, monkeypatch, dtype, kd):
+    """T = (I + A)^-1 for keys that all point one way, where A_ts = beta_t exactly
+    and the terms of T's sums cancel from row to row: summed in order, no partial
+    sum is above a few times T's elements (of at most 1) and its error stays below
+    two roundings, 2^-23 of its norm (the host build rounds the products of the
+    diagonal blocks too); where four rows apart are added first it is larger."""
+    from gpa_amd import ops
+    k = torch.zeros(1, 64, 1, kd, dtype=dtype)
+    k[..., 3] = 2.
+    beta = (torch.randn(1, 64, 1, generator=torch.Generator().manual_seed(2)) + 2).sigmoid()
+    ops.gdn_scan_hip(None, k, torch.ones(1, 64, 1, 8, dtype=dtype), torch.zeros(1, 64, 1), beta, None, chunk=64)
+    work = next(b for _, b in ops._pieces.made.values() if b[2 if dtype == torch.float32 else 3] is not None and len(b) == 8)
+    tri = work[5].view(64, 64).double()
+    a = beta.double().view(64, 1).expand(64, 64).tril(-1)
+    err = _rel(tri, torch.linalg.inv(torch.eye(64, dtype=torch.float64) + a))
+    print(err)
+    assert err < 2 ** -23
+
+
 def _off_boundary(x):
     """The same values in rows that start 2 bytes past a 16-byte boundary."""
     wide = torch.zeros(*x.shape[:-1], x.shape[-1] + 9, dtype=x.dtype)
