@@ -43,7 +43,10 @@ namespace gpa {
 // barriers.  The A operands come straight from the saved rows (16-byte reads
 // along the keys; KM/64 adjacent keys per lane and position the other way, so
 // tile i of a wave holds every KM/64-th of its keys), a chunk ahead of their
-// use where the registers allow (PF).  Bound: the chain of chunks, its MFMAs
+// use where the registers allow (PF).  D and dD enter the state in the order of their
+// positions (see ld_c_inorder): with nearly parallel keys (a spread of 0.02) the errors of
+// the final state and of dq are 0.63 and 0.87 of those of scalar sums in that order, but
+// 0.75 and 1.12 in the MFMAs' own order of 16.  Bound: the chain of chunks, its MFMAs
 // (16 KM/64 for each of the two or three products of a wave, 32 cycles each) and the
 // two exchanges.  16 columns rather than 32 double the workgroups: a scan of
 // 32 streams by 64 columns is 128 of them.  FULL: K is a multiple of 16.
@@ -79,15 +82,16 @@ __device__ __forceinline__ void load_rows(f32x4 (&a)[KM / 16], const float* rows
   for (int g = 0; g < KM / 16; ++g)
     a[g] = row4<FULL>(rows + (int64_t)pos * K, 16 * g + 4 * q, K);
 }
-// The rows of a chunk as the A operand of a product over the positions:
-// positions 16 g + 4 (l/16) + e, keys k0 .. k0 + VEC-1 (tile i holds key k0 + i).
-template <int VEC, bool FULL>
+// The rows of a chunk as the A operand of a product over the positions: keys
+// k0 .. k0 + VEC-1 (tile i holds key k0 + i), positions 16 g + 4 e + l/16, which the
+// MFMAs take in order (INORDER), or 16 g + 4 (l/16) + e.
+template <int VEC, bool FULL, bool INORDER = true>
 __device__ __forceinline__ void load_cols(f32x4 (&a)[4 * VEC], const float* rows, int k0, int q, int K) {
 #pragma unroll
   for (int g = 0; g < 4; ++g)
 #pragma unroll
     for (int e = 0; e < 4; ++e) {
-      const float* row = rows + (int64_t)(16 * g + 4 * q + e) * K;
+      const float* row = rows + (int64_t)(16 * g + (INORDER ? 4 * e + q : 4 * q + e)) * K;
       float x[VEC];
       if (FULL) {
         __builtin_memcpy(x, __builtin_assume_aligned(row + (k0 < K ? k0 : 0), 4 * VEC), sizeof x);
@@ -179,7 +183,7 @@ __global__ __launch_bounds__(NT) void gdn_state_fwd(gpa_gdn_problem p, gpa_gdn_s
     f32x4 ds4;
 #pragma unroll
     for (int e = 0; e < 4; ++e) ds4[e] = __expf(gc - gm[e]) * d[e];
-    *reinterpret_cast<f32x4*>(ds + t0) = ds4;
+    *reinterpret_cast<f32x4*>(ds + t0) = acc_inorder(ds4);
     const float decay = __expf(gc);
     if (!PF) load_first(nn, wr, u, gm, gc);
     lds_barrier();
@@ -414,7 +418,7 @@ __global__ __launch_bounds__(NT) void gdn_state_bwd(gpa_gdn_problem p, gpa_gdn_s
   };
   auto load_second = [&](int n, f32x4 (&qc)[4 * VEC], f32x4 (&wc)[4 * VEC], f32x4 (&o)[4]) {
     if (has_q) {
-      load_cols<VEC, FULL>(qc, sv.qn + rows_off(s, n, nch, 0, K), k0, q, K);
+      load_cols<VEC, FULL, false>(qc, sv.qn + rows_off(s, n, nch, 0, K), k0, q, K);
 #pragma unroll
       for (int g = 0; g < 4; ++g)
         o[g] = *reinterpret_cast<const f32x4*>(gr.o + vc_off(s, n, nch, V) + (int64_t)vc * R + 16 * g + 4 * q);
@@ -443,7 +447,7 @@ __global__ __launch_bounds__(NT) void gdn_state_bwd(gpa_gdn_problem p, gpa_gdn_s
 #pragma unroll
     for (int e = 0; e < 4; ++e) dd[e] = d0[e] + __expf(gc - gm[e]) * dd[e];
     if (vok) *reinterpret_cast<f32x4*>(gr.ddelta + vc_off(s, n, nch, V) + (int64_t)v * R + t0) = dd;
-    *reinterpret_cast<f32x4*>(ds + t0) = -dd;
+    *reinterpret_cast<f32x4*>(ds + t0) = acc_inorder(-dd);
     const float decay = __expf(gc);
     if (!PF) load_first(nn, kr, d0, gm, gc);
     lds_barrier();

@@ -32,3 +32,30 @@ def test_float32_state_matches_recurrence(case):
     errs = [_rel(a, b) for a, b in zip((*got, *dg), (*want, *dr))]
     print(case, errs)
     assert max(errs) < 1e-5, errs
+
+
+def telescoping(scan, device, kd=64):
+    """(final state's rows, last value) of a float32 scan of 150 tokens whose
+    keys all point one way and whose writes are full: S_t = k v_t^T."""
+    gen = torch.Generator().manual_seed(4)
+    t, vd = 150, 32
+    v = torch.randint(-2 ** 22 + 1, 2 ** 22, (1, t, 1, vd), generator=gen).float() / 2 ** 12
+    k = torch.zeros(1, t, 1, kd)
+    k[..., 5] = 1.
+    args = [x.to(device) for x in (k, v, torch.zeros(1, t, 1), torch.ones(1, t, 1))]
+    final = scan(None, *args, None, chunk=64, offset=0)[2]
+    want = torch.zeros_like(final)
+    want[:, :, 5] = v[:, -1].to(device)
+    return final, want
+
+
+@pytest.mark.parametrize("kd", [16, 64, 72, 128, 256])
+def test_float32_state_sums_positions_in_order(kd):
+    """Each write undoes the one before (D_t = v_t - v_{t-1}).  The values are
+    multiples of 2^-12 below 2^10, so that each difference, and each partial sum
+    of a sum in the positions' order (it is v_t), is a float32 number: the
+    final state is the last value exactly.  In another order the partial sums
+    need more bits."""
+    from gpa_amd.ops import gdn_scan_hip
+    final, want = telescoping(gdn_scan_hip, DEV, kd)
+    assert torch.equal(final, want)

@@ -23,6 +23,7 @@ import torch
 
 from tests.host_emu import harness
 from tests.test_gpu_gdn_scan import _inputs, _oracle_segments, _oracle_segments_autograd, _rel
+from tests.test_gpu_gdn_state_f32 import telescoping
 
 CASES = [
     # (B, T, H, K, V, chunk, offset, dtype)
@@ -122,6 +123,17 @@ def test_emulated_scan_backward_matches_autograd_of_recurrence(host, case, with_
     errs = {n: _rel(a.grad, r.grad) for n, a, r in zip(names, leaves, refs) if a is not None}
     print(case, with_q, errs)
     assert all(e < tol for e in errs.values()), errs
+
+
+def test_emulated_float32_state_sums_positions_in_order(host):
+    """Keys that all point one way and full writes: every position's write undoes
+    the one before (D_t = v_t - v_{t-1}).  The values are multiples of 2^-12 below 2^10,
+    so that each difference, and each partial sum of a sum in the positions'
+    order (it is v_t), is a float32 number: the final state is the last value
+    exactly.  In any other order the partial sums need more bits."""
+    from gpa_amd.ops import gdn_scan_hip
+    final, want = telescoping(gdn_scan_hip, "cpu")
+    assert torch.equal(final, want)
 
 
 @pytest.mark.parametrize("dtype,kd", [(torch.float32, 16), (torch.float32, 100), (torch.bfloat16, 16)], ids=str)
