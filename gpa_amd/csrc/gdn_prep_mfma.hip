@@ -286,23 +286,6 @@ __global__ __launch_bounds__(PREP_NT, 1) void gdn_prep_mfma(gpa_gdn_problem p, g
 }
 
 // ---------------------------------------------------------------------------
-// gdn_prep_frag: the same chunk preparation for the bf16 MFMA path (bf16
-// activations, K a multiple of 16), built around the fragments it writes.  Wave w
-// holds rows 8 w .. 8 w + 7; lane (r = l/8, l%8) holds 8-key pieces (or 8-value
-// ones) of row 8 w + r, read in 16-byte loads that are all issued first.  A
-// normalised key piece is a krow piece as it stands; the 8 x 8 in-wave
-// transpose (transpose8) of a piece is a kcol / qcol piece, and of a value
-// piece the B operand of U.  krow, then kcol pass through LDS (same place) as
-// the operands of A and W.  The fp32 T enters the products as three bf16 parts
-// (all of its 24 bits; keys and values are exact), and W is formed twice, as T Kn
-// and as Kn^T T^T, so that both orders of its fragments leave the
-// accumulators after one half-wave exchange.  The barriers order LDS alone,
-// so stores drain behind the later phases.  52 KB of LDS and 80 registers at
-// 128 keys (three workgroups per compute unit), 68 KB at 256 (two).
-// Bound: HBM.  At 128 x 128 a chunk reads 48 KB and writes 176 KB: 32 streams x
-// 64 chunks take 87 us, 5.3 TB/s; the rows and fragments through float32 LDS
-// rows, with fp32 MFMA and element-wise loads and transposed stores, took 170 us.
-// K = 256, 16 streams x 32 chunks: 92 -> 40 us; one workgroup alone: 34 -> 18 us.
 // Lanes l/8 = 0..7 of one l%8 hold the rows of an 8 x 8 bf16 matrix; returns
 // its columns the same way.  Bits 2 and 1 of the row trade places with the
 // dword index, bit 0 with the half of a dword.
@@ -358,6 +341,23 @@ __device__ __forceinline__ void put_split_rows(const f32x16& acc, int gp, __bf16
   *reinterpret_cast<bf16x8*>(frag + 512 + lane * 8) = x.lo;
 }
 
+// gdn_prep_frag: the same chunk preparation for the bf16 MFMA path (bf16
+// activations, K a multiple of 16), built around the fragments it writes.  Wave w
+// holds rows 8 w .. 8 w + 7; lane (r = l/8, l%8) holds 8-key pieces (or 8-value
+// ones) of row 8 w + r, read in 16-byte loads that are all issued first.  A
+// normalised key piece is a krow piece as it stands; the 8 x 8 in-wave
+// transpose (transpose8) of a piece is a kcol / qcol piece, and of a value
+// piece the B operand of U.  krow, then kcol pass through LDS (same place) as
+// the operands of A and W.  The fp32 T enters the products as three bf16 parts
+// (all of its 24 bits; keys and values are exact), and W is formed twice, as T Kn
+// and as Kn^T T^T, so that both orders of its fragments leave the
+// accumulators after one half-wave exchange.  The barriers order LDS alone,
+// so stores drain behind the later phases.  52 KB of LDS and 80 registers at
+// 128 keys (three workgroups per compute unit), 68 KB at 256 (two).
+// Bound: HBM.  At 128 x 128 a chunk reads 48 KB and writes 176 KB: 32 streams x
+// 64 chunks take 87 us, 5.3 TB/s; the rows and fragments through float32 LDS
+// rows, with fp32 MFMA and element-wise loads and transposed stores, took 170 us.
+// K = 256, 16 streams x 32 chunks: 92 -> 40 us; one workgroup alone: 34 -> 18 us.
 template <int KM>
 struct PrepFragLayout {
   static constexpr int FRAG = (KM < 128 ? 128 : KM) * R * 2;  // bytes of the krow / kcol fragments

@@ -383,7 +383,7 @@ __global__ __launch_bounds__(NT) void gdn_dd0(gpa_gdn_problem p, gpa_gdn_saved s
 
 // ---------------------------------------------------------------------------
 // gdn_state_bwd: reverse sequential dS; writes dS at every chunk end and dD.
-// (The layout of gdn_state_fwd; has_q and has_inj are uniform.)
+// (The layout of gdn_state_fwd; whether there are a read and injections is uniform.)
 template <int KM, bool FULL>
 __global__ __launch_bounds__(NT) void gdn_state_bwd(gpa_gdn_problem p, gpa_gdn_saved sv, gpa_gdn_grads gr,
                                                      int nch) {

@@ -249,9 +249,4 @@ __device__ __forceinline__ void mma_split_exact(f32x16& c, const SplitBf8& a, bf
   mma_bf16(c, a.lo, b);
 }
 
-template <typename E>
-__device__ __forceinline__ f32x4 round4(f32x4 x) {
-  return f32x4{round_as<E>(x.x), round_as<E>(x.y), round_as<E>(x.z), round_as<E>(x.w)};
-}
-
 }  // namespace gpa

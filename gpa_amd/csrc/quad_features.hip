@@ -14,8 +14,9 @@
 // normalisations, da = (dz b) c and db = dz (c a) rounded to E, and
 // du = dz + da L^T + db R^T as one MFMA product over the concatenated
 // [da | db] rows; dx follows through unit(x) and ||x||.  It also writes u and
-// [da | db] head-major for the weight gradients u^T [da | db] (a plain
-// batched GEMM the caller runs) and one partial sum of dc per workgroup.
+// [da | db] head-major for the weight gradients u^T [da | db] (bf16:
+// gpa_quad_weight_grads, two launches; float32: a batched product the caller
+// runs) and one partial sum of dc per workgroup.
 #include <hip/hip_runtime.h>
 
 #include <initializer_list>
