@@ -441,7 +441,7 @@ def main() -> int:
                     "peak": PEAK_BF16_TFLOPS, "unit": "TFLOP/s", "frac": dominant["tflops"] / PEAK_BF16_TFLOPS,
                     "traffic": _measured_traffic(dominant["name"]),
                     "limited_by": ("latency of the sequential chunk chain (one state step per 64 tokens)"
-                                   if chain else "issue latency at one workgroup per CU"),
+                                   if chain else "HBM traffic (see traffic) and exposed latency at one workgroup per CU"),
                     "avg_launch_us": dominant["avg_us"], "launches": dominant["launches"],
                     "share_of_step": dominant["total_ms"] / serial_ms,
                     "timed_in": f"one extra step on one stream ({serial_ms:.1f} ms)"}

@@ -21,10 +21,12 @@
 // Their fragments, and their transposes', leave the accumulators through one
 // half-wave exchange and an in-wave 8 x 8 transpose.
 //
-// Bound: a workgroup's chain of phases (one workgroup of 256 registers per compute
-// unit); the value loop's reads alone run near HBM rate.  32 streams x 64 chunks,
-// 128 x 128: 266 us (920 MB, 3.5 TB/s; 419 us with operands split by every wave
-// that reads them); 256 x 128, 16 x 32 chunks: 124 us (235).
+// Bound: the HBM traffic it chooses (the saved fragments and rows, states and their
+// gradients: 945 MB read and 135 MB written at 32 streams x 64 chunks of 128 x 128,
+// about 0.6 GB of them unavoidable), then a workgroup's chain of phases (one workgroup
+// of 256 registers per compute unit).  That launch takes 272 us, 4.0 TB/s, 85 % of a
+// copy's rate (419 us with operands split by every wave that reads them); 256 x 128,
+// 16 streams x 32 chunks: 120 us (235).
 #include <hip/hip_runtime.h>
 
 #include <type_traits>
