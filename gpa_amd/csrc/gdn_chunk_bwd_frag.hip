@@ -171,7 +171,7 @@ __global__ __launch_bounds__(CF_NT, 2) void gdn_chunk_bwd_frag(gpa_gdn_problem p
   };
   fetch(0);
 
-  // ---- row norms of the raw keys and queries (the preparation's sums).
+  // ---- row norms of the raw keys and queries.
   {
     const int row = 8 * wave + (lane >> 3), pc = lane & 7, tok = token_at(p, n, row), tt = tok >= 0 ? tok : 0;
     const gpa_operand& qsrc = HQ ? p.q : p.k;

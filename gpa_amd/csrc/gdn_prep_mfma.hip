@@ -25,16 +25,16 @@ constexpr int PREP_LT = R + 4;  // row pitch of A and T in LDS
 // of its 16 x 16 diagonal blocks; the blocks above them are not read), by every
 // thread of the workgroup: t_s starts as zeros, A and T rows PREP_LT apart.
 // Wave 0 inverts the four diagonal blocks by forward substitution, a column
-// per lane, in registers; then the inverses of neighbouring diagonal blocks
-// T11, T22 give that of twice their size, T21 = -T22 (A21 T11), for 32 and for
-// 64 rows on 16 x 16 tiles of the fp32 MFMA.  A21 T11 goes from the accumulators to
-// the next product's B operand in registers (acc_inorder).  The sums run over the
-// rows in order: for nearly parallel keys, whose terms cancel from row to row, the
-// error of T is that of forward substitution (3e-8 of its norm at b = 0.88; 1.5e-7 in
-// the order in which mma16 takes four adjacent rows a lane).
-// Bound: the latency of its three short phases.  Against forward substitution
-// through LDS with run-time trip counts and scalar block products, the prep of
-// 32 streams x 64 chunks of 128 keys takes 27 us less (of 170).
+// per lane, in registers; then block rows i = 1..3 of 16: T_ij = -T_ii sum_{j<=m<i}
+// A_im T_mj on the fp32 MFMA, block column j by wave j: its sums and tiles go from the
+// accumulators to the next product's B operand in registers (acc_inorder), so that the
+// waves do not meet in between.  Every sum runs over the
+// rows in order: for nearly parallel keys, whose terms cancel from row to row, any
+// other order adds large partial sums (an error of 1.5e-7 of T's norm at b = 0.88
+// in the order in which mma16 takes four adjacent rows a lane, 3e-8 in order).
+// Bound: the latency of 16 substitution steps and of wave 0's 36 MFMAs.  Against forward substitution
+// through LDS with run-time trip counts and scalar block products (the same sums),
+// the prep of 32 streams x 64 chunks of 128 keys takes 27 us less (of 170).
 __device__ __forceinline__ void unit_lower_inverse(const float* a_s, float* t_s, int wave, int lane) {
   constexpr int LT = PREP_LT;
   const int c = lane & 15, q = lane >> 4;
@@ -57,32 +57,24 @@ __device__ __forceinline__ void unit_lower_inverse(const float* a_s, float* t_s,
     for (int t = 0; t < 16; ++t) t_s[(16 * q + t) * LT + 16 * q + c] = x[t];
   }
   lds_barrier();
-  const f32x4 zero = {0.f, 0.f, 0.f, 0.f};
-  if (wave < 2) {  // 16 -> 32 rows: pair `wave`
-    const int lo = 32 * wave, hi = lo + 16;
-    f32x4 x = zero, y = zero;
-    mma16(x, ld_c_inorder(a_s, LT, hi + c, lo, q), ld_x_inorder(t_s, LT, lo + c, lo, q));
-    mma16(y, ld_c_inorder(t_s, LT, hi + c, hi, q), acc_inorder(x));
+  if (wave < 3) {  // block column j = wave, whose tiles stay in registers as B operands
+    const int j = wave;
+    f32x4 tj[3];
 #pragma unroll
-    for (int e = 0; e < 4; ++e) t_s[(hi + 4 * q + e) * LT + lo + c] = -y[e];
-  }
-  lds_barrier();
-  if (wave < 4) {  // 32 -> 64 rows: tile (i, j) of the corner
-    const int i = wave >> 1, j = wave & 1;
-    f32x4 x[2] = {zero, zero}, y = zero;
+    for (int m = 0; m < 3; ++m)
+      if (m == j) tj[m] = ld_x_inorder(t_s, LT, 16 * j + c, 16 * j, q);
 #pragma unroll
-    for (int m = 0; m < 2; ++m) {
-      if (m > i) continue;
+    for (int i = 1; i < 4; ++i) {
+      if (i <= j) continue;
+      f32x4 x = {0.f, 0.f, 0.f, 0.f}, y = x;
 #pragma unroll
-      for (int k = 0; k < 2; ++k)
-        if (k >= j)
-          mma16(x[m], ld_c_inorder(a_s, LT, 32 + 16 * m + c, 16 * k, q), ld_x_inorder(t_s, LT, 16 * j + c, 16 * k, q));
+      for (int m = 0; m < i; ++m)
+        if (m >= j) mma16(x, ld_c_inorder(a_s, LT, 16 * i + c, 16 * m, q), tj[m]);
+      mma16(y, ld_c_inorder(t_s, LT, 16 * i + c, 16 * i, q), acc_inorder(x));
+#pragma unroll
+      for (int e = 0; e < 4; ++e) t_s[(16 * i + 4 * q + e) * LT + 16 * j + c] = -y[e];
+      if (i < 3) tj[i] = acc_inorder(-y);
     }
-#pragma unroll
-    for (int m = 0; m < 2; ++m)
-      if (m <= i) mma16(y, ld_c_inorder(t_s, LT, 32 + 16 * i + c, 32 + 16 * m, q), acc_inorder(x[m]));
-#pragma unroll
-    for (int e = 0; e < 4; ++e) t_s[(32 + 16 * i + 4 * q + e) * LT + 16 * j + c] = -y[e];
   }
   lds_barrier();
 }
@@ -310,37 +302,6 @@ __device__ __forceinline__ bf16x8 as_bf16x8(uint4 v) {
   return r;
 }
 
-// Eight floats as three bf16 parts whose sum is the float (24 bits).
-struct Split3 {
-  bf16x8 part[3];
-};
-__device__ __forceinline__ Split3 split3(const float (&x)[8]) {
-  Split3 s;
-  float y[8];
-#pragma unroll
-  for (int e = 0; e < 8; ++e) y[e] = x[e];
-#pragma unroll
-  for (int i = 0; i < 3; ++i) {
-    uint32_t w[4];
-#pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      w[j] = bf2_pack(y[2 * j], y[2 * j + 1]);
-      y[2 * j] -= bf2_low(w[j]);
-      y[2 * j + 1] -= bf2_high(w[j]);
-    }
-    __builtin_memcpy(&s.part[i], w, 16);
-  }
-  return s;
-}
-
-// The accumulator tile's rows 16 gp .. 16 gp + 15, eight consecutive rows per lane
-// (rows + 8 in the upper lanes), as bf16 hi and lo fragment pieces.
-__device__ __forceinline__ void put_split_rows(const f32x16& acc, int gp, __bf16* frag, int lane) {
-  const SplitBf8 x = split_rows(acc, gp);
-  *reinterpret_cast<bf16x8*>(frag + lane * 8) = x.hi;
-  *reinterpret_cast<bf16x8*>(frag + 512 + lane * 8) = x.lo;
-}
-
 // gdn_prep_frag: the same chunk preparation for the bf16 MFMA path (bf16
 // activations, K a multiple of 16), built around the fragments it writes.  Wave w
 // holds rows 8 w .. 8 w + 7; lane (r = l/8, l%8) holds 8-key pieces (or 8-value
@@ -348,16 +309,19 @@ __device__ __forceinline__ void put_split_rows(const f32x16& acc, int gp, __bf16
 // normalised key piece is a krow piece as it stands; the 8 x 8 in-wave
 // transpose (transpose8) of a piece is a kcol / qcol piece, and of a value
 // piece the B operand of U.  krow, then kcol pass through LDS (same place) as
-// the operands of A and W.  The fp32 T enters the products as three bf16 parts
-// (all of its 24 bits; keys and values are exact), and W is formed twice, as T Kn
-// and as Kn^T T^T, so that both orders of its fragments leave the
-// accumulators after one half-wave exchange.  The barriers order LDS alone,
-// so stores drain behind the later phases.  52 KB of LDS and 80 registers at
-// 128 keys (three workgroups per compute unit), 68 KB at 256 (two).
+// the operands of A and W.  W and U are fp32 products, summed as in gdn_prep_mfma
+// (mma8), and the row norms as there, so that its results keep the bits that
+// element-wise loads and LDS rows gave; a tile of W gives both orders of its
+// fragments, the second through an in-wave transpose.  The barriers order LDS
+// alone, so stores drain behind the later phases.  52 KB of LDS at 128 keys
+// (three workgroups per compute unit), 68 KB at 256 (two).
 // Bound: HBM.  At 128 x 128 a chunk reads 48 KB and writes 176 KB: 32 streams x
-// 64 chunks take 87 us, 5.3 TB/s; the rows and fragments through float32 LDS
-// rows, with fp32 MFMA and element-wise loads and transposed stores, took 170 us.
-// K = 256, 16 streams x 32 chunks: 92 -> 40 us; one workgroup alone: 34 -> 18 us.
+// 64 chunks take 92 us, 5.2 TB/s; the same arithmetic with the rows and fragments
+// through float32 LDS rows, element-wise loads and transposed stores took 170 us.
+// K = 256, 16 streams x 32 chunks: 92 -> 42 us; one workgroup alone: 34 -> 20 us.
+// (T split exactly in three bf16 parts, for the bf16 MFMA, is faster by 2, 4 and 3 us
+// at the same error, but its sums round otherwise, and each bf16 rounding that flips
+// travels through the layers: 4e-4 of a layer's output, 5e-3 of the LM layer's.)
 template <int KM>
 struct PrepFragLayout {
   static constexpr int FRAG = (KM < 128 ? 128 : KM) * R * 2;  // bytes of the krow / kcol fragments
@@ -434,7 +398,7 @@ __global__ __launch_bounds__(PREP_NT, KM <= 128 ? 6 : 4) void gdn_prep_frag(gpa_
 
   // ---- normalise: x / |x| in float32, rounded to bf16.
   auto normalise = [&](uint4 (&x)[NP]) {
-    float ss = 0.f;
+    float ss[8] = {};
 #pragma unroll
     for (int j = 0; j < NP; ++j) {
       x[j] = keep(x[j], 64 * j + 8 * pc, K);
@@ -442,14 +406,31 @@ __global__ __launch_bounds__(PREP_NT, KM <= 128 ? 6 : 4) void gdn_prep_frag(gpa_
 #pragma unroll
       for (int e = 0; e < 4; ++e) {
         const float lo = bf2_low(w[e]), hi = bf2_high(w[e]);
-        ss += lo * lo;
-        ss += hi * hi;
+        ss[2 * e] += lo * lo;
+        ss[2 * e + 1] += hi * hi;
       }
     }
-    ss += __shfl_xor(ss, 1);
-    ss += __shfl_xor(ss, 2);
-    ss += __shfl_xor(ss, 4);
-    const float den = fmaxf(sqrtf(ss), 1e-6f);
+    // Keys 64 apart, then 32, 16, .. 1: the tree of sum64 over a key per lane, so that
+    // a late read's queries (gdn_prep_q) round alike.  Recursive halving over the row's
+    // eight lanes leaves element l%8 in lane l%8.
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const bool up = pc & 4;
+      const float send = up ? ss[i] : ss[i + 4], own = up ? ss[i + 4] : ss[i];
+      ss[i] = own + dpp_xor4(send);
+    }
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+      const bool up = pc & 2;
+      const float send = up ? ss[i] : ss[i + 2], own = up ? ss[i + 2] : ss[i];
+      ss[i] = own + dpp<DPP_XOR2>(send);
+    }
+    const bool up = pc & 1;
+    float sum = (up ? ss[1] : ss[0]) + dpp<DPP_XOR1>(up ? ss[0] : ss[1]);
+    sum += dpp_xor4(sum);
+    sum += dpp<DPP_XOR2>(sum);
+    sum += dpp<DPP_XOR1>(sum);
+    const float den = fmaxf(sqrtf(sum), 1e-6f);
 #pragma unroll
     for (int j = 0; j < NP; ++j) {
       uint32_t w[4] = {x[j].x, x[j].y, x[j].z, x[j].w};
@@ -544,49 +525,52 @@ __global__ __launch_bounds__(PREP_NT, KM <= 128 ? 6 : 4) void gdn_prep_frag(gpa_
       *reinterpret_cast<f32x4*>(tri + t * R + c) = *reinterpret_cast<const f32x4*>(t_s + t * LT + c);
     }
   }
-  // T rows 32 rt + l%32, columns 16 ks + 8 (l/32) .. +7, scaled per column.
-  const int rt = wave & 1, w4 = wave >> 1;
-  auto t_parts = [&](const float* scale, int ks) {
-    const int c0 = 16 * ks + 8 * hh;
-    const float* t = t_s + (32 * rt + li) * LT + c0;
-    float x[8];
-#pragma unroll
-    for (int e = 0; e < 2; ++e) {
-      const f32x4 y = *reinterpret_cast<const f32x4*>(t + 4 * e) * *reinterpret_cast<const f32x4*>(scale + c0 + 4 * e);
-#pragma unroll
-      for (int i = 0; i < 4; ++i) x[4 * e + i] = y[i];
-    }
-    return split3(x);
+  // Operands of mma8: T rows 32 rt + l%32 and, from column fragments in LDS, keys
+  // (values) 32 tile + l%32, both at positions 8 g + 4 (l/32) .. +3.  (Row tile 0 on
+  // waves 0-3, which share the SIMDs of waves 4-7: T is lower triangular, and
+  // tile 1 has twice the products.)
+  const int rt = wave >> 2, w4 = wave & 3, groups = 4 + 4 * rt;
+  auto at4 = [&](const float* a, int g) { return *reinterpret_cast<const f32x4*>(a + 8 * g + 4 * hh); };
+  auto col4 = [&](const uint4* frag, int tile, int g) {
+    const uint2 x = reinterpret_cast<const uint2*>(frag + (tile * 4 + (g >> 1)) * 64 + li + 32 * (g & 1))[hh];
+    return f32x4{bf2_low(x.x), bf2_high(x.x), bf2_low(x.y), bf2_high(x.y)};
   };
+  const float* t_row = t_s + (32 * rt + li) * LT;
   if (w4 < RB) {
-    f32x16 w[NM], wt[NM];
+    f32x16 w[NM];
 #pragma unroll
-    for (int m = 0; m < NM; ++m) w[m] = wt[m] = f32x16{};
+    for (int m = 0; m < NM; ++m) w[m] = f32x16{};
+#pragma unroll 4
+    for (int g = 0; g < groups; ++g) {
+      const f32x4 t = at4(t_row, g) * at4(sc_s, g);
 #pragma unroll
-    for (int ks = 0; ks < 4; ++ks) {
-      if (ks >= 2 + 2 * rt) continue;  // T is lower triangular
-      const Split3 t = t_parts(sc_s, ks);
-#pragma unroll
-      for (int m = 0; m < NM; ++m) {
-        if (w4 + 4 * m >= RB) continue;
-        const bf16x8 k = as_bf16x8(frag_s[((w4 + 4 * m) * 4 + ks) * 64 + lane]);
-#pragma unroll
-        for (int i = 0; i < 3; ++i) {
-          mma_bf16(w[m], t.part[i], k);
-          mma_bf16(wt[m], k, t.part[i]);
-        }
-      }
+      for (int m = 0; m < NM; ++m)
+        if (w4 + 4 * m < RB) mma8(w[m], t, col4(frag_s, w4 + 4 * m, g));
     }
     __bf16* wrow = reinterpret_cast<__bf16*>(sv.wrow) + chunk_id * frag_row_elems(K, 16);
     __bf16* wcol = reinterpret_cast<__bf16*>(sv.wcol) + chunk_id * frag_col_elems(K, 16);
+    const int oct = (lane >> 3) & 3;  // this lane's eight keys of the tile, once transposed
 #pragma unroll
     for (int m = 0; m < NM; ++m) {
       const int kt = w4 + 4 * m;
       if (kt >= RB) continue;
 #pragma unroll
       for (int gp = 0; gp < 2; ++gp) {
-        put_split_rows(w[m], gp, wcol + (int64_t)(kt * 4 + 2 * rt + gp) * 1024, lane);
-        if (2 * kt + gp < K16) put_split_rows(wt[m], gp, wrow + (int64_t)(rt * K16 + 2 * kt + gp) * 1024, lane);
+        const SplitBf8 x = split_rows(w[m], gp);
+        __bf16* col = wcol + (int64_t)(kt * 4 + 2 * rt + gp) * 1024 + lane * 8;
+        *reinterpret_cast<bf16x8*>(col) = x.hi;
+        *reinterpret_cast<bf16x8*>(col + 512) = x.lo;
+        uint4 hi, lo;
+        __builtin_memcpy(&hi, &x.hi, 16);
+        __builtin_memcpy(&lo, &x.lo, 16);
+        hi = transpose8_lanes(hi, lane);
+        lo = transpose8_lanes(lo, lane);
+        const int ks = 2 * kt + (oct >> 1);
+        __bf16* row = wrow + (int64_t)(rt * K16 + ks) * 1024 + (16 * gp + 8 * hh + (lane & 7) + 32 * (oct & 1)) * 8;
+        if (ks < K16) {
+          *reinterpret_cast<uint4*>(row) = hi;
+          *reinterpret_cast<uint4*>(row + 512) = lo;
+        }
       }
     }
   }
@@ -604,14 +588,8 @@ __global__ __launch_bounds__(PREP_NT, KM <= 128 ? 6 : 4) void gdn_prep_frag(gpa_
     lds_barrier();
     if (v0 + 32 * w4 < V) {
       f32x16 acc = {};
-#pragma unroll
-      for (int ks = 0; ks < 4; ++ks) {
-        if (ks >= 2 + 2 * rt) continue;
-        const Split3 t = t_parts(bet_s, ks);
-        const bf16x8 x = as_bf16x8(vf_s[(w4 * 4 + ks) * 64 + lane]);
-#pragma unroll
-        for (int i = 0; i < 3; ++i) mma_bf16(acc, t.part[i], x);
-      }
+#pragma unroll 4
+      for (int g = 0; g < groups; ++g) mma8(acc, at4(t_row, g), at4(bet_s, g) * col4(vf_s, w4, g));
       // Whole 32-column strips, zero past V (the padded strip is read too).
       const bool ok = v0 + 32 * w4 + li < V;
 #pragma unroll

@@ -96,6 +96,7 @@ __device__ __forceinline__ float dpp(float x) {
 __device__ __forceinline__ uint32_t dpp_xor4(uint32_t x) {
   return __builtin_amdgcn_mov_dpp(__builtin_amdgcn_mov_dpp(x, DPP_XOR7, 0xf, 0xf, false), DPP_XOR3, 0xf, 0xf, false);
 }
+__device__ __forceinline__ float dpp_xor4(float x) { return __uint_as_float(dpp_xor4(__float_as_uint(x))); }
 // Eight consecutive lanes hold the rows of an 8 x 8 bf16 matrix; returns its
 // columns the same way.  Bits 2 and 1 of the row trade places with the dword
 // index, bit 0 with the half of a dword.
@@ -123,7 +124,7 @@ __device__ __forceinline__ uint4 transpose8_lanes(uint4 v, int lane) {
 }
 
 // Sums of each of a lane's 16 accumulator-row values over the 32 lanes of its
-// half-wave, by recursive halving (lanes l ^ 16, 8, 7, 2, 1) without LDS.
+// half-wave, by recursive halving (lanes l ^ 16, 8, 4, 2, 1) without LDS.
 // Every lane returns the sum for register index sum_index(lane).
 __device__ __forceinline__ float tile_row_sum(float (&v)[16], int lane) {
 #pragma unroll
@@ -142,7 +143,7 @@ __device__ __forceinline__ float tile_row_sum(float (&v)[16], int lane) {
   for (int j = 0; j < 2; ++j) {
     const bool up = lane & 4;
     const float send = up ? v[j] : v[j + 2], keep = up ? v[j + 2] : v[j];
-    v[j] = keep + dpp<DPP_XOR7>(send);
+    v[j] = keep + dpp_xor4(send);
   }
   const bool up = lane & 2;
   const float send = up ? v[0] : v[1], keep = up ? v[1] : v[0];

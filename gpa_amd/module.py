@@ -42,7 +42,7 @@ class QuadraticFeatures(nn.Module):
 
     def forward(self, x: Tensor) -> Tensor:
         """x [..., H, D] on the GPU: one HIP launch forward, one backward (plus
-        the weight gradients' batched product), gpa_amd.features."""
+        the weight gradients), gpa_amd.features."""
         from .features import quadratic_features
         return quadratic_features(x, self.left, self.right, self.gain_raw)
 

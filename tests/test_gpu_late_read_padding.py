@@ -38,3 +38,15 @@ def test_late_read_in_new_memory(nan_memory, kd):
     errs = [_rel(a, b) for a, b in zip(res[1], res[0])]
     print(kd, errs)
     assert all(e < 2e-2 for e in errs), errs  # (a NaN fails)
+
+
+@pytest.mark.parametrize("kd,vd", [(48, 24), (128, 128), (256, 64)])
+def test_late_read_has_the_bits_of_the_read_built_in(kd, vd):
+    """Queries are normalised by two kernels (the scan's preparation and, for a
+    late read, gdn_prep_q) that sum a row's squares alike: the outputs are equal."""
+    from gpa_amd.ops import gdn_scan_deferred, gdn_scan_hip
+    q, *rest = (x.to(DEV) for x in _inputs(2, 700, 4, kd, vd, torch.bfloat16, seed=8))
+    out, states, final = gdn_scan_hip(q, *rest, chunk=64, offset=0)
+    late_states, late_final, read = gdn_scan_deferred(*rest, chunk=64, offset=0)
+    assert torch.equal(states, late_states) and torch.equal(final, late_final)
+    assert torch.equal(out, read(q))

@@ -18,6 +18,9 @@ bfloat16 scans of at most 128 keys take are not emulated (their LDS loads are
 inline global_load_lds): a plain recurrence stands in for them
 (host_emu/strip_reference.cpp), and the GPU tests cover them.
 """
+import ctypes
+import ctypes.util
+
 import pytest
 import torch
 
@@ -154,6 +157,63 @@ def test_emulated_inverse_of_parallel_keys(host, monkeypatch, dtype, kd):
     err = _rel(tri, torch.linalg.inv(torch.eye(64, dtype=torch.float64) + a))
     print(err)
     assert err < 2 ** -23
+
+
+def _chain_order(n):
+    """Contraction indices in the order in which mma8 adds them."""
+    return [8 * g + s + 4 * h for g in range(n // 8) for s in range(4) for h in range(2)]
+
+
+@pytest.mark.parametrize("kd,vd", [(16, 8), (80, 20)])
+def test_emulated_bf16_preparation_rounds_like_the_float32_products(host, kd, vd):
+    """The bf16 chunk preparation's float32 intermediates, bit for bit: the row
+    norms are sums over keys 64, 32, 16, .. 1 apart, W = T diag(b e^G) Kn and U =
+    T diag(b) V chains of fused multiply-adds in mma8's order over the float32
+    scaled operands, W leaving as bf16 hi and lo.  (An equal result in another
+    order flips bf16 roundings of everything that follows.)"""
+    from gpa_amd import ops
+    fmaf = ctypes.CDLL(ctypes.util.find_library("m")).fmaf
+    fmaf.restype, fmaf.argtypes = ctypes.c_float, [ctypes.c_float] * 3
+    _, k, v, _, beta, _ = _inputs(1, 64, 1, kd, vd, torch.bfloat16, seed=3)
+    ops.gdn_scan_hip(None, k, v, torch.zeros(1, 64, 1), beta, None, chunk=64)
+    work = next(b for _, b in ops._pieces.made.values() if len(b) == 8)
+    frag = next(b for _, b in ops._pieces.made.values() if len(b) == 5)
+    u, tri, bet = work[3], work[5].view(64, 64), work[7]
+    k16, rb = kd // 16, -(-kd // 32)
+
+    keys = torch.nn.functional.pad(k[0, :, 0].float(), (0, -kd % 64)).unflatten(1, (-1, 64))
+    tree = torch.zeros(64, 64)
+    for i in range(keys.shape[1]):
+        tree = (tree.double() + keys[:, i].double().square()).float()  # (one rounding: a fused multiply-add)
+    for apart in (32, 16, 8, 4, 2, 1):
+        tree = tree + tree[:, torch.arange(64) ^ apart]
+    kn = (k[0, :, 0].float() / tree[:, :1].sqrt().clamp_min(1e-6)).bfloat16()
+    # krow piece (t/32, k/16), lane t%32 + 32 ((k/8) % 2), element k%8
+    krow = frag[2].view(2, k16, 2, 32, 8).permute(0, 3, 1, 2, 4).reshape(64, kd)
+    assert torch.equal(krow, kn)
+
+    def product(scale, right):  # T diag(scale) right
+        left, out = (tri * scale).tolist(), torch.zeros(64, right.shape[1])
+        cols = right.t().tolist()
+        for t in range(64):
+            for j, col in enumerate(cols):
+                acc = 0.
+                for c in _chain_order(64):
+                    acc = fmaf(left[t][c], col[c], acc)
+                out[t, j] = acc
+        return out
+
+    w = product(bet, kn.float())
+    hi = w.bfloat16()
+    lo = (w - hi.float()).bfloat16()
+    wrow = frag[0].view(2, k16, 2, 2, 32, 8).permute(2, 0, 4, 1, 3, 5).reshape(2, 64, kd)
+    assert torch.equal(wrow, torch.stack((hi, lo)))
+    # wcol piece (k/32, t/16), lane k%32 + 32 ((t/8) % 2), element t%8
+    wcol = frag[1].view(rb, 4, 2, 2, 32, 8).permute(2, 1, 3, 5, 0, 4).reshape(2, 64, 32 * rb)
+    assert torch.equal(wcol[..., :kd], torch.stack((hi, lo))) and not wcol[..., kd:].any()
+    # U block [v/32][t/32][(t/8) % 4][v%32 + 32 ((t/4) % 2)][t%4]
+    uv = u.view(-1, 2, 4, 2, 32, 4).permute(1, 2, 3, 5, 0, 4).reshape(64, -1)
+    assert torch.equal(uv[:, :vd], product(torch.ones(64), bet[:, None] * v[0, :, 0].float()))
 
 
 def _off_boundary(x):
