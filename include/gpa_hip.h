@@ -725,7 +725,8 @@ int gpa_moment_scan_many(const gpa_moment_problem *problems, int32_t n, hipStrea
  * u and d(a)|d(b): float32 [heads][DP][DP], sums rounded to bf16.  Spans of the rows
  * are summed apart in `partials`, gpa_quad_grad_partials(problem) floats (-1 for a
  * problem that no entry point takes), then in the order of the rows: equal calls give
- * equal bits.  Its buffers start on 16-byte boundaries. */
+ * equal bits.  (Of buffers off 16-byte boundaries the spans are added by atomics, in
+ * any order.) */
 #define GPA_QUAD_MAX_DIM 256
 
 typedef struct gpa_quad_problem {
