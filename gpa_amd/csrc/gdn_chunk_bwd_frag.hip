@@ -22,11 +22,11 @@
 // half-wave exchange and an in-wave 8 x 8 transpose.
 //
 // Bound: the HBM traffic it chooses (the saved fragments and rows, states and their
-// gradients: 945 MB read and 135 MB written at 32 streams x 64 chunks of 128 x 128,
+// gradients: 948 MB read and 135 MB written at 32 streams x 64 chunks of 128 x 128,
 // about 0.6 GB of them unavoidable), then a workgroup's chain of phases (one workgroup
-// of 256 registers per compute unit).  That launch takes 272 us, 4.0 TB/s, 85 % of a
+// of 256 registers per compute unit).  That launch takes 270 us, 4.0 TB/s, 85 % of a
 // copy's rate (419 us with operands split by every wave that reads them); 256 x 128,
-// 16 streams x 32 chunks: 120 us (235).
+// 16 streams x 32 chunks: 123 us (235).
 #include <hip/hip_runtime.h>
 
 #include <type_traits>

@@ -316,9 +316,9 @@ __device__ __forceinline__ bf16x8 as_bf16x8(uint4 v) {
 // alone, so stores drain behind the later phases.  52 KB of LDS at 128 keys
 // (three workgroups per compute unit), 68 KB at 256 (two).
 // Bound: HBM.  At 128 x 128 a chunk reads 48 KB and writes 176 KB: 32 streams x
-// 64 chunks take 92 us, 5.2 TB/s; the same arithmetic with the rows and fragments
+// 64 chunks take 92-97 us, 5.0-5.2 TB/s; the same arithmetic with the rows and fragments
 // through float32 LDS rows, element-wise loads and transposed stores took 170 us.
-// K = 256, 16 streams x 32 chunks: 92 -> 42 us; one workgroup alone: 34 -> 20 us.
+// K = 256, 16 streams x 32 chunks: 92 -> 43 us; one workgroup alone: 34 -> 20 us.
 // (T split exactly in three bf16 parts, for the bf16 MFMA, is faster by 2, 4 and 3 us
 // at the same error, but its sums round otherwise, and each bf16 rounding that flips
 // travels through the layers: 4e-4 of a layer's output, 5e-3 of the LM layer's.)
