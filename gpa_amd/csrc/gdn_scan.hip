@@ -43,16 +43,21 @@ namespace gpa {
 // barriers.  The A operands come straight from the saved rows (16-byte reads
 // along the keys; KM/64 adjacent keys per lane and position the other way, so
 // tile i of a wave holds every KM/64-th of its keys), a chunk ahead of their
-// use where the registers allow (PF).  D and dD enter the state in the order of their
-// positions (see ld_c_inorder): with nearly parallel keys (a spread of 0.02) the errors of
-// the final state and of dq are 0.63 and 0.87 of those of scalar sums in that order, but
-// 0.75 and 1.12 in the MFMAs' own order of 16.  Bound: the chain of chunks, its MFMAs
-// (16 KM/64 for each of the two or three products of a wave, 32 cycles each) and the
-// two exchanges.  16 columns rather than 32 double the workgroups: a scan of
+// use where the registers allow (PF).  Every sum is the scalar recurrence's chain of fused
+// multiply-adds: D starts at U and takes the keys in order, dD at dd0, a row of the state at
+// position 0's product and then e^G_C S and positions 1, 2, ..., one of dS at e^G_C dS
+// and takes the positions in order, and the rows' factors e^{G_C-G} are on Kn, not on the products.
+// An MFMA adds its four contraction indices in order, so lanes l/16 + 4 e hold
+// consecutive indices (acc_inorder), and the results have the bits of scalar FMAs, with
+// nearly parallel keys too (sums after U, in the MFMAs' own order of 16, moved the float32 layer's
+// gate gradients by up to twice their error either way).  Bound: the chain of chunks, its
+// MFMAs (16 KM/64 for each of the two or three products of a wave, 32 cycles each) and
+// the two exchanges.  16 columns rather than 32 double the workgroups: a scan of
 // 32 streams by 64 columns is 128 of them.  FULL: K is a multiple of 16.
 // Measured at 32 streams x 16 chunks against scalar FMA products over operands
-// staged through LDS: K = 64, V = 64: 349 -> 28 us forward, 509 -> 38 us
-// backward; K = 128, V = 64: 681 -> 54 us and 1021 -> 64 us.
+// staged through LDS: K = 64, V = 64: 349 -> 30 us forward, 509 -> 40 us
+// backward; K = 128, V = 64: 681 -> 58 us and 1021 -> 63 us (of which the order
+// and its exchanges cost 5, 2, 7 and 3 us).
 constexpr int SC = 16;  // state columns per workgroup
 
 // Element 4 j + e (e < 4) of a lane's KM/16 keys, as the accumulators hold them.
@@ -84,14 +89,14 @@ __device__ __forceinline__ void load_rows(f32x4 (&a)[KM / 16], const float* rows
 }
 // The rows of a chunk as the A operand of a product over the positions: keys
 // k0 .. k0 + VEC-1 (tile i holds key k0 + i), positions 16 g + 4 e + l/16, which the
-// MFMAs take in order (INORDER), or 16 g + 4 (l/16) + e.
-template <int VEC, bool FULL, bool INORDER = true>
+// MFMAs take in order.
+template <int VEC, bool FULL>
 __device__ __forceinline__ void load_cols(f32x4 (&a)[4 * VEC], const float* rows, int k0, int q, int K) {
 #pragma unroll
   for (int g = 0; g < 4; ++g)
 #pragma unroll
     for (int e = 0; e < 4; ++e) {
-      const float* row = rows + (int64_t)(16 * g + (INORDER ? 4 * e + q : 4 * q + e)) * K;
+      const float* row = rows + (int64_t)(16 * g + 4 * e + q) * K;
       float x[VEC];
       if (FULL) {
         __builtin_memcpy(x, __builtin_assume_aligned(row + (k0 < K ? k0 : 0), 4 * VEC), sizeof x);
@@ -103,17 +108,22 @@ __device__ __forceinline__ void load_cols(f32x4 (&a)[4 * VEC], const float* rows
       for (int i = 0; i < VEC; ++i) a[4 * i + g][e] = x[i];
     }
 }
-// rows A (load_rows) times the 16 state columns in LDS.
+// Rows (load_rows), scaled, as the A operand that takes the keys in order.
+template <int N>
+__device__ __forceinline__ void scaled_inorder(f32x4 (&a)[N], const f32x4 (&rows)[N], float scale) {
+#pragma unroll
+  for (int g = 0; g < N; ++g) a[g] = acc_inorder(rows[g] * scale);
+}
+// acc += A (scaled_inorder) times the 16 state columns in LDS, in the order of the keys.
 template <int KM>
-__device__ __forceinline__ f32x4 keys_product(const f32x4 (&a)[KM / 16], const float* st, int q, int K) {
-  f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+__device__ __forceinline__ f32x4 keys_product(f32x4 acc, const f32x4 (&a)[KM / 16], const float* st, int q, int K) {
 #pragma unroll
   for (int g = 0; g < KM / 16; ++g)
     if (16 * g < K) mma16(acc, a[g], *reinterpret_cast<const f32x4*>(st + 16 * g + 4 * q));
   return acc;
 }
 // A lane's state column to global memory, value-major (and to LDS as the next
-// product's B operand, keys past K zero).
+// product's B operand: of each 16 keys, key 4 e + x at 4 x + e; keys past K zero).
 template <int VEC, bool FULL>
 __device__ __forceinline__ void put_state(const f32x4 (&s)[VEC], float* global, float* lds, int kb, int K, bool store) {
 #pragma unroll
@@ -129,7 +139,8 @@ __device__ __forceinline__ void put_state(const f32x4 (&s)[VEC], float* global, 
         x[e] = k + e < K ? x[e] : 0.f;
       }
     }
-    *reinterpret_cast<f32x4*>(lds + k) = x;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) lds[(k & ~15) + 4 * e + (k >> 2 & 3)] = x[e];
   }
 }
 
@@ -139,6 +150,7 @@ __global__ __launch_bounds__(NT) void gdn_state_fwd(gpa_gdn_problem p, gpa_gdn_s
   constexpr bool PF = KM <= 128;  // operands of the next chunk in registers of their own
   __shared__ __align__(16) float st_s[SC * (KM + 4)];
   __shared__ __align__(16) float d_s[SC * (R + 4)];
+  __shared__ __align__(16) float rs_s[R];  // e^{G_C-G}, laid out as a column of d_s
   const int s = blockIdx.y, b = s / p.heads, h = s % p.heads;
   const int K = p.kdim, V = p.vdim, tid = threadIdx.x, w = tid / 64, col = tid % 16, q = tid % 64 / 16;
   const int v = blockIdx.x * SC + col, vc = v < V ? v : V - 1;
@@ -147,7 +159,7 @@ __global__ __launch_bounds__(NT) void gdn_state_fwd(gpa_gdn_problem p, gpa_gdn_s
   float* st = st_s + col * (KM + 4);
   float* ds = d_s + col * (R + 4);
 
-  f32x4 S[VEC], wr[KM / 16], kc[4 * VEC], u, gm;
+  f32x4 S[VEC], wr[KM / 16], kc[4 * VEC], kf[VEC], u, gm;
   float gc;
 #pragma unroll
   for (int j = 0; j < 4 * VEC; ++j) {
@@ -162,34 +174,55 @@ __global__ __launch_bounds__(NT) void gdn_state_fwd(gpa_gdn_problem p, gpa_gdn_s
     gm = *reinterpret_cast<const f32x4*>(gam + t0);
     gc = gam[R - 1];
   };
-  auto load_second = [&](int n, f32x4 (&kc)[4 * VEC]) {
-    load_cols<VEC, FULL>(kc, sv.kn + rows_off(s, n, nch, 0, K), k0, q, K);
+  auto load_second = [&](int n, f32x4 (&kc)[4 * VEC], f32x4 (&kf)[VEC]) {
+    const float* kn = sv.kn + rows_off(s, n, nch, 0, K);
+    load_cols<VEC, FULL>(kc, kn, k0, q, K);
+#pragma unroll
+    for (int j = 0; j < VEC; ++j) kf[j] = row4<FULL>(kn, kb + 4 * j, K);
   };
   load_first(0, wr, u, gm, gc);
-  load_second(0, kc);
+  load_second(0, kc, kf);
+  if (PF) scaled_inorder(wr, wr, -1.f);
   for (int n = 0; n < nch; ++n) {
     const int nn = n + 1 < nch ? n + 1 : n;
-    f32x4 wr2[KM / 16], kc2[4 * VEC], u2, gm2;
+    f32x4 wr2[KM / 16], kc2[4 * VEC], kf2[VEC], u2, gm2;
     float gc2;
     if (PF) {
       load_first(nn, wr2, u2, gm2, gc2);
-      load_second(nn, kc2);
+      load_second(nn, kc2, kf2);
     }
+    f32x4 rs;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) rs[e] = __expf(gc - gm[e]);
+    rs = acc_inorder(rs);
+    if (col == 0) *reinterpret_cast<f32x4*>(rs_s + t0) = rs;
+    if (!PF) scaled_inorder(wr, wr, -1.f);
     put_state<VEC, FULL>(S, sv.states + state_off(s, n, nch, K, V) + (int64_t)vc * K, st, kb, K, vok);
     lds_barrier();
     // D = U - W S
-    const f32x4 d = u - keys_product<KM>(wr, st, q, K);
+    const f32x4 d = keys_product<KM>(u, wr, st, q, K);
     if (vok) *reinterpret_cast<f32x4*>(sv.delta + vc_off(s, n, nch, V) + (int64_t)v * R + t0) = d;
-    f32x4 ds4;
-#pragma unroll
-    for (int e = 0; e < 4; ++e) ds4[e] = __expf(gc - gm[e]) * d[e];
-    *reinterpret_cast<f32x4*>(ds + t0) = acc_inorder(ds4);
+    *reinterpret_cast<f32x4*>(ds + t0) = acc_inorder(d);
     const float decay = __expf(gc);
+    // diag(e^{G_C-G}) Kn: position 0's for the state's rows apart, a zero in the product
+    const float r0 = rs_s[0];
+#pragma unroll
+    for (int j = 0; j < VEC; ++j) kf[j] *= r0;
+#pragma unroll
+    for (int g = 0; g < 4; ++g) {
+      f32x4 r = *reinterpret_cast<const f32x4*>(rs_s + 16 * g + 4 * q);
+      if (g == 0 && q == 0) r[0] = 0.f;
+#pragma unroll
+      for (int i = 0; i < VEC; ++i) kc[4 * i + g] *= r;
+    }
     if (!PF) load_first(nn, wr, u, gm, gc);
     lds_barrier();
-    // S = e^{G_C} S + Kn^T diag(e^{G_C-G}) D
+    // S = e^{G_C} S + (diag(e^{G_C-G}) Kn)^T D: position 0's product rounded, e^{G_C} S
+    // added to it, then the other positions
+    const float d0 = ds[0];
 #pragma unroll
-    for (int i = 0; i < VEC; ++i) S[i] *= decay;
+    for (int j = 0; j < 4 * VEC; ++j)
+      S[j % VEC][j / VEC] = __builtin_fmaf(decay, S[j % VEC][j / VEC], kf[j / 4][j % 4] * d0);
     if (KM / 4 * w < K)
 #pragma unroll
       for (int g = 0; g < 4; ++g) {
@@ -197,14 +230,15 @@ __global__ __launch_bounds__(NT) void gdn_state_fwd(gpa_gdn_problem p, gpa_gdn_s
 #pragma unroll
         for (int i = 0; i < VEC; ++i) mma16(S[i], kc[4 * i + g], x);
       }
-    if (PF) {
-#pragma unroll
-      for (int g = 0; g < KM / 16; ++g) wr[g] = wr2[g];
+    if (PF) {  // (the exchanges run beside the MFMAs)
+      scaled_inorder(wr, wr2, -1.f);
 #pragma unroll
       for (int j = 0; j < 4 * VEC; ++j) kc[j] = kc2[j];
+#pragma unroll
+      for (int j = 0; j < VEC; ++j) kf[j] = kf2[j];
       u = u2; gm = gm2; gc = gc2;
     } else {
-      load_second(nn, kc);
+      load_second(nn, kc, kf);
     }
   }
   if (vok)
@@ -401,36 +435,44 @@ __global__ __launch_bounds__(NT) void gdn_state_bwd(gpa_gdn_problem p, gpa_gdn_s
   float* ds = d_s + col * (R + 4);
   const f32x4 zero = {0.f, 0.f, 0.f, 0.f};
 
-  f32x4 S[VEC], kr[KM / 16], qc[4 * VEC], wc[4 * VEC], o[4], d0, gm;
-  float gc;
+  f32x4 S[VEC], kr[KM / 16], qc[4 * VEC], wc[4 * VEC], o[4], d0;
+  float gm, gc;
 #pragma unroll
   for (int j = 0; j < 4 * VEC; ++j) {
     const int k = kb + j;
     const float x = gr.dfinal ? gr.dfinal[(int64_t)s * K * V + (int64_t)(k < K ? k : 0) * V + vc] : 0.f;
     S[j % VEC][j / VEC] = k < K ? x : 0.f;
   }
-  auto load_first = [&](int n, f32x4 (&kr)[KM / 16], f32x4& d0, f32x4& gm, float& gc) {
+  auto load_first = [&](int n, f32x4 (&kr)[KM / 16], f32x4& d0, float& gm, float& gc) {
     const float* gam = sv.gam + rows_off(s, n, nch, 0, 1);
     load_rows<KM, FULL>(kr, sv.kn + rows_off(s, n, nch, 0, K), 16 * w + col, q, K);
     d0 = gr.dd0 ? *reinterpret_cast<const f32x4*>(gr.dd0 + vc_off(s, n, nch, V) + (int64_t)vc * R + t0) : zero;
-    gm = *reinterpret_cast<const f32x4*>(gam + t0);
+    gm = gam[16 * w + col];
     gc = gam[R - 1];
   };
   auto load_second = [&](int n, f32x4 (&qc)[4 * VEC], f32x4 (&wc)[4 * VEC], f32x4 (&o)[4]) {
     if (has_q) {
-      load_cols<VEC, FULL, false>(qc, sv.qn + rows_off(s, n, nch, 0, K), k0, q, K);
+      load_cols<VEC, FULL>(qc, sv.qn + rows_off(s, n, nch, 0, K), k0, q, K);
 #pragma unroll
       for (int g = 0; g < 4; ++g)
         o[g] = *reinterpret_cast<const f32x4*>(gr.o + vc_off(s, n, nch, V) + (int64_t)vc * R + 16 * g + 4 * q);
     }
     load_cols<VEC, FULL>(wc, sv.w + rows_off(s, n, nch, 0, K), k0, q, K);
   };
+  auto o_inorder = [&](f32x4 (&o)[4], const f32x4 (&rows)[4]) {
+#pragma unroll
+    for (int g = 0; g < 4; ++g) o[g] = acc_inorder(rows[g]);
+  };
   load_first(nch - 1, kr, d0, gm, gc);
   load_second(nch - 1, qc, wc, o);
+  if (PF) {
+    scaled_inorder(kr, kr, __expf(gc - gm));
+    if (has_q) o_inorder(o, o);
+  }
   for (int n = nch - 1; n >= 0; --n) {
     const int nn = n > 0 ? n - 1 : 0;
-    f32x4 kr2[KM / 16], qc2[4 * VEC], wc2[4 * VEC], o2[4], d02, gm2;
-    float gc2;
+    f32x4 kr2[KM / 16], qc2[4 * VEC], wc2[4 * VEC], o2[4], d02;
+    float gm2, gc2;
     if (PF) {
       load_first(nn, kr2, d02, gm2, gc2);
       load_second(nn, qc2, wc2, o2);
@@ -440,12 +482,14 @@ __global__ __launch_bounds__(NT) void gdn_state_bwd(gpa_gdn_problem p, gpa_gdn_s
     if (gr.dstates)
 #pragma unroll
       for (int j = 0; j < VEC; ++j) inj[j] = row4<FULL>(gr.dstates + so, kb + 4 * j, K);
+    if (!PF) {
+      scaled_inorder(kr, kr, __expf(gc - gm));
+      if (has_q) o_inorder(o, o);
+    }
     put_state<VEC, FULL>(S, gr.dhend + so, st, kb, K, vok);
     lds_barrier();
-    // dD = dd0 + diag(e^{G_C-G}) Kn dS
-    f32x4 dd = keys_product<KM>(kr, st, q, K);
-#pragma unroll
-    for (int e = 0; e < 4; ++e) dd[e] = d0[e] + __expf(gc - gm[e]) * dd[e];
+    // dD = dd0 + (diag(e^{G_C-G}) Kn) dS
+    const f32x4 dd = keys_product<KM>(d0, kr, st, q, K);
     if (vok) *reinterpret_cast<f32x4*>(gr.ddelta + vc_off(s, n, nch, V) + (int64_t)v * R + t0) = dd;
     *reinterpret_cast<f32x4*>(ds + t0) = acc_inorder(-dd);
     const float decay = __expf(gc);
@@ -471,12 +515,10 @@ __global__ __launch_bounds__(NT) void gdn_state_bwd(gpa_gdn_problem p, gpa_gdn_s
 #pragma unroll
       for (int j = 0; j < 4 * VEC; ++j) S[j % VEC][j / VEC] += inj[j / 4][j % 4];
     if (PF) {
-#pragma unroll
-      for (int g = 0; g < KM / 16; ++g) kr[g] = kr2[g];
+      scaled_inorder(kr, kr2, __expf(gc2 - gm2));
 #pragma unroll
       for (int j = 0; j < 4 * VEC; ++j) { qc[j] = qc2[j]; wc[j] = wc2[j]; }
-#pragma unroll
-      for (int g = 0; g < 4; ++g) o[g] = o2[g];
+      if (has_q) o_inorder(o, o2);
       d0 = d02; gm = gm2; gc = gc2;
     } else {
       load_second(nn, qc, wc, o);

@@ -59,3 +59,50 @@ def test_float32_state_sums_positions_in_order(kd):
     from gpa_amd.ops import gdn_scan_hip
     final, want = telescoping(gdn_scan_hip, DEV, kd)
     assert torch.equal(final, want)
+
+
+def exact_order(scan, device, kd=16):
+    """[(got, want)] of one-token float32 scans whose sums are exact in the
+    recurrences' order only.  The key has 1/2 at keys 0, 4, 5 and 8 and writes are
+    full; rows of the state there are 2 A, 2 B, -2 B and 2 t with t far below an ulp of
+    A and B.  D = U - W S with U = A is A - A - B + B - t; where the sum over the keys
+    comes before U, or key 8 before key 5, t is lost.  dD = dd0 + Kn dS is the same
+    sum.  The state's new row is e^G S + k D with the product rounded and e^G S
+    added to it in one rounding."""
+    gen = torch.Generator().manual_seed(6)
+    vd = 32
+    odd = lambda lo, hi: (2 * torch.randint(lo // 2, hi // 2, (vd,), generator=gen) + 1).float()
+    a, b, t = odd(2 ** 21, 2 ** 22), odd(2 ** 21, 2 ** 22), odd(1, 2 ** 10) / 2 ** 14
+    k = torch.zeros(1, 1, 1, kd)
+    k[..., [0, 4, 5, 8]] = 0.5
+
+    def rows(*x):
+        s = torch.zeros(1, 1, kd, vd)
+        s[0, 0, [0, 4, 5, 8]] = torch.stack(x)
+        return s
+
+    one, zero = torch.ones(1, 1, 1), torch.zeros(1, 1, 1)
+    v = a.view(1, 1, 1, vd)
+    move = lambda *xs: [x.to(device).requires_grad_() for x in xs]
+    out = []
+    args = move(k, k, v, zero, one, rows(2 * a, 2 * b, -2 * b, 2 * t))
+    got = scan(*args, chunk=64, offset=0)
+    out.append((got[2][0, 0, 8], 1.5 * t))
+    dv, = torch.autograd.grad([got[0], got[2]], [args[2]],
+                              [v.to(device), rows(-2 * a, 2 * b, -2 * b, 2 * t).to(device)])
+    out.append((dv.flatten(), t))
+
+    s0 = rows(*torch.randn(4, vd, generator=gen))
+    s0[0, 0, 8] = 0.  # the new row is k D
+    s0[0, 0, 1] = 1.  # ... and e^G
+    v = torch.randn(1, 1, 1, vd, generator=gen)
+    final = scan(None, *move(k, v, zero - 0.3, one, s0), chunk=64, offset=0)[2][0, 0].detach().double().cpu()
+    out.append((final[0], (final[1] * s0[0, 0, 0].double() + final[8]).float()))
+    return [(x.detach().float().cpu(), y) for x, y in out]
+
+
+@pytest.mark.parametrize("kd", [16, 18, 128, 256])
+def test_float32_state_sums_in_the_recurrences_order(kd):
+    from gpa_amd.ops import gdn_scan_hip
+    for got, want in exact_order(gdn_scan_hip, DEV, kd):
+        assert torch.equal(got, want)

@@ -26,7 +26,7 @@ import torch
 
 from tests.host_emu import harness
 from tests.test_gpu_gdn_scan import _inputs, _oracle_segments, _oracle_segments_autograd, _rel
-from tests.test_gpu_gdn_state_f32 import telescoping
+from tests.test_gpu_gdn_state_f32 import exact_order, telescoping
 
 CASES = [
     # (B, T, H, K, V, chunk, offset, dtype)
@@ -137,6 +137,13 @@ def test_emulated_float32_state_sums_positions_in_order(host):
     from gpa_amd.ops import gdn_scan_hip
     final, want = telescoping(gdn_scan_hip, "cpu")
     assert torch.equal(final, want)
+
+
+@pytest.mark.parametrize("kd", [16, 18, 128])
+def test_emulated_float32_state_sums_in_the_recurrences_order(host, kd):
+    from gpa_amd.ops import gdn_scan_hip
+    for got, want in exact_order(gdn_scan_hip, "cpu", kd):
+        assert torch.equal(got, want)
 
 
 @pytest.mark.parametrize("dtype,kd", [(torch.float32, 16), (torch.float32, 100), (torch.bfloat16, 16)], ids=str)
