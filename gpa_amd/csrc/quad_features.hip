@@ -44,10 +44,10 @@ struct QLayout {
   E* dab;       // [32][DLD] d(a) | d(b) rows
   float* nrm;   // [32] ||x||_eps = sqrt(sum x^2 + 1e-12)
   float* xn;    // [32] sqrt(sum x^2)
-  float* part;  // [8][32] per-block row partial sums
-  float* ra;    // [32] row factors of the phase at hand
+  float* part;  // [2][8][32] per-block row partial sums
+  float* ra;    // [32] row values of the phase at hand
   float* rb;
-  float* dn;    // [32] d ||x||_eps / ||x||_eps
+  float* dn;    // [32] d ||x||_eps
   float* wsum;  // [4] per-wave partial of dc
 };
 
@@ -64,7 +64,7 @@ __host__ __device__ inline size_t q_lds_bytes(int dim, bool backward) {
   const int DP = qpad(dim), ULD = DP + 16 / (int)sizeof(E), DLD = 2 * DP + 16 / (int)sizeof(E);
   const int rows = backward && q_raw_in_lds<E>(dim) ? 2 : 1;
   const size_t b = (size_t)QR * ULD * sizeof(E) * rows + (backward ? (size_t)QR * DLD * sizeof(E) : 0);
-  return b + (5 * QR + 8 * QR + 4) * sizeof(float);
+  return b + (5 * QR + 16 * QR + 4) * sizeof(float);
 }
 
 template <typename E>
@@ -93,7 +93,7 @@ __device__ QLayout<E> q_layout(char* smem, int dim, bool backward) {
   L.rb = f + 3 * QR;
   L.dn = f + 4 * QR;
   L.part = f + 5 * QR;
-  L.wsum = f + 13 * QR;
+  L.wsum = f + 21 * QR;
   return L;
 }
 
@@ -148,7 +148,8 @@ __device__ void q_rows(const gpa_quad_problem& p, const E* dout, E* uo, int h, i
   const E* xh = reinterpret_cast<const E*>(p.x) + (int64_t)h * D;
   const E* gh = ROWS ? dout + (int64_t)h * D : nullptr;
   const int64_t gs = (int64_t)p.heads * D;
-  constexpr bool PUT = VEC && ROWS;  // the pieces are not in LDS yet
+  constexpr bool PUT = VEC && ROWS;  // dout's pieces are not in LDS yet
+  E* raw = RAW ? L.x : L.u;
   QPiece<E> xv[PM], gv[PUT ? PM : 1];
   if constexpr (VEC) {
 #pragma unroll
@@ -163,7 +164,6 @@ __device__ void q_rows(const gpa_quad_problem& p, const E* dout, E* uo, int h, i
         gv[i] = q_get(gh + grow * gs + (d < D ? d : 0));
       }
   } else {
-    E* raw = RAW ? L.x : L.u;
     q_stage(p, xh, p.row_stride, r0, L, raw);
     if constexpr (ROWS) q_stage(p, gh, gs, r0, L, L.g);
     lds_barrier();
@@ -173,18 +173,28 @@ __device__ void q_rows(const gpa_quad_problem& p, const E* dout, E* uo, int h, i
       xv[i] = q_get(raw + row * L.ULD + (d < L.DP ? d : 0));
     }
   }
-  float ss = 0.f;
+  if constexpr (VEC) {
 #pragma unroll
-  for (int i = 0; i < PM; ++i)
+    for (int i = 0; i < PM; ++i) {
+      const int d = (part + 8 * i) * N;
 #pragma unroll
-    for (int e = 0; e < N; ++e) {
-      const bool ok = live && (part + 8 * i) * N + e < D;
-      if (!ok) xv[i].v[e] = from_f32<E>(0.f);
-      if constexpr (PUT)
-        if (!ok) gv[i].v[e] = from_f32<E>(0.f);
-      const float x = to_f32(xv[i].v[e]);
-      ss += x * x;
+      for (int e = 0; e < N; ++e) {
+        const bool ok = live && d + e < D;
+        if (!ok) xv[i].v[e] = from_f32<E>(0.f);
+        if constexpr (PUT)
+          if (!ok) gv[i].v[e] = from_f32<E>(0.f);
+      }
+      if (d < L.DP) q_put(raw + row * L.ULD + d, xv[i]);
     }
+    lds_barrier();
+  }
+  // The sum of squares: elements t%8, t%8 + 8, ... in order, then the eight lanes.
+  float ss = 0.f;
+#pragma unroll 4
+  for (int i = 0; i < L.DP / 8; ++i) {
+    const float x = to_f32(raw[row * L.ULD + part + 8 * i]);
+    ss += x * x;
+  }
   ss += __shfl_xor(ss, 1, 64);
   ss += __shfl_xor(ss, 2, 64);
   ss += __shfl_xor(ss, 4, 64);
@@ -193,7 +203,6 @@ __device__ void q_rows(const gpa_quad_problem& p, const E* dout, E* uo, int h, i
   for (int i = 0; i < PM; ++i) {
     const int d = (part + 8 * i) * N;
     if (d >= L.DP) continue;
-    if constexpr (PUT && RAW) q_put(L.x + row * L.ULD + d, xv[i]);
     if constexpr (PUT) q_put(L.g + row * L.ULD + d, gv[i]);
 #pragma unroll
     for (int e = 0; e < N; ++e) xv[i].v[e] = from_f32<E>(to_f32(xv[i].v[e]) / den);
@@ -304,10 +313,11 @@ __device__ __forceinline__ void q_z(const gpa_quad_problem& p, int h, int cb, co
 }
 
 // Rows move between HBM and LDS in 16-byte pieces, a row per 8 lanes, and the
-// per-row factors of an elementwise phase (roots, reciprocals) are formed once per
-// row by 32 threads.  Bound: HBM (the backward moves 6 rows of dim per row); element-
-// wise 2-byte accesses and a root and up to four divisions per element before.
-// bf16, 8192 rows x 16 heads x 128: forward 67 -> 50 us, backward 210 -> 95 us.
+// per-row values of an elementwise phase (roots, cubes) are formed once per row
+// by 32 threads; the divisions stay per element, since a reciprocal per row rounds
+// otherwise (3 and 15 us less, but other bits).  Bound: HBM (the backward moves 6 rows of dim
+// per row) and those divisions; element-wise 2-byte accesses and a root per element before.
+// bf16, 8192 rows x 16 heads x 128: forward 67 -> 52 us, backward 210 -> 104 us.
 // VEC: dim a whole number of 16-byte pieces, every row on a 16-byte boundary.
 template <typename E, bool VEC, int QB>
 __global__ __launch_bounds__(QT) void quad_fwd(gpa_quad_problem p) {
@@ -326,16 +336,17 @@ __global__ __launch_bounds__(QT) void quad_fwd(gpa_quad_problem p) {
   }
   lds_barrier();
   if (threadIdx.x < QR)
-    L.ra[threadIdx.x] = L.nrm[threadIdx.x] / fmaxf(sqrtf(q_row_total(L.part, L.NB, threadIdx.x)), 1e-6f);
+    L.ra[threadIdx.x] = fmaxf(sqrtf(q_row_total(L.part, L.NB, threadIdx.x)), 1e-6f);
   lds_barrier();
-  float f[16];
-  q_at_rows(L.ra, f);
+  float zn[16], nrm[16];
+  q_at_rows(L.ra, zn);
+  q_at_rows(L.nrm, nrm);
 #pragma unroll
   for (int bi = 0; bi < QB; ++bi) {
     const int cb = w + 4 * bi;
     if (cb >= L.NB) break;
 #pragma unroll
-    for (int r = 0; r < 16; ++r) L.u[acc_row(r, l >> 5) * L.ULD + cb * 32 + (l & 31)] = from_f32<E>(z[bi][r] * f[r]);
+    for (int r = 0; r < 16; ++r) L.u[acc_row(r, l >> 5) * L.ULD + cb * 32 + (l & 31)] = from_f32<E>(z[bi][r] / zn[r] * nrm[r]);
   }
   lds_barrier();
   q_rows_out(p, r0, reinterpret_cast<E*>(p.out) + ((int64_t)r0 * p.heads + h) * p.dim, (int64_t)p.heads * p.dim, p.dim,
@@ -363,27 +374,34 @@ __global__ __launch_bounds__(QT) void quad_bwd(gpa_quad_problem p, gpa_quad_grad
     for (int r = 0; r < 16; ++r) gv[bi][r] = to_f32(L.g[at(r, cb)]);
   }
   lds_barrier();
-  float zt = 0.f;
-  if (t < QR) zt = sqrtf(q_row_total(L.part, L.NB, t));
+  if (t < QR) L.ra[t] = fmaxf(sqrtf(q_row_total(L.part, L.NB, t)), 1e-6f);
   lds_barrier();
   // out = unit(z) nrm: d nrm = sum g unit(z), d unit(z) = g nrm; the
-  // normalisation backward needs sum d unit(z) . z = nrm sum g z per row.
+  // normalisation backward needs sum d unit(z) . z per row.
+  {
+    float zn[16], nrm[16];
+    q_at_rows(L.ra, zn);
+    q_at_rows(L.nrm, nrm);
 #pragma unroll
-  for (int bi = 0; bi < QB; ++bi) {
-    const int cb = w + 4 * bi;
-    if (cb >= L.NB) break;
-    float gz[16];
+    for (int bi = 0; bi < QB; ++bi) {
+      const int cb = w + 4 * bi;
+      if (cb >= L.NB) break;
+      float s1[16], s2[16];
 #pragma unroll
-    for (int r = 0; r < 16; ++r) gz[r] = gv[bi][r] * z[bi][r];
-    q_row_part(gz, L.part, cb);
+      for (int r = 0; r < 16; ++r) {
+        s1[r] = gv[bi][r] * (z[bi][r] / zn[r]);
+        gv[bi][r] *= nrm[r];
+        s2[r] = gv[bi][r] * z[bi][r];
+      }
+      q_row_part(s1, L.part, cb);
+      q_row_part(s2, L.part + 8 * QR, cb);
+    }
   }
   lds_barrier();
-  if (t < QR) {  // dz = g ra - z rb
-    const float gz = q_row_total(L.part, L.NB, t), n = L.nrm[t];
-    const float i = zt > 1e-6f ? 1.f / zt : 1e6f;
-    L.ra[t] = n * i;
-    L.rb[t] = zt > 1e-6f ? n * gz * i * i * i : 0.f;
-    L.dn[t] = gz / fmaxf(zt, 1e-6f) / n;
+  if (t < QR) {  // dz = g nrm / ra - z rb
+    const float zt = L.ra[t];
+    L.dn[t] = q_row_total(L.part, L.NB, t);
+    L.rb[t] = q_row_total(L.part + 8 * QR, L.NB, t) / (zt * zt * zt);
   }
   lds_barrier();
   // dz, then da = (dz b) c, db = dz (c a) in E; du starts as dz rounded to E.
@@ -398,7 +416,8 @@ __global__ __launch_bounds__(QT) void quad_bwd(gpa_quad_problem p, gpa_quad_grad
       if (cb >= L.NB) break;
 #pragma unroll
       for (int r = 0; r < 16; ++r) {
-        const float dz = gv[bi][r] * ra[r] - z[bi][r] * rb[r];
+        const float du = gv[bi][r] / ra[r];
+        const float dz = ra[r] > 1e-6f ? du - z[bi][r] * rb[r] : du;
         const float t1 = dz * bv[bi][r];
         dc += t1 * av[bi][r];
         E* d = L.dab + acc_row(r, l >> 5) * L.DLD + cb * 32 + (l & 31);
@@ -461,21 +480,27 @@ __global__ __launch_bounds__(QT) void quad_bwd(gpa_quad_problem p, gpa_quad_grad
     q_row_part(s3, L.part, cb);
   }
   lds_barrier();
-  if (t < QR) {  // dx = du ra - x rb, through unit(x) and ||x||_eps
-    const float n = L.xn[t], i = n > 1e-6f ? 1.f / n : 1e6f;
-    L.ra[t] = i;
-    L.rb[t] = (n > 1e-6f ? q_row_total(L.part, L.NB, t) * i * i * i : 0.f) - L.dn[t];
+  if (t < QR) {  // dx = du / ra - x rb, through unit(x), + dn x / nrm, through ||x||_eps
+    const float n = fmaxf(L.xn[t], 1e-6f);
+    L.ra[t] = n;
+    L.rb[t] = q_row_total(L.part, L.NB, t) / (n * n * n);
   }
   lds_barrier();
-  float ra[16], rb[16];
+  float ra[16], rb[16], dn[16], nrm[16];
   q_at_rows(L.ra, ra);
   q_at_rows(L.rb, rb);
+  q_at_rows(L.dn, dn);
+  q_at_rows(L.nrm, nrm);
 #pragma unroll
   for (int bi = 0; bi < QB; ++bi) {
     const int cb = w + 4 * bi;
     if (cb >= L.NB) break;
 #pragma unroll
-    for (int r = 0; r < 16; ++r) L.u[at(r, cb)] = from_f32<E>(z[bi][r] * ra[r] - av[bi][r] * rb[r]);
+    for (int r = 0; r < 16; ++r) {
+      const float x = av[bi][r], du = z[bi][r] / ra[r];
+      const float d = ra[r] > 1e-6f ? du - x * rb[r] : du;
+      L.u[at(r, cb)] = from_f32<E>(d + dn[r] * x / nrm[r]);
+    }
   }
   lds_barrier();
   q_rows_out(p, r0, reinterpret_cast<E*>(g.dx) + ((int64_t)r0 * p.heads + h) * D, (int64_t)p.heads * D, D, L.u, L.ULD, VEC);

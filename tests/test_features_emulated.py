@@ -80,3 +80,19 @@ def test_quad_features_refuse_parameters_on_another_device(host, name):
     params[name] = params[name].to("meta")
     with pytest.raises(_lib.HipBackendError, match="quadratic features"):
         features._QuadFeatures.apply(torch.randn(5, 2, 8), *params.values())
+
+
+@pytest.mark.parametrize("dim", [16, 130])
+def test_quad_features_round_every_quotient(host, dim):
+    """out = unit(x)/|unit(x)| |x| with zero weight matrices and two nonzero elements
+    a row, in two lanes' sums, so that no sum depends on an order: bit for bit, each
+    quotient rounded by itself (a factor |x|/|unit(x)| per row rounds otherwise)."""
+    gen, at = torch.Generator().manual_seed(dim), [3, 12]
+    x, want = torch.zeros(40, 1, dim), torch.zeros(40, 1, dim)
+    pair = torch.randn(40, 1, 2, generator=gen)
+    ss = (pair * pair).sum(-1, keepdim=True)
+    u = pair / ss.sqrt()
+    x[..., at] = pair
+    want[..., at] = u / (u * u).sum(-1, keepdim=True).sqrt() * (ss + 1e-12).sqrt()
+    zero = torch.zeros(1, dim, dim)
+    assert torch.equal(features._QuadFeatures.apply(x, zero, zero, torch.ones(1)), want)
